@@ -69,11 +69,16 @@ __device__ __forceinline__ double obs_terms(const ModelL96<T, D, LPP>& m,
 #pragma unroll
     for (int i = 0; i + 1 < DL; i += 2) {
       const int j = i + o;  // local index of an observed dimension
-      const double xv = (double)(o ? x[i + 1] : x[i]);
+      // two values, not an element picked by a run-time index (which the
+      // compiler would turn into a chain of compares over the slice)
+      T xe = x[i], xo = x[i + 1];
+      asm("" : "+v"(xe), "+v"(xo));
+      const double xv = (double)(o ? xo : xe);
       const double z = (y[(lo + j) >> 1] - xv) * inv;
       s += -0.5 * (z * z) + c;
     }
-    if (o == 0) {  // the last element is observed only for even starts
+    // the last element is observed only for even starts, in lanes that have it
+    if (o == 0 && (!ModelL96<T, D, LPP>::UNEVEN || lo % (2 * DL - 1) == 0)) {
       const double z = (y[(lo + DL - 1) >> 1] - (double)x[DL - 1]) * inv;
       s += -0.5 * (z * z) + c;
     }
@@ -111,8 +116,10 @@ __device__ __forceinline__ void noise_after(const M& m, uint64_t seed, uint32_t 
 #pragma unroll
   for (int i = 0; i < M::DL; ++i) x[i] = x[i] + sd * z[i];
   if (zout != nullptr) {
+    const int g = (int)threadIdx.x & (M::LPP - 1);
 #pragma unroll
-    for (int i = 0; i < M::DL; ++i) zout[(size_t)(lo + i) * ld + p] = z[i];
+    for (int i = 0; i < M::DL; ++i)
+      if (slice_has<M>(g, i)) zout[(size_t)(lo + i) * ld + p] = z[i];
   }
 }
 

@@ -1,8 +1,9 @@
 // Device-side models and ODE integrators.
 //
 // One particle is owned by a group of LPP consecutive lanes of a wavefront;
-// lane g of the group holds state dimensions [g*DL, (g+1)*DL) in registers
-// (DL = D / LPP).  The Lorenz-96 stencil fetches its three halo values from
+// lane g of the group holds the state dimensions from slice_lo(g) on in
+// registers, DL of them (DL = D / LPP rounded up; where LPP does not divide D
+// the even lanes hold DL and the odd ones DL - 1).  The Lorenz-96 stencil fetches its three halo values from
 // the neighbouring lanes of the group; error norms are group butterfly sums,
 // so every lane of a group computes bit-identical step-control decisions and
 // the group never diverges internally.
@@ -34,9 +35,9 @@ struct ModelArgs {
 };
 
 // ---------------------------------------------------------------- lane groups
-// Cross-lane moves inside a group.  Groups of four use DPP quad permutations
+// Cross-lane moves inside a group.  Groups of two, four and sixteen use DPP
 // (a VALU operand modifier, no LDS traffic); other sizes use ds_bpermute.
-// A quad permutation reads only lanes of the same group, which are active
+// Such a permutation reads only lanes of the same group, which are active
 // together, so bound_ctrl (zero for an invalid source lane) never applies; it
 // is set because it lets the compiler fold the move into the consuming
 // instruction's DPP operand.
@@ -44,6 +45,12 @@ constexpr int QP_PREV = 3 | (0 << 2) | (1 << 4) | (2 << 6);  // lane g reads g-1
 constexpr int QP_NEXT = 1 | (2 << 2) | (3 << 4) | (0 << 6);  // lane g reads g+1 (mod 4)
 constexpr int QP_XOR1 = 1 | (0 << 2) | (3 << 4) | (2 << 6);
 constexpr int QP_XOR2 = 2 | (3 << 2) | (0 << 4) | (1 << 6);
+constexpr int QP_ODD = 1 | (1 << 2) | (3 << 4) | (3 << 6);  // both lanes of a pair read its odd one
+// Groups of sixteen are DPP rows: a rotation of the row is the group's ring.
+constexpr int ROW_ROR1 = 0x121;         // lane g reads g-1 (mod 16)
+constexpr int ROW_ROR15 = 0x12F;        // lane g reads g+1 (mod 16)
+constexpr int ROW_MIRROR = 0x140;       // lane g reads 15-g
+constexpr int ROW_HALF_MIRROR = 0x141;  // lane g reads 7-g within its eight
 
 template <int CTRL>
 __device__ __forceinline__ float dpp(float v) {
@@ -73,6 +80,8 @@ struct Group {
       return dpp<QP_XOR1>(v);
     } else if constexpr (LPP == 4) {
       return dpp<QP_PREV>(v);
+    } else if constexpr (LPP == 16) {
+      return dpp<ROW_ROR1>(v);
     } else {
       const int src = (lane & ~(LPP - 1)) | ((g + LPP - 1) & (LPP - 1));
       return __shfl(v, src, WAVE);
@@ -86,10 +95,22 @@ struct Group {
       return dpp<QP_XOR1>(v);
     } else if constexpr (LPP == 4) {
       return dpp<QP_NEXT>(v);
+    } else if constexpr (LPP == 16) {
+      return dpp<ROW_ROR15>(v);
     } else {
       const int src = (lane & ~(LPP - 1)) | ((g + 1) & (LPP - 1));
       return __shfl(v, src, WAVE);
     }
+  }
+  // LPP 16: sum over the eight pairs of lanes of a value that is equal within
+  // each pair (equal quads, then equal halves: a mirror reads the other one's)
+  template <class T>
+  __device__ __forceinline__ T sum_pairs(T v) const {
+    static_assert(LPP == 16, "pairs of a DPP row");
+    v += dpp<QP_XOR2>(v);
+    v += dpp<ROW_HALF_MIRROR>(v);
+    v += dpp<ROW_MIRROR>(v);
+    return v;
   }
   // butterfly sum: every lane of the group gets the same bits
   template <class T>
@@ -100,6 +121,8 @@ struct Group {
       v += dpp<QP_XOR1>(v);
       v += dpp<QP_XOR2>(v);
       return v;
+    } else if constexpr (LPP == 16) {
+      return sum_pairs(v + dpp<QP_XOR1>(v));
     } else {
 #pragma unroll
       for (int o = 1; o < LPP; o <<= 1) v += __shfl_xor(v, o, WAVE);
@@ -115,6 +138,7 @@ struct ModelPZ {
   static constexpr int D = 2, LPP = 1, DL = 2, NOBS = 1;
   static constexpr bool NOISE_FIRST = true;
   static constexpr bool HAS_FORCING = false;
+  static constexpr int MIN_WAVES = 1;
   T c, e, ml, mq, alpha;
   double mu, sigma, obs_sd;
   __device__ __forceinline__ explicit ModelPZ(const ModelArgs& a) {
@@ -136,13 +160,25 @@ struct ModelPZ {
 };
 
 // Lorenz-96: dx_i/dt = (x_{i+1} - x_{i-2}) x_{i-1} - x_i + F, cyclic.
+//
+// UNEVEN: LPP leaves LPP / 2 of D over; the even lanes of a group then hold DL
+// elements and the odd ones DL - 1, their last register standing for nothing
+// (its derivative is kept at zero, so it adds nothing to an error norm, and no
+// neighbour reads it).
 template <class T, int D_, int LPP_>
 struct ModelL96 {
-  static constexpr int D = D_, LPP = LPP_, DL = D_ / LPP_, NOBS = D_ / 2;
+  static constexpr int D = D_, LPP = LPP_, DL = (D_ + LPP_ - 1) / LPP_, NOBS = D_ / 2;
+  static constexpr bool UNEVEN = D_ % LPP_ != 0;
   static constexpr bool NOISE_FIRST = false;
   // the right-hand side is g(x) + F with a constant forcing F (rhs_unforced: g)
   static constexpr bool HAS_FORCING = true;
-  static_assert(D_ % LPP_ == 0 && DL >= 2 && D_ % 2 == 0, "even dimension, lane slice >= 2");
+  // d = 200 in double over sixteen lanes: 288 registers and one wave per SIMD
+  // unaided; at two, a few spills (208 us against 268 us per 2^16 particles).
+  // The others measured no faster capped (d = 40 in float at five waves
+  // spills: 215 us against 203 us per 2^20).
+  static constexpr int MIN_WAVES = sizeof(T) == 8 && DL >= 12 ? 2 : 1;
+  static_assert(D_ % LPP_ == 0 || (2 * (D_ % LPP_) == LPP_ && LPP_ == 16), "slices");
+  static_assert(DL >= (UNEVEN ? 4 : 2) && D_ % 2 == 0, "even dimension, lane slice >= 2");
   T F;
   double noise_sd, obs_sd;
   __device__ __forceinline__ explicit ModelL96(const ModelArgs& a) {
@@ -153,7 +189,23 @@ struct ModelL96 {
   template <bool FORCED, class G>
   __device__ __forceinline__ void eval(const G& grp, const T (&x)[DL], T (&k)[DL]) const {
     T xm2, xm1, xp1;  // x[lo-2], x[lo-1], x[hi]
-    if constexpr (LPP == 1) {
+    if constexpr (UNEVEN) {
+      const bool full = (grp.g & 1) == 0;
+      xm2 = grp.prev(full ? x[DL - 2] : x[DL - 3]);
+      xm1 = grp.prev(full ? x[DL - 1] : x[DL - 2]);
+      xp1 = grp.next(x[0]);
+      const T xr = full ? x[DL - 1] : xp1;  // right of element DL - 2
+#pragma unroll
+      for (int i = 0; i < DL; ++i) {
+        const T a = (i + 2 < DL) ? x[i + 2 < DL ? i + 1 : 0] : (i + 2 == DL ? xr : xp1);
+        const T b = (i >= 2) ? x[i >= 2 ? i - 2 : 0] : (i == 1 ? xm1 : xm2);
+        const T c = (i >= 1) ? x[i >= 1 ? i - 1 : 0] : xm1;
+        if constexpr (FORCED) k[i] = (a - b) * c - x[i] + F;
+        else k[i] = (a - b) * c - x[i];
+      }
+      k[DL - 1] = full ? k[DL - 1] : T(0);
+      return;
+    } else if constexpr (LPP == 1) {
       xm2 = x[DL - 2];
       xm1 = x[DL - 1];
       xp1 = x[0];
@@ -188,6 +240,7 @@ struct ModelLG {
   static constexpr int D = 1, LPP = 1, DL = 1, NOBS = 1;
   static constexpr bool NOISE_FIRST = false;
   static constexpr bool HAS_FORCING = false;
+  static constexpr int MIN_WAVES = 1;
   T lambda;
   double noise_sd, obs_sd;
   __device__ __forceinline__ explicit ModelLG(const ModelArgs& a) {
@@ -200,6 +253,45 @@ struct ModelLG {
     k[0] = -lambda * x[0];
   }
 };
+
+// Slices of model M: whether odd lanes hold one element less, the first
+// dimension of lane g, and whether element i of the register slice is one of
+// lane g's dimensions.
+template <class M>
+constexpr bool uneven_slices() {
+  if constexpr (M::D % M::LPP == 0) return false;
+  else return M::UNEVEN;
+}
+template <class M>
+__device__ __forceinline__ int slice_lo(int g) {
+  if constexpr (!uneven_slices<M>()) return g * M::DL;
+  else return (g >> 1) * (2 * M::DL - 1) + (g & 1) * M::DL;
+}
+template <class M>
+__device__ __forceinline__ bool slice_has(int g, int i) {
+  if constexpr (!uneven_slices<M>()) return true;
+  else return i + 1 < M::DL || (g & 1) == 0;
+}
+
+// Sum of squares over the particle's dimensions, the same bits in every lane of
+// the group: each slice in order, then the slices by a butterfly.  With uneven
+// slices a pair of lanes is summed in order as one slice (the even lane's sum
+// is where the odd lane starts), as half as many lanes would.
+template <class M, class G, class T, int DL>
+__device__ __forceinline__ T sum_squares(const G& grp, const T (&e)[DL]) {
+  T s = T(0);
+#pragma unroll
+  for (int i = 0; i < DL; ++i) s += e[i] * e[i];
+  if constexpr (uneven_slices<M>()) {
+    const T before = grp.prev(s);  // outside the choice: every lane takes part
+    s = (grp.g & 1) != 0 ? before : T(0);
+#pragma unroll
+    for (int i = 0; i < DL; ++i) s += e[i] * e[i];
+    return grp.sum_pairs(dpp<QP_ODD>(s));
+  } else {
+    return grp.sum(s);
+  }
+}
 
 // ---------------------------------------------------------------- integrators
 // RK4IntegratorHost::update for one particle; returns the number of steps.
@@ -248,26 +340,15 @@ __device__ __forceinline__ int integrate_rk4(const M& m, const G& grp, T (&x0)[M
 
 // Scaled error of one component: err h / (atol + rtol max(|a|, |b|)).
 // double: as written.  float: err / den with v_rcp_f32 (1 ulp; the norm only
-// steers h), the factor h applied once to the whole norm by the caller, and
-// the larger magnitude by one v_max_f32 with absolute-value source modifiers
-// (a NaN state already makes err, hence the norm, NaN).
+// steers h), the factor h applied once to the whole norm, and the larger
+// magnitude by one v_max_f32 with absolute-value source modifiers (a NaN
+// state already makes err, hence the norm, NaN).
 __device__ __forceinline__ float max_abs(float a, float b) {
   // one instruction with the operands' absolute values (the compiler's fmaxf
   // first canonicalizes operands it cannot prove quiet, two more instructions)
   float r;
   asm("v_max_f32_e64 %0, |%1|, |%2|" : "=v"(r) : "v"(a), "v"(b));
   return r;
-}
-
-template <class T>
-__device__ __forceinline__ T err_scale(T err, T h, T atol, T rtol, T a, T b) {
-  if constexpr (sizeof(T) == 4) {
-    const T den = atol + rtol * max_abs(a, b);
-    return err * __builtin_amdgcn_rcpf(den);
-  } else {
-    const T den = atol + rtol * fmax(fabs(a), fabs(b));
-    return err * h / den;
-  }
 }
 
 // DOPRI5IntegratorHost::update for one particle; returns the number of steps.
@@ -328,91 +409,111 @@ __device__ __forceinline__ int dopri5_loop(const M& m, const G& grp, T (&x0)[M::
     const T hT = (T)h;
     if (!k1in) stage_rhs<FOLD>(m, grp, x0, k1);
     k1in = true;
-    T xs[DL], a3[DL], a4[DL], a5[DL], a6[DL], y6[DL], er[DL], k[DL];
+    // Most of the loop's instructions are 8 bytes (a literal coefficient or a
+    // third operand).  It runs faster when they start 4 bytes past a multiple of
+    // 8 (203 us against 237 us per 2^20 particles of Lorenz-96 d = 40, 46 against
+    // 53 for d = 8), so the stages start there; slices of an odd length mix
+    // both (no difference).  No result depends on it.
+    if constexpr (F32 && DL % 2 == 0) asm volatile(".p2align 3\n\ts_nop 0");
+    // Each stage sums the stored derivatives when it needs them, in the order
+    // an accumulator per stage would add them (the same bits, seven arrays in
+    // registers at most instead of nine: in banks Lorenz-96 d = 40 keeps four
+    // waves per SIMD instead of three, 149 us against 159 us).
+    T xs[DL], k2[DL], k3[DL], k4[DL], k5[DL], y6[DL], er[DL], k[DL];
     // stage 1
-    if constexpr (FOLD) {
 #pragma unroll
-      for (int i = 0; i < DL; ++i) {
-        xs[i] = hT * (T(0.2) * k1[i] + c2F) + x0[i];
-        a3[i] = T(3.0 / 40.0) * k1[i] + c3F;
-        a4[i] = T(44.0 / 45.0) * k1[i] + c4F;
-        a5[i] = T(19372.0 / 6561.0) * k1[i] + c5F;
-        a6[i] = T(9017.0 / 3168.0) * k1[i] + fc;
-        y6[i] = T(35.0 / 384.0) * k1[i] + fc;
-        er[i] = T(71.0 / 57600.0) * k1[i];
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < DL; ++i) {
-        xs[i] = hT * (T(0.2) * k1[i]) + x0[i];
-        a3[i] = T(3.0 / 40.0) * k1[i];
-        a4[i] = T(44.0 / 45.0) * k1[i];
-        a5[i] = T(19372.0 / 6561.0) * k1[i];
-        a6[i] = T(9017.0 / 3168.0) * k1[i];
-        y6[i] = T(35.0 / 384.0) * k1[i];
-        er[i] = T(71.0 / 57600.0) * k1[i];
-      }
+    for (int i = 0; i < DL; ++i) {
+      T s = T(0.2) * k1[i];
+      if constexpr (FOLD) s += c2F;
+      xs[i] = hT * s + x0[i];
     }
     // stage 2
-    stage_rhs<FOLD>(m, grp, xs, k);
+    stage_rhs<FOLD>(m, grp, xs, k2);
 #pragma unroll
     for (int i = 0; i < DL; ++i) {
-      a3[i] += T(9.0 / 40.0) * k[i];
-      a4[i] += T(-56.0 / 15.0) * k[i];
-      a5[i] += T(-25360.0 / 2187.0) * k[i];
-      a6[i] += T(-355.0 / 33.0) * k[i];
-      xs[i] = hT * a3[i] + x0[i];
+      T s = T(3.0 / 40.0) * k1[i];
+      if constexpr (FOLD) s += c3F;
+      s += T(9.0 / 40.0) * k2[i];
+      xs[i] = hT * s + x0[i];
     }
     // stage 3
-    stage_rhs<FOLD>(m, grp, xs, k);
+    stage_rhs<FOLD>(m, grp, xs, k3);
 #pragma unroll
     for (int i = 0; i < DL; ++i) {
-      a4[i] += T(32.0 / 9.0) * k[i];
-      a5[i] += T(64448.0 / 6561.0) * k[i];
-      a6[i] += T(46732.0 / 5247.0) * k[i];
-      y6[i] += T(500.0 / 1113.0) * k[i];
-      er[i] += T(-71.0 / 16695.0) * k[i];
-      xs[i] = hT * a4[i] + x0[i];
+      T s = T(44.0 / 45.0) * k1[i];
+      if constexpr (FOLD) s += c4F;
+      s += T(-56.0 / 15.0) * k2[i];
+      s += T(32.0 / 9.0) * k3[i];
+      xs[i] = hT * s + x0[i];
     }
     // stage 4
-    stage_rhs<FOLD>(m, grp, xs, k);
+    stage_rhs<FOLD>(m, grp, xs, k4);
 #pragma unroll
     for (int i = 0; i < DL; ++i) {
-      a5[i] += T(-212.0 / 729.0) * k[i];
-      a6[i] += T(49.0 / 176.0) * k[i];
-      y6[i] += T(125.0 / 192.0) * k[i];
-      er[i] += T(71.0 / 1920.0) * k[i];
-      xs[i] = hT * a5[i] + x0[i];
+      T s = T(19372.0 / 6561.0) * k1[i];
+      if constexpr (FOLD) s += c5F;
+      s += T(-25360.0 / 2187.0) * k2[i];
+      s += T(64448.0 / 6561.0) * k3[i];
+      s += T(-212.0 / 729.0) * k4[i];
+      xs[i] = hT * s + x0[i];
     }
     // stage 5
-    stage_rhs<FOLD>(m, grp, xs, k);
+    stage_rhs<FOLD>(m, grp, xs, k5);
 #pragma unroll
     for (int i = 0; i < DL; ++i) {
-      a6[i] += T(-5103.0 / 18656.0) * k[i];
-      y6[i] += T(-2187.0 / 6784.0) * k[i];
-      er[i] += T(-17253.0 / 339200.0) * k[i];
-      xs[i] = hT * a6[i] + x0[i];
+      T s = T(9017.0 / 3168.0) * k1[i];
+      if constexpr (FOLD) s += fc;
+      s += T(-355.0 / 33.0) * k2[i];
+      s += T(46732.0 / 5247.0) * k3[i];
+      s += T(49.0 / 176.0) * k4[i];
+      s += T(-5103.0 / 18656.0) * k5[i];
+      xs[i] = hT * s + x0[i];
     }
     // stage 6: xs now holds x5
     stage_rhs<FOLD>(m, grp, xs, k);
 #pragma unroll
     for (int i = 0; i < DL; ++i) {
-      y6[i] += T(11.0 / 84.0) * k[i];
-      er[i] += T(22.0 / 525.0) * k[i];
-      y6[i] = hT * y6[i] + x0[i];
+      T s = T(35.0 / 384.0) * k1[i];
+      if constexpr (FOLD) s += fc;
+      s += T(500.0 / 1113.0) * k3[i];
+      s += T(125.0 / 192.0) * k4[i];
+      s += T(-2187.0 / 6784.0) * k5[i];
+      s += T(11.0 / 84.0) * k[i];
+      y6[i] = hT * s + x0[i];
+      T e = T(71.0 / 57600.0) * k1[i];
+      e += T(-71.0 / 16695.0) * k3[i];
+      e += T(71.0 / 1920.0) * k4[i];
+      e += T(-17253.0 / 339200.0) * k5[i];
+      e += T(22.0 / 525.0) * k[i];
+      er[i] = e;
     }
     // stage 7 (FSAL): k7 at x6 into k; the reference host evaluates it at
     // x5, which is k6 = f(x5) already in k
     if constexpr (!QUIRK) stage_rhs<FOLD>(m, grp, y6, k);
-    T e2l = T(0);
+    if constexpr (F32) {
+      // the reciprocals one after another: between other instructions each
+      // costs about twice its 8 cycles
+      T den[DL];
 #pragma unroll
-    for (int i = 0; i < DL; ++i) {
-      er[i] += T(-1.0 / 40.0) * k[i];
-      const T e = err_scale(er[i], hT, atol, rtol, x0[i], y6[i]);
-      e2l += e * e;
+      for (int i = 0; i < DL; ++i) den[i] = atol + rtol * max_abs(x0[i], y6[i]);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < DL; ++i) den[i] = __builtin_amdgcn_rcpf(den[i]);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < DL; ++i) {
+        er[i] += T(-1.0 / 40.0) * k[i];
+        er[i] = er[i] * den[i];
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < DL; ++i) {
+        er[i] += T(-1.0 / 40.0) * k[i];
+        er[i] = er[i] * hT / (atol + rtol * fmax(fabs(x0[i]), fabs(y6[i])));
+      }
     }
-    T e2 = grp.sum(e2l) * invD;
-    if constexpr (sizeof(T) == 4) e2 *= hT * hT;  // err_scale leaves h out for float
+    T e2 = sum_squares<M>(grp, er) * invD;
+    if constexpr (F32) e2 *= hT * hT;
     if (e2 <= T(1)) {
       t += h;
 #pragma unroll
@@ -483,7 +584,7 @@ __device__ __forceinline__ void slice_normals(uint64_t seed, uint32_t index, uin
     }
     return;
   }
-  constexpr int NB = (DL + 3) / 4 + 1;
+  constexpr int NB = (DL + 3 + 3) / 4;  // a slice starts up to 3 into its first block
   T Z[4 * NB];
   const int b0 = lo >> 2, s = lo & 3;
   const bool need_last = (s + DL) > 4 * (NB - 1);
@@ -498,11 +599,11 @@ __device__ __forceinline__ void slice_normals(uint64_t seed, uint32_t index, uin
 #pragma unroll
     for (int i = 0; i < 4; ++i) Z[4 * b + i] = q[i];
   }
+  // drop the first s normals: by one, then by two
 #pragma unroll
-  for (int i = 0; i < DL; ++i) {
-    const T v0 = Z[i], v1 = Z[i + 1], v2 = Z[i + 2], v3 = Z[i + 3];
-    z[i] = s == 0 ? v0 : (s == 1 ? v1 : (s == 2 ? v2 : v3));
-  }
+  for (int i = 0; i + 1 < 4 * NB; ++i) Z[i] = (s & 1) != 0 ? Z[i + 1] : Z[i];
+#pragma unroll
+  for (int i = 0; i < DL; ++i) z[i] = (s & 2) != 0 ? Z[i + 2] : Z[i];
 }
 
 }  // namespace bihip

@@ -61,12 +61,10 @@ __device__ __forceinline__ double uniform(double v) {
 // SCHED: the filter step has a schedule or inputs (times, observed flags,
 // per-step parameters); without them the kernel is compiled without that code,
 // which costs the plain step about 7% when present but unused.
-// Waves per SIMD the compiler must leave room for: a generated functor names
-// its own (MIN_WAVES), the hand-written ones fit their budget unaided.
+// Waves per SIMD the compiler must leave room for: the functor names its own.
 template <class M>
 constexpr int trans_min_waves() {
-  if constexpr (is_generated<M>::value) return M::MIN_WAVES;
-  else return 1;
+  return M::MIN_WAVES;
 }
 
 // ONE: a generated model's interval is one sub-interval of its delta that
@@ -95,10 +93,9 @@ void k_transition(TransArgs a) {
     a.m.obs_c = uniform(row[17]);
   }
   const int blk = xcd_block(blockIdx.x, gridDim.x);
-  const int tid = blk * TRANS_BLOCK + threadIdx.x;
-  const int p = tid / LPP;
+  const int p = blk * (TRANS_BLOCK / LPP) + (int)threadIdx.x / LPP;
   const Group<LPP> grp;
-  const int lo = grp.g * DL;
+  const int lo = slice_lo<M>(grp.g);
   const bool active = p < a.P;
 
   bool gather = a.as != nullptr;
@@ -132,7 +129,8 @@ void k_transition(TransArgs a) {
     const T* Xin = static_cast<const T*>(a.Xin);
     T x[DL];
 #pragma unroll
-    for (int i = 0; i < DL; ++i) x[i] = Xin[(size_t)(lo + i) * a.ld + src];
+    for (int i = 0; i < DL; ++i)
+      x[i] = slice_has<M>(grp.g, i) ? Xin[(size_t)(lo + i) * a.ld + src] : T(0);
 
     auto model = [&]() {
       if (!SCHED || in == nullptr) return M(a.m);
@@ -177,7 +175,8 @@ void k_transition(TransArgs a) {
 
     T* Xout = static_cast<T*>(a.Xout);
 #pragma unroll
-    for (int i = 0; i < DL; ++i) Xout[(size_t)(lo + i) * a.ld + p] = x[i];
+    for (int i = 0; i < DL; ++i)
+      if (slice_has<M>(grp.g, i)) Xout[(size_t)(lo + i) * a.ld + p] = x[i];
     if (a.nsteps_out != nullptr && grp.g == 0) a.nsteps_out[p] = n;
 
     if (y != nullptr) {
@@ -217,10 +216,9 @@ __global__ __launch_bounds__(TRANS_BLOCK) void k_init(ModelArgs ma, uint64_t see
     batch += (uint32_t)f;
     Xv = bank_shift(Xv, f * bx * (long)sizeof(T));
   }
-  const int tid = blockIdx.x * TRANS_BLOCK + threadIdx.x;
-  const int p = tid / LPP;
+  const int p = blockIdx.x * (TRANS_BLOCK / LPP) + (int)threadIdx.x / LPP;
   const Group<LPP> grp;
-  const int lo = grp.g * DL;
+  const int lo = slice_lo<M>(grp.g);
   if (p >= P) return;
   T* X = static_cast<T*>(Xv);
   if constexpr (is_generated<M>::value) {
@@ -239,6 +237,7 @@ __global__ __launch_bounds__(TRANS_BLOCK) void k_init(ModelArgs ma, uint64_t see
       v = i == 0 ? exp(ma.par[7] + ma.par[8] * (double)z[0])
                  : exp(ma.par[9] + ma.par[10] * (double)z[1]);
     } else if (ma.model == BIHIP_MODEL_L96) {
+      if (!slice_has<M>(grp.g, i)) break;
       v = mean0[lo + i] + ma.par[3] * (double)z[i];
     } else {
       v = ma.par[3] + ma.par[4] * (double)z[i];
@@ -254,15 +253,15 @@ __global__ __launch_bounds__(TRANS_BLOCK) void k_obs_logdensity(ModelArgs ma, co
                                                                 double* lws) {
   using T = typename M::real_t;
   constexpr int LPP = M::LPP, DL = M::DL;
-  const int tid = blockIdx.x * TRANS_BLOCK + threadIdx.x;
-  const int p = tid / LPP;
+  const int p = blockIdx.x * (TRANS_BLOCK / LPP) + (int)threadIdx.x / LPP;
   const Group<LPP> grp;
-  const int lo = grp.g * DL;
+  const int lo = slice_lo<M>(grp.g);
   if (p >= P) return;
   const T* X = static_cast<const T*>(Xv);
   T x[DL];
 #pragma unroll
-  for (int i = 0; i < DL; ++i) x[i] = X[(size_t)(lo + i) * ld + p];
+  for (int i = 0; i < DL; ++i)
+    x[i] = slice_has<M>(grp.g, i) ? X[(size_t)(lo + i) * ld + p] : T(0);
   M m(ma);
   const double part = grp.sum(obs_of(m, x, y, lo));
   if (grp.g == 0) lws[p] = lws[p] + part;
@@ -359,6 +358,11 @@ bool model_supported(const bihip_model* m) {
 #ifndef L96_D40_LPP
 #define L96_D40_LPP 4
 #endif
+// d = 200: sixteen lanes of 13 or 12 dimensions, the group a DPP row.  Eight
+// lanes of 25 needed 262 to 309 registers (one wave per SIMD) and LDS
+// permutes for the halos: 487 us against 317 us per N = 2^18 FP32 transition,
+// 369 us against 208 us per 2^16 FP64 ones.
+constexpr int L96_D200_LPP = 16;
 
 // Calls F::template run<M>() for the model type selected by m.
 template <class F>
@@ -373,7 +377,8 @@ static int with_model(const bihip_model* m, F& f) {
         return f64 ? f.template run<L96<double, 40, L96_D40_LPP>>()
                    : f.template run<L96<float, 40, L96_D40_LPP>>();
       if (m->d == 200)
-        return f64 ? f.template run<L96<double, 200, 8>>() : f.template run<L96<float, 200, 8>>();
+        return f64 ? f.template run<L96<double, 200, L96_D200_LPP>>()
+                   : f.template run<L96<float, 200, L96_D200_LPP>>();
       return f64 ? f.template run<L96<double, 8, 2>>() : f.template run<L96<float, 8, 2>>();
     default:
       return f64 ? f.template run<LG<double>>() : f.template run<LG<float>>();
@@ -382,7 +387,7 @@ static int with_model(const bihip_model* m, F& f) {
 
 int transition_blocks(const bihip_model* m, int P) {
   int lpp = 1;
-  if (m->model == BIHIP_MODEL_L96) lpp = m->d == 200 ? 8 : (m->d == 40 ? L96_D40_LPP : 2);
+  if (m->model == BIHIP_MODEL_L96) lpp = m->d == 200 ? L96_D200_LPP : (m->d == 40 ? L96_D40_LPP : 2);
   if (const GenInfo* g = generated_info(m->model)) lpp = g->lpp;
   return ceil_div((long)P * lpp, TRANS_BLOCK);
 }

@@ -79,7 +79,7 @@ def test_l96_filter_fp64_parity(ctx, orc):
 
 
 def test_l96_d200_filter_fp64_parity(ctx, orc):
-    """Lorenz-96 d=200 (eight lanes per particle, 25 dimensions each: the
+    """Lorenz-96 d=200 (sixteen lanes per particle, 13 or 12 dimensions each: the
     observed even dimensions alternate between lanes), FP64, N=2048, T=8."""
     om0 = orc.make_model("l96", d=200)
     mean0 = l96_spun_up(orc, d=200)

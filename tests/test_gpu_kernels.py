@@ -131,7 +131,7 @@ def test_transition_parity(ctx, orc, torch_gpu, kind, integ, prec, quirk):
 
 @pytest.mark.parametrize("prec", [capi.F64, capi.F32])
 def test_l96_d200_transition_and_density(ctx, orc, torch_gpu, prec):
-    """d=200: eight lanes per particle with 25-dimension slices."""
+    """d=200: sixteen lanes per particle with slices of 13 and 12 dimensions."""
     P = 700
     gm = capi.make_model("l96", d=200, precision=prec)
     om = oracle_model(orc, gm)
@@ -153,6 +153,42 @@ def test_l96_d200_transition_and_density(ctx, orc, torch_gpu, prec):
     capi.check(L().bihip_obs_logdensity(ctx.h, ctypes.byref(gm), _c(dev(y)), P, _c(Xout), P,
                                         _c(lws)))
     ref_l = orc.obs_logdensity(om, y, got, lws0)
+    np.testing.assert_allclose(host(lws), ref_l, rtol=1e-12, atol=1e-10)
+
+
+@pytest.mark.parametrize("integ", [capi.DOPRI5, capi.RK4])
+@pytest.mark.parametrize("prec", [capi.F64, capi.F32])
+@pytest.mark.parametrize("P", [1, 3, 5, 16, 17, 255])
+def test_l96_d200_uneven_slices(ctx, orc, torch_gpu, P, prec, integ):
+    """Particle counts around a wave's four and a workgroup's sixteen particles of
+    d = 200: initial samples, transition and density against the oracle, in a wider
+    leading dimension whose padding stays untouched."""
+    ld = P + 3
+    gm = capi.make_model("l96", d=200, precision=prec, integrator=integ, h0=0.02)
+    om = oracle_model(orc, gm)
+    mean0 = np.ascontiguousarray(l96_spun_up(orc, d=200))
+    npdt = np.float64 if prec == capi.F64 else np.float32
+    X = np.full((200, ld), 1e30, npdt)
+    Xin, Xout = dev(X), dev(X)
+    capi.check(L().bihip_init_samples(ctx.h, ctypes.byref(gm), 21, 0, P, _c(Xin), ld,
+                                      mean0.ctypes.data_as(ctypes.POINTER(ctypes.c_double))))
+    X0 = host(Xin)
+    tol = 1e-13 if prec == capi.F64 else 2e-6
+    np.testing.assert_allclose(X0[:, :P].astype(np.float64),
+                               orc.init_samples(om, 21, P, mean0=mean0), rtol=tol, atol=tol)
+    capi.check(L().bihip_transition(ctx.h, ctypes.byref(gm), 5, 0, 4, 0.25, 0.30, P, _c(Xin),
+                                    _c(Xout), ld, None, None))
+    ref = orc.transition(om, 5, 4, 0.25, 0.30, X0[:, :P].astype(np.float64))
+    got = host(Xout)
+    tol = _tol(prec, "l96")
+    np.testing.assert_allclose(got[:, :P].astype(np.float64), ref, rtol=tol, atol=tol)
+    assert (X0[:, P:] == npdt(1e30)).all() and (got[:, P:] == npdt(1e30)).all()
+    y = np.linspace(-3.0, 5.0, 100)
+    lws = dev(np.zeros(P))
+    capi.check(L().bihip_obs_logdensity(ctx.h, ctypes.byref(gm), _c(dev(y)), P, _c(Xout), ld,
+                                        _c(lws)))
+    ref_l = orc.obs_logdensity(om, y, np.ascontiguousarray(got[:, :P].astype(np.float64)),
+                               np.zeros(P))
     np.testing.assert_allclose(host(lws), ref_l, rtol=1e-12, atol=1e-10)
 
 
