@@ -1299,7 +1299,7 @@ int bihip_pf_set_surrogate(bihip_pf* pf, bihip_mlp* mlp, const bihip_surrogate_n
     S.net = mlp_view(mlp);
     if (S.net.L != 4 || S.net.dims[0] != 41 || S.net.dims[4] != 40)
       return set_error(BIHIP_EINVAL, "the surrogate must be a 41-256-256-256-40 network");
-    if ((rc = mlp_inference_weights(mlp, S.Winf))) return rc;
+    if ((rc = mlp_inference_weights(mlp, pf->ctx->stream, S.Winf))) return rc;
     S.x_shift = norm->x_shift;
     S.x_scale = norm->x_scale;
     S.dx_scale = norm->dx_scale;
@@ -1340,7 +1340,7 @@ int bihip_pf_set_guided(bihip_pf* pf, bihip_mlp* mlp, const bihip_guided_norm* n
     G.net = mlp_view(mlp);
     if (G.net.L != 4 || G.net.dims[0] != 301 || G.net.dims[4] != 400)
       return set_error(BIHIP_EINVAL, "the proposal must be a 301-256-256-256-400 network");
-    if ((rc = mlp_inference_weights(mlp, G.Winf, G.binf, 16))) return rc;
+    if ((rc = mlp_inference_weights(mlp, pf->ctx->stream, G.Winf, G.binf, 16))) return rc;
     G.x_shift = norm->x_shift;
     G.x_scale = norm->x_scale;
     G.innov_scale = norm->innov_scale;

@@ -444,8 +444,21 @@ MlpView mlp_view(const bihip_mlp* m);
 // out_interleave outputs, [m of outputs 16 t .., then s of the same outputs],
 // for networks whose outputs are a mean (first half) and a log variance;
 // b (nullable) then gets biases in the same row order.
-int mlp_inference_weights(bihip_mlp* m, const uint16_t* W[MLP_MAX_LAYERS],
+// Written by a kernel on the network's stream; `user` is the stream that reads
+// them next (the call waits for the kernel if it is another one).
+int mlp_inference_weights(bihip_mlp* m, hipStream_t user, const uint16_t* W[MLP_MAX_LAYERS],
                           const float* b[MLP_MAX_LAYERS] = nullptr, int out_interleave = 0);
+
+struct InferenceWeightsArgs {
+  const float* P;               // FP32 parameters: [all W | all b]
+  uint16_t* W;                  // inference weights, laid out as the W part
+  float* b;                     // inference biases
+  int L, interleave, dout;
+  long nW, nb;                  // elements of W and b
+  int pad[MLP_MAX_LAYERS + 1];
+  long offW[MLP_MAX_LAYERS], offb[MLP_MAX_LAYERS];
+};
+int launch_inference_weights(const InferenceWeightsArgs& a, hipStream_t s);
 
 // ---- learned surrogate flow (surrogate.hip)
 struct SurrogateLaunch {

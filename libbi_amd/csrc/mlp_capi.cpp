@@ -213,18 +213,8 @@ void unpack(const bihip_mlp* m, const std::vector<float>& P, float* flat) {
 
 }  // namespace
 
-namespace {
-uint16_t host_f2bf(float f) {  // round to nearest even
-  uint32_t u;
-  std::memcpy(&u, &f, 4);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((u >> 16) | 0x40u);
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return (uint16_t)(u >> 16);
-}
-}  // namespace
-
 namespace bihip {
-int mlp_inference_weights(bihip_mlp* m, const uint16_t* W[MLP_MAX_LAYERS],
+int mlp_inference_weights(bihip_mlp* m, hipStream_t user, const uint16_t* W[MLP_MAX_LAYERS],
                           const float* b[MLP_MAX_LAYERS], int out_interleave) {
   if (m->L > MLP_MAX_LAYERS) return set_error(BIHIP_EINVAL, "too many layers");
   const int L = m->L, dout = m->dims[L];
@@ -235,38 +225,24 @@ int mlp_inference_weights(bihip_mlp* m, const uint16_t* W[MLP_MAX_LAYERS],
   if (m->Winf == nullptr && (rc = dalloc(&m->Winf, m->nW))) return rc;
   if (m->binf == nullptr && (rc = dalloc(&m->binf, m->ntot - m->nW))) return rc;
   hipStream_t s = ctx_stream_of(m->ctx);
-  std::vector<float> P(m->ntot);
-  BIHIP_HIP(hipMemcpyAsync(P.data(), m->P, sizeof(float) * m->ntot, hipMemcpyDeviceToHost, s));
-  BIHIP_HIP(hipStreamSynchronize(s));
-  std::vector<uint16_t> H(m->nW, 0);
-  std::vector<float> B(m->ntot - m->nW, 0.0f);
+  InferenceWeightsArgs a{};
+  a.P = m->P;
+  a.W = m->Winf;
+  a.b = m->binf;
+  a.L = L;
+  a.nW = m->nW;
+  a.nb = m->ntot - m->nW;
+  a.interleave = out_interleave;
+  a.dout = dout;
+  for (int l = 0; l <= L; ++l) a.pad[l] = m->pad[l];
   for (int l = 0; l < L; ++l) {
-    const int K = m->pad[l], N = m->pad[l + 1];
-    for (int n = 0; n < N; ++n) {
-      // source row: natural, or for the interleaved output layer block t of
-      // 2 out_interleave rows = [m of outputs t*oi .., s of the same outputs]
-      int srow = n;
-      if (l == L - 1 && out_interleave > 0) {
-        const int oi = out_interleave, t = n / (2 * oi), r = n % (2 * oi);
-        const int dim = t * oi + (r < oi ? r : r - oi);
-        srow = dim < dout / 2 ? (r < oi ? dim : dout / 2 + dim) : -1;
-      }
-      const long boff = m->offb[l] - m->nW;
-      B[boff + n] = srow >= 0 ? P[m->offb[l] + srow] : 0.0f;
-      for (int k = 0; k < K; ++k) {
-        // position 16 c + p holds input 16 c + perm(p), perm = [0-3, 8-11, 4-7, 12-15]
-        const int c = k >> 4, q = k & 15;
-        const int src = l == 0 ? k : 16 * c + 8 * ((q & 7) >> 2) + 4 * (q >> 3) + (q & 3);
-        H[m->offW[l] + (long)n * K + k] =
-            srow >= 0 ? host_f2bf(P[m->offW[l] + (long)srow * K + src]) : (uint16_t)0;
-      }
-    }
+    a.offW[l] = m->offW[l];
+    a.offb[l] = m->offb[l] - m->nW;
     W[l] = m->Winf + m->offW[l];
-    if (b != nullptr) b[l] = m->binf + (m->offb[l] - m->nW);
+    if (b != nullptr) b[l] = m->binf + a.offb[l];
   }
-  BIHIP_HIP(hipMemcpyAsync(m->Winf, H.data(), sizeof(uint16_t) * m->nW, hipMemcpyHostToDevice, s));
-  BIHIP_HIP(hipMemcpyAsync(m->binf, B.data(), sizeof(float) * B.size(), hipMemcpyHostToDevice, s));
-  BIHIP_HIP(hipStreamSynchronize(s));
+  if ((rc = launch_inference_weights(a, s))) return rc;
+  if (user != s) BIHIP_HIP(hipStreamSynchronize(s));  // no order between the streams
   return BIHIP_OK;
 }
 
@@ -535,7 +511,7 @@ int bihip_surrogate_flow(bihip_ctx* ctx, bihip_mlp* m, const bihip_surrogate_nor
   if (Xin_dev == Xout_dev) return set_error(BIHIP_EINVAL, "the flow is out of place");
   SurrogateLaunch L{};
   L.net = mlp_view(m);
-  if ((rc = mlp_inference_weights(m, L.Winf))) return rc;
+  if ((rc = mlp_inference_weights(m, ctx_stream_of(ctx), L.Winf))) return rc;
   L.x_shift = norm->x_shift;
   L.x_scale = norm->x_scale;
   L.dx_scale = norm->dx_scale;
@@ -561,7 +537,7 @@ int bihip_guided_propose(bihip_ctx* ctx, bihip_mlp* m, const bihip_guided_norm* 
   if (P < 0 || ld < P) return set_error(BIHIP_EINVAL, "need 0 <= P <= ld");
   GuidedLaunch G{};
   G.net = mlp_view(m);
-  if ((rc = mlp_inference_weights(m, G.Winf, G.binf, 16))) return rc;
+  if ((rc = mlp_inference_weights(m, ctx_stream_of(ctx), G.Winf, G.binf, 16))) return rc;
   G.x_shift = norm->x_shift;
   G.x_scale = norm->x_scale;
   G.innov_scale = norm->innov_scale;

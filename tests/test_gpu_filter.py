@@ -95,7 +95,7 @@ def test_l96_d200_filter_fp64_parity(ctx, orc):
 
 
 def test_l96_d200_filter_fp32_mixed_precision(ctx, orc):
-    """d=200 with FP32 state (eight lanes per particle, the forcing carried in the
+    """d=200 with FP32 state (sixteen lanes per particle, the forcing carried in the
     stage constants) and no resampling: the FP64 oracle's logZ and ESS to FP32
     rounding."""
     om0 = orc.make_model("l96", d=200)

@@ -84,3 +84,34 @@ def test_filter_step_is_flow_noise_and_density(ctx, torch_gpu, orc):
         x = Xd[:, :P].clone()
     pf.close()
     net.close()
+
+
+@pytest.mark.parametrize("other_stream", [False, True])
+def test_inference_weights_follow_the_parameters(ctx, torch_gpu, other_stream):
+    """New parameters reach the fused kernel at the next call, also from a context on
+    another stream than the network's: equal to a network that had them from the start."""
+    torch = torch_gpu
+    norm = capi.SurrogateNorm(x_shift=2.3, x_scale=3.6, par_shift=8.0, par_scale=1.0,
+                              dx_scale=0.3)
+    X = torch.randn((40, 1000), device="cuda")
+    new = capi.MLP(ctx, surrogate.DIMS, seed=9)
+    net = capi.MLP(ctx, surrogate.DIMS, seed=4)
+    user = net
+    s = torch.cuda.Stream()
+    if other_stream:
+        torch.cuda.synchronize()  # X was made on torch's stream
+        c2 = capi.Context(0, stream=s)
+        user = capi.MLP.__new__(capi.MLP)
+        user.ctx, user.dims, user.h = c2, net.dims, net.h
+    first = user.surrogate_flow(norm, 8.1, X)
+    net.set_params(new.get_params())
+    second = user.surrogate_flow(norm, 8.1, X)
+    torch.cuda.synchronize()
+    ref = new.surrogate_flow(norm, 8.1, X)
+    torch.cuda.synchronize()
+    assert torch.equal(second, ref) and not torch.equal(first, ref)
+    if other_stream:
+        user.h = None
+        c2.close()
+    net.close()
+    new.close()
