@@ -6,7 +6,7 @@ integrator."""
 import numpy as np
 import pytest
 
-from libbi_amd import capi
+from libbi_amd import capi, surrogate
 
 pytestmark = pytest.mark.gpu
 
