@@ -17,10 +17,14 @@
 //
 // Network 301-256-256-256-400 (outputs: m for 200 dimensions, then s), BF16
 // MFMA with FP32 accumulation, laid out as the surrogate kernel's (32
-// particles per wave, weights staged in LDS in row chunks, activations in
-// registers).  The inference weights of the output layer interleave the rows
+// particles per wave, weights staged in LDS in row chunks that are copied
+// while the chunk before is computed, activations in registers).  2^17
+// particles take 0.160 ms (508 TFLOP/s); with every state of the output read
+// behind the store before it and the chunks loaded between barriers, 0.233 ms.  The inference weights of the output layer interleave the rows
 // per 16 dimensions (m of dimensions 16 t .. 16 t + 15, then their s), so one
 // 32-row output tile carries both numbers of the dimensions it covers.
+#include <type_traits>
+
 #include "blockreduce.hpp"
 #include "internal.hpp"
 #include "mlp.hpp"
@@ -58,13 +62,16 @@ constexpr int GP_THREADS = 512, GP_TILE = 256;
 constexpr int GD = 200, GNOBS = 100, GH = 256;
 constexpr int GK0 = 320;                 // 301 inputs padded
 constexpr int GOUT_TILES = (GD + 15) / 16;  // 13 tiles of 16 dimensions (m and s)
-constexpr int LDSK_H = GH + 8, LDSK_0 = GK0 + 8;
+constexpr int GHR = GH / 2;              // rows of a chunk of a hidden layer
+constexpr int G0R = 64;                  // rows of a chunk of layer 0
 
 template <bool FILTER>
 __global__ __launch_bounds__(GP_THREADS) void k_guided(GuidedArgs a) {
-  // layer 0 is staged in two halves of 128 rows (168 KB would not fit)
-  constexpr int LDS_ELEMS = GH * LDSK_H > 128 * LDSK_0 ? GH * LDSK_H : 128 * LDSK_0;
-  __shared__ __attribute__((aligned(16))) uint16_t Ws[LDS_ELEMS];
+  // two chunks of weights (stage_async) and the biases: 128 KB + 4.7 KB
+  static_assert(StagedRows<GK0>::bytes(G0R) <= StagedRows<GH>::bytes(GHR), "chunks of layer 0");
+  __shared__ __attribute__((aligned(16))) uint8_t buf[2][StagedRows<GH>::bytes(GHR)];
+  __shared__ __attribute__((aligned(16))) float bias[3 * GH + 32 * GOUT_TILES];
+  __shared__ double ys[GNOBS];  // the step's observations
 
   if constexpr (FILTER) {
     const long f = blockIdx.y;
@@ -75,6 +82,10 @@ __global__ __launch_bounds__(GP_THREADS) void k_guided(GuidedArgs a) {
     a.batch += (uint32_t)f;
     if (a.par_u_bank != nullptr) a.par_u = a.par_u_bank[f];
   }
+  stage_async<G0R, GK0, GP_THREADS>(a.W[0], 0, buf[0]);
+#pragma unroll
+  for (int l = 0; l < 4; ++l)
+    copy_floats(a.b[l], l < 3 ? GH : 32 * GOUT_TILES, bias + l * GH, GP_THREADS);
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, h = lane >> 5;
   const int p = blockIdx.x * GP_TILE + w * 32 + (lane & 31);
   const bool active = p < a.P;
@@ -92,7 +103,11 @@ __global__ __launch_bounds__(GP_THREADS) void k_guided(GuidedArgs a) {
     y = a.y_base + (size_t)a.dev->k * a.nobs;
   }
 
-  // layer-0 operand: inputs 16 c + 8 h + j
+  if (tid < GNOBS) ys[tid] = y[tid];
+  __syncthreads();
+
+  // layer-0 operand: inputs 16 c + 8 h + j; the loads without a branch (a
+  // particle past the end reads particle 0), so that many are in flight
   uint32_t in0[GK0 / 16][4];
 #pragma unroll
   for (int c = 0; c < GK0 / 16; ++c) {
@@ -105,7 +120,7 @@ __global__ __launch_bounds__(GP_THREADS) void k_guided(GuidedArgs a) {
         v = (a.X[(size_t)f * a.ld + pc] - a.x_shift) * a.x_inv_scale;
       } else if (f < GD + GNOBS) {
         const int o = f - GD;
-        v = (float)(y[o] - (double)a.X[(size_t)(2 * o) * a.ld + pc]) * a.innov_inv;
+        v = (float)(ys[o] - (double)a.X[(size_t)(2 * o) * a.ld + pc]) * a.innov_inv;
       } else if (f == GD + GNOBS) {
         v = a.par_u;
       }
@@ -113,64 +128,104 @@ __global__ __launch_bounds__(GP_THREADS) void k_guided(GuidedArgs a) {
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j) in0[c][j] = pack_bf2(u[2 * j], u[2 * j + 1]);
+    // at most 32 loads in flight: all 310 of them would spill
+    if ((c & 3) == 3) __builtin_amdgcn_sched_barrier(0);
   }
 
   uint32_t cur[GH / 16][4], nxt[GH / 16][4];
-  stage_rows<128, GK0, LDSK_0, GP_THREADS>(a.W[0], 0, Ws);
-  __syncthreads();
-  gelu_tiles<GK0 / 16, GH / 16, LDSK_0, 0, 4>(Ws, a.b[0], in0, nxt, lane);
-  __syncthreads();
-  stage_rows<128, GK0, LDSK_0, GP_THREADS>(a.W[0], 128, Ws);
-  __syncthreads();
-  gelu_tiles<GK0 / 16, GH / 16, LDSK_0, 4, 8>(Ws, a.b[0], in0, nxt, lane);
-  __syncthreads();
-  stage_rows<GH, GH, LDSK_H, GP_THREADS>(a.W[1], 0, Ws);
-  __syncthreads();
-  gelu_tiles<GH / 16, GH / 16, LDSK_H, 0, 8>(Ws, a.b[1], nxt, cur, lane);
-  __syncthreads();
-  stage_rows<GH, GH, LDSK_H, GP_THREADS>(a.W[2], 0, Ws);
-  __syncthreads();
-  gelu_tiles<GH / 16, GH / 16, LDSK_H, 0, 8>(Ws, a.b[2], cur, nxt, lane);
+  // each chunk of rows is copied while the one before is computed
+  stage_wait();
+  stage_async<G0R, GK0, GP_THREADS>(a.W[0], G0R, buf[1]);
+  gelu_tiles<GK0 / 16, GH / 16, GK0, 0, 2>(buf[0], bias, in0, nxt, lane);
+  stage_wait();
+  stage_async<G0R, GK0, GP_THREADS>(a.W[0], 2 * G0R, buf[0]);
+  gelu_tiles<GK0 / 16, GH / 16, GK0, 2, 4>(buf[1], bias, in0, nxt, lane);
+  stage_wait();
+  stage_async<G0R, GK0, GP_THREADS>(a.W[0], 3 * G0R, buf[1]);
+  gelu_tiles<GK0 / 16, GH / 16, GK0, 4, 6>(buf[0], bias, in0, nxt, lane);
+  stage_wait();
+  stage_async<GHR, GH, GP_THREADS>(a.W[1], 0, buf[0]);
+  gelu_tiles<GK0 / 16, GH / 16, GK0, 6, 8>(buf[1], bias, in0, nxt, lane);
+  stage_wait();
+  stage_async<GHR, GH, GP_THREADS>(a.W[1], GHR, buf[1]);
+  gelu_tiles<GH / 16, GH / 16, GH, 0, 4>(buf[0], bias + GH, nxt, cur, lane);
+  stage_wait();
+  stage_async<GHR, GH, GP_THREADS>(a.W[2], 0, buf[0]);
+  gelu_tiles<GH / 16, GH / 16, GH, 4, 8>(buf[1], bias + GH, nxt, cur, lane);
+  stage_wait();
+  stage_async<GHR, GH, GP_THREADS>(a.W[2], GHR, buf[1]);
+  gelu_tiles<GH / 16, GH / 16, GH, 0, 4>(buf[0], bias + 2 * GH, cur, nxt, lane);
+  stage_wait();
+  stage_async<GHR, GH, GP_THREADS>(a.W[3], 0, buf[0]);
+  gelu_tiles<GH / 16, GH / 16, GH, 4, 8>(buf[1], bias + 2 * GH, cur, nxt, lane);
 
   // output layer in chunks of four tiles; each tile: 16 dimensions (m, s)
   const double inv_obs = 1.0 / a.obs_sd;
   const double c_obs = -HALF_LOG_TWO_PI - log(a.obs_sd);
   double acc_w = 0.0;
+  // this lane's states of output tile t (dimensions 16 t + 8 q + 4 h + i), read
+  // one tile ahead of their use
+  auto load_tile = [&](int t, float (&x)[8]) {
 #pragma unroll
-  for (int t0 = 0; t0 < GOUT_TILES; t0 += 4) {
-    constexpr int CH = 4;
-    const int nt = GOUT_TILES - t0 < CH ? GOUT_TILES - t0 : CH;  // tiles in this chunk
-    __syncthreads();
-    stage_rows_n<GH, LDSK_H, GP_THREADS>(a.W[3], 32 * t0, 32 * nt, Ws);
-    __syncthreads();
+    for (int q = 0; q < 2; ++q)
 #pragma unroll
-    for (int dt = 0; dt < CH; ++dt) {
-      const int t = t0 + dt;
-      if (dt >= nt) break;
-      const f32x16 o = linear_tile<GH / 16, LDSK_H>(Ws, t, t0, a.b[3], nxt, lane);
+      for (int i = 0; i < 4; ++i)
+        if (16 * t + 8 * q < GD) x[4 * q + i] = a.X[(size_t)(16 * t + 8 * q + 4 * h + i) * a.ld + pc];
+  };
+  float xn[8];
+  load_tile(0, xn);
+  // chunk AT of up to four tiles, in buffer AT % 2
+  auto chunk = [&](auto at_c) {
+    constexpr int AT = decltype(at_c)::value, T0 = 4 * AT;
+    constexpr int NT = GOUT_TILES - T0 < 4 ? GOUT_TILES - T0 : 4;
+    constexpr int LEFT = GOUT_TILES - T0 - 4;  // tiles after this chunk
+    stage_wait();
+    if constexpr (LEFT > 0)
+      stage_async<32 * (LEFT < 4 ? LEFT : 4), GH, GP_THREADS>(a.W[3], 32 * (T0 + 4),
+                                                              buf[(AT + 1) & 1]);
+#pragma unroll
+    for (int dt = 0; dt < NT; ++dt) {
+      const int t = T0 + dt;
+      float xt[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) xt[i] = xn[i];
+      if (t + 1 < GOUT_TILES) load_tile(t + 1, xn);
+      const f32x16 o = linear_tile<GH / 16, GH>(buf[AT & 1], dt, t, bias + 3 * GH, nxt, lane);
 #pragma unroll
       for (int q = 0; q < 2; ++q) {
-        const int f0 = 16 * t + 8 * q + 4 * h;  // dimensions f0 .. f0 + 3
-        if (f0 >= GD || !active) continue;
-        float z[4];
-        normals4<float>(a.seed, (uint32_t)p, step, TAG_NOISE, a.batch, (uint32_t)(f0 >> 2), z);
+        if (16 * t + 8 * q < GD) {
+          const int f0 = 16 * t + 8 * q + 4 * h;  // dimensions f0 .. f0 + 3
+          float z[4];
+          normals4<float>(a.seed, (uint32_t)p, step, TAG_NOISE, a.batch, (uint32_t)(f0 >> 2), z);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int f = f0 + i;
-          const float m = o[4 * q + i], s = o[8 + 4 * q + i];
-          const float d = m + __expf(0.5f * s) * z[i];  // (x' - Phi) / q
-          float* xp = &a.X[(size_t)f * a.ld + p];
-          const float x = *xp + a.q * d;
-          *xp = x;
-          acc_w += (double)(-0.5f * d * d + 0.5f * z[i] * z[i] + 0.5f * s);
-          if ((f & 1) == 0) {
-            const double e = (y[f >> 1] - (double)x) * inv_obs;
-            acc_w += -0.5 * (e * e) + c_obs;
+          for (int i = 0; i < 4; ++i) {
+            const int f = f0 + i;
+            const float m = o[4 * q + i], s = o[8 + 4 * q + i];
+            const float d = m + __expf(0.5f * s) * z[i];  // (x' - Phi) / q
+            const float x = xt[4 * q + i] + a.q * d;
+            xt[4 * q + i] = x;
+            acc_w += (double)(-0.5f * d * d + 0.5f * z[i] * z[i] + 0.5f * s);
+            if ((i & 1) == 0) {
+              const double e = (ys[f >> 1] - (double)x) * inv_obs;
+              acc_w += -0.5 * (e * e) + c_obs;
+            }
           }
+          if (active) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) a.X[(size_t)(f0 + i) * a.ld + p] = xt[4 * q + i];
+          }
+          // keep the sum here: moved to its use after the last tile, it would
+          // hold every tile's values in registers until then
+          asm volatile("" : "+v"(acc_w));
         }
       }
     }
-  }
+  };
+  static_assert(GOUT_TILES > 12 && GOUT_TILES <= 16, "four chunks");
+  chunk(std::integral_constant<int, 0>{});
+  chunk(std::integral_constant<int, 1>{});
+  chunk(std::integral_constant<int, 2>{});
+  chunk(std::integral_constant<int, 3>{});
   acc_w += __shfl_xor(acc_w, 32, WAVE);  // the particle's other half-wave
   if constexpr (FILTER) {
     double lw = __builtin_nan("");

@@ -11,13 +11,22 @@
 //
 // Layout: a workgroup of 8 waves takes 256 particles, 32 per wave.  Each
 // layer is computed transposed, out^T = W in^T, with the weights as the MFMA
-// A operand (staged in LDS, one layer at a time) and the activations as the B
-// operand, held in registers: the accumulator of an output tile lands in the
-// lane that owns the particle, so it becomes the next layer's B operand
-// without any data movement.  The accumulator's row order inside a 16-wide
-// k block ([0-3, 8-11, 4-7, 12-15] across the two half-waves) is absorbed by
-// storing the weights of layers l >= 1 with their input columns permuted the
-// same way (mlp_capi.cpp, inference weights).
+// A operand and the activations as the B operand, held in registers: the
+// accumulator of an output tile lands in the lane that owns the particle, so
+// it becomes the next layer's B operand without any data movement.  The
+// accumulator's row order inside a 16-wide k block ([0-3, 8-11, 4-7, 12-15]
+// across the two half-waves) is absorbed by storing the weights of layers
+// l >= 1 with their input columns permuted the same way (the inference
+// weights).  The weights pass through LDS in chunks of 128 rows, each copied
+// while the one before is computed (mlp.hpp).
+//
+// What bounds it: 2^20 particles take 0.416 ms (762 TFLOP/s, 30% of the dense
+// bf16 rate).  Before, every layer was loaded through registers behind two
+// barriers, and the input and output states were read one load after another
+// (each behind its own branch): 0.94 ms, 60% of the wave cycles waiting, now
+// 40%.  The rest is vector work: 4450 vector instructions a wave, an
+// exponential and a reciprocal per activation among them, at two waves per
+// SIMD (182 registers).
 #include "blockreduce.hpp"
 #include "internal.hpp"
 #include "mlp.hpp"
@@ -57,9 +66,13 @@ template <int D, int H, int NL, bool STEP>
 __global__ __launch_bounds__(SG_THREADS) void k_surrogate(SurrArgs a) {
   constexpr int K0 = (D + 1 + 63) / 64 * 64;  // padded input width (state + parameter)
   constexpr int DO = (D + 63) / 64 * 64;      // padded output width
-  constexpr int LDSK = H + 8;                 // LDS row stride (bank spread)
-  static_assert(NL >= 2 && H % 32 == 0 && K0 <= H && DO <= H, "surrogate shape");
-  __shared__ __attribute__((aligned(16))) uint16_t Ws[H * LDSK];
+  constexpr int HR = H / 2, HT = H / 64;      // rows and tiles of half a hidden layer
+  static_assert(D % 8 == 0 && NL == 4 && StagedRows<K0>::bytes(H) <= StagedRows<H>::bytes(HR) && DO <= HR,
+                "surrogate shape");
+  // two chunks of weights (stage_async) and the biases: 128 KB + 3.3 KB
+  __shared__ __attribute__((aligned(16))) uint8_t buf[2][StagedRows<H>::bytes(HR)];
+  __shared__ __attribute__((aligned(16))) float bias[3 * H + DO];
+  __shared__ double ys[STEP ? D / 2 : 1];  // the step's observations
 
   if constexpr (STEP) {
     const long f = blockIdx.y;
@@ -72,6 +85,10 @@ __global__ __launch_bounds__(SG_THREADS) void k_surrogate(SurrArgs a) {
     a.batch += (uint32_t)f;
     if (a.par_u_bank != nullptr) a.par_u = a.par_u_bank[f];
   }
+  stage_async<H, K0, SG_THREADS>(a.W[0], 0, buf[0]);
+#pragma unroll
+  for (int l = 0; l < NL; ++l)
+    copy_floats(a.b[l], l + 1 < NL ? H : DO, bias + l * H, SG_THREADS);
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, h = lane >> 5;
   const int p = blockIdx.x * SG_TILE + w * 32 + (lane & 31);
   const bool active = p < a.P;
@@ -88,6 +105,7 @@ __global__ __launch_bounds__(SG_THREADS) void k_surrogate(SurrArgs a) {
     const int k = a.dev->k;
     step = (uint32_t)(k + 1);
     y = a.y_base + (size_t)k * a.nobs;
+    if (tid < D / 2) ys[tid] = y[tid];  // read after the chunks' barriers
   }
   const int src = active ? (gather ? a.as[p] : p) : 0;
 
@@ -98,52 +116,54 @@ __global__ __launch_bounds__(SG_THREADS) void k_surrogate(SurrArgs a) {
     float u[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
+      // loads without a branch (a particle past the end reads particle 0, a
+      // feature past the last that one), so that they all are in flight together
       const int f = 16 * c + 8 * h + j;
       u[j] = 0.0f;
-      if (f < D) {
-        if (active) u[j] = (a.Xin[(size_t)f * a.ld + src] - a.x_shift) * a.x_inv_scale;
-      } else if (f == D) {
-        u[j] = a.par_u;
+      if (16 * c + j < D) {
+        const float x = a.Xin[(size_t)(f < D ? f : D - 1) * a.ld + src];
+        u[j] = (x - a.x_shift) * a.x_inv_scale;
       }
+      if (16 * c + 8 + j >= D) u[j] = f < D ? u[j] : (f == D ? a.par_u : 0.0f);
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j) in0[c][j] = pack_bf2(u[2 * j], u[2 * j + 1]);
   }
 
-  // hidden layers
-  stage_rows<H, K0, LDSK, SG_THREADS>(a.W[0], 0, Ws);
-  __syncthreads();
-  gelu_tiles<K0 / 16, H / 16, LDSK, 0, H / 32>(Ws, a.b[0], in0, nxt, lane);
+  // hidden layers: each chunk of rows is copied while the one before is computed
+  stage_wait();
+  stage_async<HR, H, SG_THREADS>(a.W[1], 0, buf[1]);
+  gelu_tiles<K0 / 16, H / 16, K0, 0, 2 * HT>(buf[0], bias, in0, nxt, lane);
+  stage_wait();
+  stage_async<HR, H, SG_THREADS>(a.W[1], HR, buf[0]);
+  gelu_tiles<H / 16, H / 16, H, 0, HT>(buf[1], bias + H, nxt, cur, lane);
+  stage_wait();
+  stage_async<HR, H, SG_THREADS>(a.W[2], 0, buf[1]);
+  gelu_tiles<H / 16, H / 16, H, HT, 2 * HT>(buf[0], bias + H, nxt, cur, lane);
+  stage_wait();
+  stage_async<HR, H, SG_THREADS>(a.W[2], HR, buf[0]);
+  gelu_tiles<H / 16, H / 16, H, 0, HT>(buf[1], bias + 2 * H, cur, nxt, lane);
+  stage_wait();
+  stage_async<DO, H, SG_THREADS>(a.W[3], 0, buf[1]);
+  gelu_tiles<H / 16, H / 16, H, HT, 2 * HT>(buf[0], bias + 2 * H, cur, nxt, lane);
+
+  // the states of the output's features 32 t + acc_row(r, lane), again
+  float xv[DO / 32][16];
 #pragma unroll
-  for (int l = 1; l < NL - 1; ++l) {
-    __syncthreads();  // every wave is done with the previous layer's weights
-    stage_rows<H, H, LDSK, SG_THREADS>(a.W[l], 0, Ws);
-    __syncthreads();
-    if (l & 1) gelu_tiles<H / 16, H / 16, LDSK, 0, H / 32>(Ws, a.b[l], nxt, cur, lane);
-    else gelu_tiles<H / 16, H / 16, LDSK, 0, H / 32>(Ws, a.b[l], cur, nxt, lane);
-  }
-  const uint32_t(&last)[H / 16][4] = ((NL - 2) & 1) ? cur : nxt;
+  for (int t = 0; t < DO / 32; ++t)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int f = 32 * t + acc_row(r, lane);
+      if (32 * t + 8 * (r >> 2) < D)
+        xv[t][r] = a.Xin[(size_t)f * a.ld + src];
+    }
 
   // output layer: y for features 32 t + acc_row(r, lane)
-  __syncthreads();
-  stage_rows<DO, H, LDSK, SG_THREADS>(a.W[NL - 1], 0, Ws);
-  __syncthreads();
-  float yv[DO / 32][16];
+  stage_wait();
+  f32x16 yv[DO / 32];
 #pragma unroll
-  for (int t = 0; t < DO / 32; ++t) {
-    f32x16 acc;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
-#pragma unroll
-    for (int c = 0; c < H / 16; ++c) {
-      const u16x8 wa = *reinterpret_cast<const u16x8*>(
-          &Ws[(32 * t + (lane & 31)) * LDSK + 16 * c + 8 * h]);
-      const u32v4 bv = {last[c][0], last[c][1], last[c][2], last[c][3]};
-      acc = mfma32(wa, bv, acc);
-    }
-#pragma unroll
-    for (int r = 0; r < 16; ++r) yv[t][r] = acc[r] + a.b[NL - 1][32 * t + acc_row(r, lane)];
-  }
+  for (int t = 0; t < DO / 32; ++t)
+    yv[t] = linear_tile<H / 16, H>(buf[1], t, t, bias + 3 * H, nxt, lane);
 
   // x' = x + s_dx y (+ noise), observation density over the even dimensions
   double obs = 0.0;
@@ -153,22 +173,25 @@ __global__ __launch_bounds__(SG_THREADS) void k_surrogate(SurrArgs a) {
   for (int t = 0; t < DO / 32; ++t) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
+      if (32 * t + 8 * q >= D) continue;
       const int f0 = 32 * t + 8 * q + 4 * h;  // four consecutive features f0 .. f0 + 3
-      if (f0 >= D) continue;
       float z[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-      if (STEP && active) normals4<float>(a.seed, (uint32_t)p, step, TAG_NOISE, a.batch,
-                                          (uint32_t)(f0 >> 2), z);
+      if (STEP) normals4<float>(a.seed, (uint32_t)p, step, TAG_NOISE, a.batch,
+                                (uint32_t)(f0 >> 2), z);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int f = f0 + i;
-        if (f >= D || !active) continue;
-        float x = a.Xin[(size_t)f * a.ld + src] + a.dx_scale * yv[t][4 * q + i];
+        float x = xv[t][4 * q + i] + a.dx_scale * yv[t][4 * q + i];
         if (STEP) x = x + a.noise_sd * z[i];
-        a.Xout[(size_t)f * a.ld + p] = x;
-        if (STEP && (f & 1) == 0) {
-          const double e = (y[f >> 1] - (double)x) * inv_obs;
+        xv[t][4 * q + i] = x;
+        if (STEP && (i & 1) == 0) {
+          const double e = (ys[f >> 1] - (double)x) * inv_obs;
           obs += -0.5 * (e * e) + c_obs;
         }
+      }
+      if (active) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) a.Xout[(size_t)(f0 + i) * a.ld + p] = xv[t][4 * q + i];
       }
     }
   }

@@ -3,10 +3,12 @@ uses it (bihip_pf_set_surrogate): the fused kernel against the GEMM path and
 the oracle's MLP, the filter step against its composition (flow, Philox
 noise, observation density), and a trained surrogate against the exact
 integrator."""
+import ctypes
+
 import numpy as np
 import pytest
 
-from libbi_amd import capi, surrogate
+from libbi_amd import capi, guided, surrogate
 
 pytestmark = pytest.mark.gpu
 
@@ -115,3 +117,37 @@ def test_inference_weights_follow_the_parameters(ctx, torch_gpu, other_stream):
         c2.close()
     net.close()
     new.close()
+
+
+@pytest.mark.parametrize("P", [1, 31, 33, 256, 257, 600])
+def test_fused_networks_at_ragged_particle_counts(ctx, torch_gpu, P):
+    """Particles around a wave's 32 and a workgroup's 256: the same bits as in a larger
+    batch, the columns past the last particle untouched."""
+    torch = torch_gpu
+    big, ld = 700, 700
+    norm = _norm()
+    net = capi.MLP(ctx, surrogate.DIMS, seed=4)
+    X = torch.from_numpy(_states(big, seed=3)).cuda()
+    ref = net.surrogate_flow(norm, 8.1, X)
+    out = torch.full_like(X, 7.0)
+    capi.check(capi.lib().bihip_surrogate_flow(ctx.h, net.h, ctypes.byref(norm), 8.1, capi.ptr(X),
+                                               capi.ptr(out), ld, P))
+    assert torch.equal(out[:, :P], ref[:, :P]) and bool((out[:, P:] == 7.0).all())
+    net.close()
+
+    gnorm = capi.GuidedNorm(x_shift=2.3, x_scale=3.6, innov_scale=1.0, par_shift=8.0,
+                            par_scale=1.0)
+    gnet = capi.MLP(ctx, guided.DIMS, seed=5)
+    Phi = 2.3 + 3.6 * torch.randn((200, big), device="cuda")
+    y = torch.randn(100, dtype=torch.float64, device="cuda")
+    got = []
+    for n in (big, P):
+        Z, inc = Phi.clone(), torch.full((big,), 7.0, dtype=torch.float64, device="cuda")
+        capi.check(capi.lib().bihip_guided_propose(
+            ctx.h, gnet.h, ctypes.byref(gnorm), 8.2, capi.ptr(Z), ld, n, capi.ptr(y), 5, 2, 3,
+            0.1, 1.0, capi.ptr(inc)))
+        got.append((Z, inc))
+    (Za, ia), (Zb, ib) = got
+    assert torch.equal(Zb[:, :P], Za[:, :P]) and torch.equal(Zb[:, P:], Phi[:, P:])
+    assert torch.equal(ib[:P], ia[:P]) and bool((ib[P:] == 7.0).all())
+    gnet.close()
