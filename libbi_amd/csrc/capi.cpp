@@ -746,8 +746,8 @@ static int pf_enqueue_step(bihip_pf* pf, hipStream_t s, int timing) {
   R.ws = pf->ws;
   R.mc = pf->mc_buf != nullptr ? &pf->mc : nullptr;
   // the previous correct step stored the tile weight sums (fixed per filter)
-  const bool stored_sums =
-      correct_stores_sums(pf->nparts) && ceil_div(P, SCAN_TILE) <= pf->ws.max_tiles;
+  const bool stored_sums = !resample_in_one_block(P) && correct_stores_sums(pf->nparts) &&
+                           ceil_div(P, SCAN_TILE) <= pf->ws.max_tiles;
   R.sums_ready = stored_sums ? 1 : 0;
   if (pf->imp_r == nullptr) {
     if ((rc = launch_resample_tiles(R, s))) return rc;

@@ -307,6 +307,8 @@ struct ResampleTilesLaunch {
 // Where the tiled chain keeps its tile weight sums (2 words per tile).
 uint64_t* tile_sum_words(const ScanWorkspace& ws);
 int launch_resample_tiles(const ResampleTilesLaunch& L, hipStream_t s);
+// The chain runs as one workgroup per filter (it sums the weights itself).
+bool resample_in_one_block(int P);
 struct MultinomialLaunch {
   const double* Ws;
   int P, n;

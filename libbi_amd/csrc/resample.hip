@@ -610,6 +610,191 @@ int launch_ancestors_permute(const int* in, bool cumulative, int P, int* as, uin
   return place_from_sums(in, cumulative, P, nt, as, EF, w, gate, s);
 }
 
+// ---------------------------------------------------------------- small filters
+// The whole chain of one filter of at most SMALL_CHAIN particles in one
+// workgroup: weights, offspring and ancestors without a launch or a trip to
+// memory between them, ITEMS consecutive particles a thread.  The same exact
+// integer sums and expressions as the tiled chain, so the same ancestors.
+//
+// Bound by its latency (two block scans, the FP64 weights and quotients of
+// ITEMS particles on one CU, a search of log2 P LDS reads), where the chain's
+// three or four launches cost about that latency each.  A predator-prey step
+// (graph replay): systematic 30.1 -> 21.9 us at 1000 particles, 32.4 -> 27.8
+// at 4096, multinomial 43.9 -> 23.0 and 56.6 -> 35.6; a bank of 64 x 4096 46.7
+// -> 37.5.  At 8192 (eight particles a thread) it lost to the tiles, 37.3
+// against 32.5 us, so the line lies at 4096.
+constexpr int SMALL_BLOCK = 1024;
+constexpr int SMALL_CHAIN = 4 * SMALL_BLOCK;
+
+struct SmallChainArgs {
+  const double* lws;
+  const double* mx;
+  int P, n;
+  uint64_t seed;
+  uint32_t batch;
+  const PFDevice* gate;
+  PFDevice* status;
+  int* as;
+  BankStrides bk;
+};
+
+// Inclusive scan of one value per thread over the workgroup's waves; total
+// receives the sum.
+template <class V>
+__device__ __forceinline__ V small_inclusive_scan(V v, V* lds, V& total) {
+  constexpr int NW = SMALL_BLOCK / WAVE;
+  const int lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE;
+#pragma unroll
+  for (int o = 1; o < WAVE; o <<= 1) {
+    const V u = shfl_up_v(v, o);
+    if (lane >= o) v = u + v;
+  }
+  if (lane == WAVE - 1) lds[w] = v;
+  __syncthreads();
+  V pre(0), tot(0);
+#pragma unroll
+  for (int i = 0; i < NW; ++i) {
+    const V x = lds[i];
+    if (i < w) pre = pre + x;
+    tot = tot + x;
+  }
+  total = tot;
+  return pre + v;
+}
+
+template <int MODE, int ITEMS>
+__global__ __launch_bounds__(SMALL_BLOCK) void k_resample_small(SmallChainArgs a) {
+  constexpr int N = SMALL_BLOCK * ITEMS;
+  __shared__ u128 l128[SMALL_BLOCK / WAVE];
+  __shared__ uint64_t l64[SMALL_BLOCK / WAVE];
+  __shared__ uint16_t E[N];
+  __shared__ double Ws[MODE == BIHIP_MULTINOMIAL ? N : 1];
+  __shared__ int count[MODE == BIHIP_MULTINOMIAL ? N : 1];
+  static_assert(N <= 1 << 16, "E holds 16-bit sums of extra copies");
+  {
+    const long f = bank_f();
+    a.lws = bank_shift(a.lws, f * a.bk.p * 8);
+    a.mx = bank_shift(a.mx, f * DEV_BYTES);
+    a.batch += (uint32_t)f;
+    a.gate = bank_shift(a.gate, f * DEV_BYTES);
+    a.status = bank_shift(a.status, f * DEV_BYTES);
+    a.as = bank_shift(a.as, f * a.bk.p * 4);
+  }
+  const int base = (int)threadIdx.x * ITEMS;
+  double lw[ITEMS];
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i) lw[i] = base + i < a.P ? a.lws[base + i] : 0.0;
+  const double m = *a.mx;
+  if (!gate_open(a.gate)) return;
+  const uint32_t step = (uint32_t)a.gate->k;
+
+  // inclusive fixed-point weight sums
+  u128 v[ITEMS];
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i)
+    v[i] = base + i < a.P ? fix_weight(nanexp(lw[i] - m)) : u128(0);
+#pragma unroll
+  for (int i = 1; i < ITEMS; ++i) v[i] = v[i - 1] + v[i];
+  u128 tot;
+  const u128 start = small_inclusive_scan(v[ITEMS - 1], l128, tot) - v[ITEMS - 1];
+  const double W = fix_to_double(tot);
+  if (!(W > 0.0)) {
+    if (a.status != nullptr && threadIdx.x == 0) a.status->status = BIHIP_DEGENERATE;
+    return;
+  }
+
+  // offspring counts
+  int o[ITEMS];
+  if constexpr (MODE == BIHIP_MULTINOMIAL) {
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+      Ws[base + i] = fix_to_double(start + v[i]);
+      count[base + i] = 0;
+    }
+    __syncthreads();
+    for (int j = threadIdx.x; j < a.n; j += SMALL_BLOCK) {
+      const u32x4 r = philox_block(a.seed, (uint32_t)j, step, TAG_MULTINOMIAL, a.batch, 0);
+      const double u = W * u53(r.x, r.y);
+      int lo = 0, hi = a.P;  // first i with Ws_i > u
+      while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (Ws[mid] <= u) lo = mid + 1;
+        else hi = mid;
+      }
+      atomicAdd(&count[lo < a.P ? lo : a.P - 1], 1);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) o[i] = base + i < a.P ? count[base + i] : 1;
+  } else {
+    double av = 0.0;
+    if (MODE == BIHIP_SYSTEMATIC) {
+      const u32x4 r = philox_block(a.seed, 0, step, TAG_SYSTEMATIC, a.batch, 0);
+      av = u53(r.x, r.y);
+    }
+    auto cumulative = [&](const u128& incl) -> int {
+      const double Wsi = fix_to_double(incl);
+      if (MODE == BIHIP_SYSTEMATIC) return systematic_offspring(Wsi, W, a.n, av);
+      const double reach = stratified_reach(Wsi, W, a.n);
+      int k = (int)reach;
+      if (k > a.n - 1) k = a.n - 1;
+      const u32x4 r = philox_block(a.seed, (uint32_t)k, step, TAG_STRATIFIED, a.batch, 0);
+      return stratified_offspring(reach, u53(r.x, r.y), a.n);
+    };
+    int prev = base > 0 && base < a.P ? cumulative(start) : 0;
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+      o[i] = 1;  // past the end: no extras, not free
+      if (base + i < a.P) {
+        const int O = cumulative(start + v[i]);
+        o[i] = O - prev;
+        prev = O;
+      }
+    }
+  }
+
+  // exclusive sums of extra copies (E) and free slots
+  uint64_t t = 0;
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i) t += ef_pair(o[i]);
+  uint64_t eftot;
+  uint64_t run = small_inclusive_scan(t, l64, eftot) - t;
+  int rank[ITEMS];  // of a free slot; -1: occupied
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i) {
+    E[base + i] = (uint16_t)run;
+    rank[i] = o[i] == 0 ? (int)(run >> 32) : -1;
+    run += ef_pair(o[i]);
+  }
+  __syncthreads();
+
+  // the free slot of rank r receives the last i with E_i <= r
+  int pos[ITEMS];
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i) pos[i] = 0;  // E_0 = 0
+  for (int s = 1 << (31 - __clz(a.P)); s > 0; s >>= 1) {
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+      const int c = pos[i] + s;
+      if (c < a.P && (int)E[c] <= rank[i]) pos[i] = c;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i)
+    if (base + i < a.P) a.as[base + i] = rank[i] < 0 ? base + i : pos[i];
+}
+
+template <int MODE>
+static void launch_small(const SmallChainArgs& a, int banks, hipStream_t s) {
+  const dim3 grid(1, banks), block(SMALL_BLOCK);
+  if (a.P <= SMALL_BLOCK) hipLaunchKernelGGL((k_resample_small<MODE, 1>), grid, block, 0, s, a);
+  else if (a.P <= 2 * SMALL_BLOCK)
+    hipLaunchKernelGGL((k_resample_small<MODE, 2>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((k_resample_small<MODE, 4>), grid, block, 0, s, a);
+}
+
+bool resample_in_one_block(int P) { return P <= SMALL_CHAIN; }
+
 int launch_resample_tiles(const ResampleTilesLaunch& L, hipStream_t s) {
   if (L.P <= 0) return BIHIP_OK;
   if (L.gate == nullptr) return set_error(BIHIP_EINVAL, "the tiled resampling chain needs a gate");
@@ -619,6 +804,17 @@ int launch_resample_tiles(const ResampleTilesLaunch& L, hipStream_t s) {
   const int banks = L.banks > 1 ? L.banks : 1;
   if (banks > 1 && L.mode == BIHIP_MULTINOMIAL)
     return set_error(BIHIP_EINVAL, "filter banks resample systematically or stratified");
+  if (resample_in_one_block(L.P)) {
+    const SmallChainArgs a{L.lws, L.mx, L.P, L.n, L.seed, L.batch, L.gate, L.status, L.as, L.bk};
+    switch (L.mode) {
+      case BIHIP_SYSTEMATIC: launch_small<BIHIP_SYSTEMATIC>(a, banks, s); break;
+      case BIHIP_STRATIFIED: launch_small<BIHIP_STRATIFIED>(a, banks, s); break;
+      case BIHIP_MULTINOMIAL: launch_small<BIHIP_MULTINOMIAL>(a, banks, s); break;
+      default: return set_error(BIHIP_EINVAL, "unknown resampler %d", L.mode);
+    }
+    BIHIP_LAUNCH_CHECK();
+    return BIHIP_OK;
+  }
   if (!L.sums_ready) {
     hipLaunchKernelGGL(k_weight_sums, dim3(nt, banks), dim3(SCAN_BLOCK), 0, s, L.lws, L.mx, L.P,
                        w.wsum, L.gate, L.bk);

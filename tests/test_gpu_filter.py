@@ -49,6 +49,24 @@ def test_pz_filter_fp64_parity(ctx, orc, resampler):
 
 
 @pytest.mark.parametrize("resampler", [capi.SYSTEMATIC, capi.STRATIFIED, capi.MULTINOMIAL])
+@pytest.mark.parametrize("P", [1, 2, 63, 257, 1024, 1025, 2048, 2049, 4095, 4097])
+def test_pz_filter_small_population_parity(ctx, orc, P, resampler):
+    """One, two and four particles a thread of the one-workgroup resampling chain and
+    the first size past it: ancestors bit-exact, with weights concentrated on a few
+    particles (a sharp observation density) as well as spread."""
+    y = _pz_data(orc, 6)
+    for obs_sd in (0.2, 0.004):
+        gm = capi.make_model("pz", precision=capi.F64, obs_sd=obs_sd)
+        om = oracle_model(orc, gm)
+        logZ, out, anc = _run_gpu(ctx, gm, y, P, 1.0, 44, resampler, 1.0)
+        ref = orc.pf_run(om, y, P, 1.0, 44, resampler=resampler, ess_rel=1.0,
+                         want_ancestors=True)
+        assert logZ == pytest.approx(ref["logZ"], rel=1e-10)
+        np.testing.assert_array_equal(out["resampled"], ref["resampled"])
+        np.testing.assert_array_equal(anc, ref["ancestors"])
+
+
+@pytest.mark.parametrize("resampler", [capi.SYSTEMATIC, capi.STRATIFIED, capi.MULTINOMIAL])
 def test_pz_filter_large_population_parity(ctx, orc, resampler):
     """N = 2^21 + 5: more than 1024 tiles of 2048 particles, so the resampling
     chain scans its tile sums in a launch of their own; ancestors stay bit-exact."""
