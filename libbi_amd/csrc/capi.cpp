@@ -621,6 +621,7 @@ struct bihip_pf {
   bihip_pf_config cfg{};
   int ld = 0, elem = 4, nobs = 1, nparts = 0;
   bool one_delta = false;  // gen_one_delta over the run's steps
+  bool small = false;      // small_filter_fits: plain steps run in one workgroup
   void* X[2] = {nullptr, nullptr};
   int cur = 0;
   double* lws = nullptr;
@@ -891,6 +892,39 @@ static int pf_capture(bihip_pf* pf, int parity) {
   return rc;
 }
 
+// Whole steps in one workgroup (small_filter.hip): nothing but the plain step of
+// a small filter.
+static bool pf_small_steps(const bihip_pf* pf) {
+  return pf->small && !pf->timing && pf->imp_r == nullptr && pf->times == nullptr &&
+         pf->obs_mask == nullptr && pf->inputs == nullptr && !pf->surr && !pf->guided;
+}
+
+// At most this many steps a launch, so that no launch lasts long.
+constexpr int SMALL_STEPS = 128;
+
+static int pf_enqueue_small(bihip_pf* pf, int n, hipStream_t s) {
+  SmallFilterLaunch L{};
+  L.model = &pf->model;
+  L.X = pf->X[pf->cur];
+  L.Xother = pf->X[1 - pf->cur];
+  L.ld = pf->ld;
+  L.P = pf->cfg.P;
+  L.steps = n;
+  L.resampler = pf->cfg.resampler;
+  L.nobs = pf->nobs;
+  L.as = pf->as;
+  L.lws = pf->lws;
+  L.dev = pf->dev;
+  L.hist = PFHistory{pf->hist_li, pf->hist_ess, pf->hist_res};
+  L.y = pf->y;
+  L.t0 = pf->cfg.t0;
+  L.dt = pf->cfg.dt;
+  L.essRel = pf->cfg.essRel;
+  L.seed = pf->cfg.seed;
+  L.batch = pf->cfg.batch;
+  return launch_small_filter(L, s);
+}
+
 extern "C" {
 
 int bihip_pf_create(bihip_ctx* ctx, const bihip_model* m, const bihip_pf_config* cfg,
@@ -915,6 +949,7 @@ int bihip_pf_create(bihip_ctx* ctx, const bihip_model* m, const bihip_pf_config*
   pf->model = *m;
   pf->cfg = *cfg;
   pf->one_delta = gen_one_delta(m, cfg->t0, cfg->dt, cfg->T);
+  pf->small = cfg->record == 0 && small_filter_fits(m, cfg->P, pf->one_delta);
   const int P = cfg->P;
   pf->ld = (P + 63) / 64 * 64;
   pf->elem = bihip_model_elem_size(m);
@@ -1081,6 +1116,16 @@ int bihip_pf_step(bihip_pf* pf, int n) {
   int rc = ctx_enter(pf->ctx);
   if (rc) return rc;
   hipStream_t s = pf->ctx->stream;
+  if (pf_small_steps(pf)) {
+    while (n > 0) {
+      const int m = std::min(n, SMALL_STEPS);
+      if ((rc = pf_enqueue_small(pf, m, s))) return rc;
+      pf->cur = (pf->cur + m) & 1;
+      pf->k += m;
+      n -= m;
+    }
+    return BIHIP_OK;
+  }
   for (int i = 0; i < n; ++i) {
     if (pf->cfg.use_graph && !pf->timing) {
       if (pf->graph[pf->cur] == nullptr) {

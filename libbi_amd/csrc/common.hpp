@@ -132,9 +132,18 @@ __device__ __forceinline__ int xcd_block(int b, int nb) {
 // ---------------------------------------------------------------- wave helpers
 constexpr int WAVE = 64;
 
-template <class T>
-__device__ __forceinline__ T shfl_xor(T v, int mask) {
-  return __shfl_xor(v, mask, WAVE);
+// The value of the lane that a DPP control names (models.hpp and
+// blockreduce.hpp); every lane that is read must be active.
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xF, 0xF, true));
+}
+template <int CTRL>
+__device__ __forceinline__ double dpp(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_mov_dpp((int)b, CTRL, 0xF, 0xF, true);
+  const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), CTRL, 0xF, 0xF, true);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 
 }  // namespace bihip

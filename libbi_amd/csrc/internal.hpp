@@ -309,6 +309,26 @@ uint64_t* tile_sum_words(const ScanWorkspace& ws);
 int launch_resample_tiles(const ResampleTilesLaunch& L, hipStream_t s);
 // The chain runs as one workgroup per filter (it sums the weights itself).
 bool resample_in_one_block(int P);
+
+// ---- whole steps of a small filter in one workgroup (small_filter.hip): a lone
+// filter without schedule, inputs, recording, imposed history or networks
+struct SmallFilterLaunch {
+  const bihip_model* model;
+  void *X, *Xother;  // the current state and the other buffer, which take turns
+  int ld, P, steps, resampler, nobs;
+  int* as;
+  double* lws;
+  PFDevice* dev;
+  PFHistory hist;
+  const double* y;
+  double t0, dt, essRel;
+  uint64_t seed;
+  uint32_t batch;
+};
+// The model and size are compiled for it (one_delta: every interval of the
+// filter is one delta of its generated model, gen_one_delta).
+bool small_filter_fits(const bihip_model* m, int P, bool one_delta);
+int launch_small_filter(const SmallFilterLaunch& L, hipStream_t s);
 struct MultinomialLaunch {
   const double* Ws;
   int P, n;

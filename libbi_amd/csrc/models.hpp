@@ -52,18 +52,6 @@ constexpr int ROW_ROR15 = 0x12F;        // lane g reads g+1 (mod 16)
 constexpr int ROW_MIRROR = 0x140;       // lane g reads 15-g
 constexpr int ROW_HALF_MIRROR = 0x141;  // lane g reads 7-g within its eight
 
-template <int CTRL>
-__device__ __forceinline__ float dpp(float v) {
-  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xF, 0xF, true));
-}
-template <int CTRL>
-__device__ __forceinline__ double dpp(double v) {
-  const long long b = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_mov_dpp((int)b, CTRL, 0xF, 0xF, true);
-  const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), CTRL, 0xF, 0xF, true);
-  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
-
 template <int LPP>
 struct Group {
   int lane;  // lane in the wavefront

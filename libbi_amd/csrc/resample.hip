@@ -20,31 +20,11 @@
 #include <algorithm>
 
 #include "scan.hpp"
+#include "small_chain.hpp"
 
 namespace bihip {
 
 constexpr int RS_BLOCK = 256;
-
-// O_i = min(n, (int)(Ws_i / W * n + a)) with every operation rounded as
-// written (SystematicResampler.hpp:47-50).
-__device__ __forceinline__ int systematic_offspring(double Ws, double W, int n, double a) {
-#pragma clang fp contract(off)
-  const double v = Ws / W * (double)n + a;
-  const int o = (int)v;
-  return o < n ? o : n;
-}
-
-// StratifiedResamplerHost.hpp:68-71
-__device__ __forceinline__ double stratified_reach(double Ws, double W, int n) {
-#pragma clang fp contract(off)
-  return Ws / W * (double)n;
-}
-
-__device__ __forceinline__ int stratified_offspring(double reach, double alpha, int n) {
-#pragma clang fp contract(off)
-  const int o = (int)(reach + alpha);
-  return o < n ? o : n;
-}
 
 __device__ __forceinline__ bool gate_open(const PFDevice* g) {
   return g == nullptr || (g->resample != 0 && g->status == BIHIP_OK);
@@ -132,13 +112,6 @@ constexpr int SMALL_TILES = 1024;
 
 __device__ __forceinline__ int offspring_at(const int* in, bool cumulative, long i) {
   return cumulative ? in[i] - (i > 0 ? in[i - 1] : 0) : in[i];
-}
-
-// (e, f) = (max(o - 1, 0), [o == 0]) packed as e | f << 32.
-__device__ __forceinline__ uint64_t ef_pair(int o) {
-  const uint64_t e = o > 1 ? (uint64_t)(o - 1) : 0u;
-  const uint64_t f = o == 0 ? 1u : 0u;
-  return e | (f << 32);
 }
 
 // Regions of the workspace's tile-chain words (the upper half of each tile's
@@ -623,7 +596,6 @@ int launch_ancestors_permute(const int* in, bool cumulative, int P, int* as, uin
 // at 4096, multinomial 43.9 -> 23.0 and 56.6 -> 35.6; a bank of 64 x 4096 46.7
 // -> 37.5.  At 8192 (eight particles a thread) it lost to the tiles, 37.3
 // against 32.5 us, so the line lies at 4096.
-constexpr int SMALL_BLOCK = 1024;
 constexpr int SMALL_CHAIN = 4 * SMALL_BLOCK;
 
 struct SmallChainArgs {
@@ -638,39 +610,9 @@ struct SmallChainArgs {
   BankStrides bk;
 };
 
-// Inclusive scan of one value per thread over the workgroup's waves; total
-// receives the sum.
-template <class V>
-__device__ __forceinline__ V small_inclusive_scan(V v, V* lds, V& total) {
-  constexpr int NW = SMALL_BLOCK / WAVE;
-  const int lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE;
-#pragma unroll
-  for (int o = 1; o < WAVE; o <<= 1) {
-    const V u = shfl_up_v(v, o);
-    if (lane >= o) v = u + v;
-  }
-  if (lane == WAVE - 1) lds[w] = v;
-  __syncthreads();
-  V pre(0), tot(0);
-#pragma unroll
-  for (int i = 0; i < NW; ++i) {
-    const V x = lds[i];
-    if (i < w) pre = pre + x;
-    tot = tot + x;
-  }
-  total = tot;
-  return pre + v;
-}
-
 template <int MODE, int ITEMS>
 __global__ __launch_bounds__(SMALL_BLOCK) void k_resample_small(SmallChainArgs a) {
-  constexpr int N = SMALL_BLOCK * ITEMS;
-  __shared__ u128 l128[SMALL_BLOCK / WAVE];
-  __shared__ uint64_t l64[SMALL_BLOCK / WAVE];
-  __shared__ uint16_t E[N];
-  __shared__ double Ws[MODE == BIHIP_MULTINOMIAL ? N : 1];
-  __shared__ int count[MODE == BIHIP_MULTINOMIAL ? N : 1];
-  static_assert(N <= 1 << 16, "E holds 16-bit sums of extra copies");
+  __shared__ SmallChainLds<ITEMS, MODE == BIHIP_MULTINOMIAL> lds;
   {
     const long f = bank_f();
     a.lws = bank_shift(a.lws, f * a.bk.p * 8);
@@ -688,105 +630,21 @@ __global__ __launch_bounds__(SMALL_BLOCK) void k_resample_small(SmallChainArgs a
   if (!gate_open(a.gate)) return;
   const uint32_t step = (uint32_t)a.gate->k;
 
-  // inclusive fixed-point weight sums
-  u128 v[ITEMS];
-#pragma unroll
-  for (int i = 0; i < ITEMS; ++i)
-    v[i] = base + i < a.P ? fix_weight(nanexp(lw[i] - m)) : u128(0);
-#pragma unroll
-  for (int i = 1; i < ITEMS; ++i) v[i] = v[i - 1] + v[i];
-  u128 tot;
-  const u128 start = small_inclusive_scan(v[ITEMS - 1], l128, tot) - v[ITEMS - 1];
-  const double W = fix_to_double(tot);
-  if (!(W > 0.0)) {
+  int src[ITEMS];
+  if (!small_chain<MODE>(lw, m, a.P, a.n, a.seed, step, a.batch, lds, src)) {
     if (a.status != nullptr && threadIdx.x == 0) a.status->status = BIHIP_DEGENERATE;
     return;
   }
-
-  // offspring counts
-  int o[ITEMS];
-  if constexpr (MODE == BIHIP_MULTINOMIAL) {
-#pragma unroll
-    for (int i = 0; i < ITEMS; ++i) {
-      Ws[base + i] = fix_to_double(start + v[i]);
-      count[base + i] = 0;
-    }
-    __syncthreads();
-    for (int j = threadIdx.x; j < a.n; j += SMALL_BLOCK) {
-      const u32x4 r = philox_block(a.seed, (uint32_t)j, step, TAG_MULTINOMIAL, a.batch, 0);
-      const double u = W * u53(r.x, r.y);
-      int lo = 0, hi = a.P;  // first i with Ws_i > u
-      while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (Ws[mid] <= u) lo = mid + 1;
-        else hi = mid;
-      }
-      atomicAdd(&count[lo < a.P ? lo : a.P - 1], 1);
-    }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < ITEMS; ++i) o[i] = base + i < a.P ? count[base + i] : 1;
-  } else {
-    double av = 0.0;
-    if (MODE == BIHIP_SYSTEMATIC) {
-      const u32x4 r = philox_block(a.seed, 0, step, TAG_SYSTEMATIC, a.batch, 0);
-      av = u53(r.x, r.y);
-    }
-    auto cumulative = [&](const u128& incl) -> int {
-      const double Wsi = fix_to_double(incl);
-      if (MODE == BIHIP_SYSTEMATIC) return systematic_offspring(Wsi, W, a.n, av);
-      const double reach = stratified_reach(Wsi, W, a.n);
-      int k = (int)reach;
-      if (k > a.n - 1) k = a.n - 1;
-      const u32x4 r = philox_block(a.seed, (uint32_t)k, step, TAG_STRATIFIED, a.batch, 0);
-      return stratified_offspring(reach, u53(r.x, r.y), a.n);
-    };
-    int prev = base > 0 && base < a.P ? cumulative(start) : 0;
-#pragma unroll
-    for (int i = 0; i < ITEMS; ++i) {
-      o[i] = 1;  // past the end: no extras, not free
-      if (base + i < a.P) {
-        const int O = cumulative(start + v[i]);
-        o[i] = O - prev;
-        prev = O;
-      }
-    }
-  }
-
-  // exclusive sums of extra copies (E) and free slots
-  uint64_t t = 0;
-#pragma unroll
-  for (int i = 0; i < ITEMS; ++i) t += ef_pair(o[i]);
-  uint64_t eftot;
-  uint64_t run = small_inclusive_scan(t, l64, eftot) - t;
-  int rank[ITEMS];  // of a free slot; -1: occupied
-#pragma unroll
-  for (int i = 0; i < ITEMS; ++i) {
-    E[base + i] = (uint16_t)run;
-    rank[i] = o[i] == 0 ? (int)(run >> 32) : -1;
-    run += ef_pair(o[i]);
-  }
-  __syncthreads();
-
-  // the free slot of rank r receives the last i with E_i <= r
-  int pos[ITEMS];
-#pragma unroll
-  for (int i = 0; i < ITEMS; ++i) pos[i] = 0;  // E_0 = 0
-  for (int s = 1 << (31 - __clz(a.P)); s > 0; s >>= 1) {
-#pragma unroll
-    for (int i = 0; i < ITEMS; ++i) {
-      const int c = pos[i] + s;
-      if (c < a.P && (int)E[c] <= rank[i]) pos[i] = c;
-    }
-  }
 #pragma unroll
   for (int i = 0; i < ITEMS; ++i)
-    if (base + i < a.P) a.as[base + i] = rank[i] < 0 ? base + i : pos[i];
+    if (base + i < a.P) a.as[base + i] = src[i];
 }
 
 template <int MODE>
 static void launch_small(const SmallChainArgs& a, int banks, hipStream_t s) {
-  const dim3 grid(1, banks), block(SMALL_BLOCK);
+  // as many waves as the particles fill
+  const int items = a.P <= SMALL_BLOCK ? 1 : (a.P <= 2 * SMALL_BLOCK ? 2 : 4);
+  const dim3 grid(1, banks), block(ceil_div(ceil_div(a.P, items), WAVE) * WAVE);
   if (a.P <= SMALL_BLOCK) hipLaunchKernelGGL((k_resample_small<MODE, 1>), grid, block, 0, s, a);
   else if (a.P <= 2 * SMALL_BLOCK)
     hipLaunchKernelGGL((k_resample_small<MODE, 2>), grid, block, 0, s, a);

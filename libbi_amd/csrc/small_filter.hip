@@ -1,0 +1,257 @@
+// Whole steps of one small filter in one workgroup: BootstrapPF::step
+// (share/src/bi/filter/BootstrapPF.hpp:156-167) for n observation intervals in
+// one launch.
+//
+// A filter of at most 1024 particles leaves the chip idle whatever its kernels
+// do: its step is the latency of its dependent launches.  Here one workgroup,
+// one particle a thread, runs the resampling chain (small_chain.hpp), the
+// gathered transition, the observation density, the weight partials and the
+// bookkeeping of a step, and goes on to the next; the log-weights, the log-
+// likelihood and the resampling decision stay in registers between steps.  Every
+// sum keeps the order of the separate kernels (partials of 256 particles, then
+// the combination's butterfly), so results equal theirs bit for bit.
+//
+// Bound by the latency of a step's arithmetic on one CU, and above 512 particles
+// by its FP64 rate.  Predator-prey filter in FP64, resampling every step: 6.8 us
+// a step at 256 particles, 9.3 at 512, 14.9 at 1000, against 29 to 30 us in five
+// launches (21.7 to 21.9 in three).  Two particles a thread would be slower than
+// the separate launches, so the line lies at 1024.
+#include "blockreduce.hpp"
+#include "gen_model.hpp"
+#include "internal.hpp"
+#include "model_ops.hpp"
+#include "small_chain.hpp"
+
+namespace bihip {
+
+struct SmallFilterArgs {
+  ModelArgs m;
+  void* X[2];  // X[0]: the current state
+  int ld, P, steps, resampler, nobs;
+  int* as;
+  double* lws;
+  PFDevice* dev;
+  PFHistory hist;
+  const double* y;
+  double t0, dt, essRel;
+  uint64_t seed;
+  uint32_t batch;
+};
+
+// Models it is compiled for: one lane per particle, few states (the workgroup
+// leaves 128 registers a thread).
+template <class M>
+constexpr bool small_filter_model() {
+  return M::LPP == 1 && M::D <= 4;
+}
+
+template <class M, int INTEG>
+__global__ __launch_bounds__(SMALL_BLOCK) void k_filter_small(SmallFilterArgs a) {
+  using T = typename M::real_t;
+  constexpr int DL = M::DL, NB = SMALL_BLOCK / TRANS_BLOCK, WPB = TRANS_BLOCK / WAVE;
+  static_assert(NB == 4 && WPB == 4, "a quad of lanes combines the partials");
+  __shared__ SmallChainLds<1, true> chain;
+  __shared__ double wm[SMALL_BLOCK / WAVE], w1[SMALL_BLOCK / WAVE], w2[SMALL_BLOCK / WAVE];
+  const int p = threadIdx.x, lane = p & (WAVE - 1), w = p / WAVE;
+  const bool active = p < a.P;
+  const int nb = (a.P + TRANS_BLOCK - 1) / TRANS_BLOCK;
+  const Group<1> grp;
+
+  int k = a.dev->k, status = a.dev->status;
+  bool resample = a.dev->resample != 0;
+  double ll = a.dev->logLikelihood, mx = a.dev->mx, ess = a.dev->ess, lW = a.dev->lW;
+  double lw = active ? a.lws[p] : 0.0;
+  const double logP = log((double)a.P);
+
+  for (int s = 0; s < a.steps; ++s) {
+    // ---- resample
+    int src = p;
+    bool gather = resample && status == BIHIP_OK;
+    if (gather) {
+      const double l[1] = {lw};
+      int anc[1];
+      bool ok;
+      if (a.resampler == BIHIP_SYSTEMATIC)
+        ok = small_chain<BIHIP_SYSTEMATIC>(l, mx, a.P, a.P, a.seed, (uint32_t)k, a.batch, chain,
+                                           anc);
+      else if (a.resampler == BIHIP_STRATIFIED)
+        ok = small_chain<BIHIP_STRATIFIED>(l, mx, a.P, a.P, a.seed, (uint32_t)k, a.batch, chain,
+                                           anc);
+      else
+        ok = small_chain<BIHIP_MULTINOMIAL>(l, mx, a.P, a.P, a.seed, (uint32_t)k, a.batch, chain,
+                                            anc);
+      if (ok) {
+        src = anc[0];
+        if (active) a.as[p] = src;
+      } else {
+        status = BIHIP_DEGENERATE;
+        gather = false;
+      }
+    }
+
+    // ---- predict + correct
+    const double t1 = a.t0 + k * a.dt, t2 = a.t0 + (k + 1) * a.dt;
+    const uint32_t step = (uint32_t)(k + 1);
+    double nlw = __builtin_nan("");
+    if (active) {
+      const T* Xin = static_cast<const T*>(a.X[s & 1]);
+      T* Xout = static_cast<T*>(a.X[1 - (s & 1)]);
+      T x[DL];
+#pragma unroll
+      for (int i = 0; i < DL; ++i) x[i] = Xin[(size_t)i * a.ld + src];
+      M m(a.m);
+      if constexpr (is_generated<M>::value) {
+        m.template transition<INTEG, true>(grp, x, t1, t2, a.m, a.seed, a.batch, (uint32_t)p,
+                                           step);
+      } else {
+        if constexpr (M::NOISE_FIRST) noise_first(m, a.seed, a.batch, p, step);
+        if constexpr (INTEG == BIHIP_RK4) integrate_rk4(m, grp, x, t1, t2, a.m.h0);
+        else integrate_dopri5(m, grp, x, t1, t2, a.m);
+        if constexpr (!M::NOISE_FIRST) noise_after(m, a.seed, a.batch, p, 0, step, x);
+      }
+#pragma unroll
+      for (int i = 0; i < DL; ++i) Xout[(size_t)i * a.ld + p] = x[i];
+      const double part = obs_of(m, x, a.y + (size_t)k * a.nobs, 0, &a.m);
+      nlw = (gather ? ll : lw) + part;
+    }
+
+    // ---- partials of TRANS_BLOCK particles, as block_weight_partial forms them
+    const double vm = wave_max(nlw);
+    if (lane == 0) wm[w] = vm;
+    __syncthreads();  // also: the new states are visible to the next step's gather
+    auto max4 = [&](int q) {
+      double r = wm[WPB * q];
+#pragma unroll
+      for (int i = 1; i < WPB; ++i) r = nan_max(r, wm[WPB * q + i]);
+      return r;
+    };
+    const double z = nanexp(nlw - max4(w / WPB));
+    const double v1 = wave_sum(z), v2 = wave_sum(z * z);
+    if (lane == 0) {
+      w1[w] = v1;
+      w2[w] = v2;
+    }
+    __syncthreads();
+    // ---- their combination (reduce.hip): lane quad q holds partial q, the
+    // butterfly's first two exchanges add the four
+    const int q = lane & (NB - 1);
+    const double mq = q < nb ? max4(q) : __builtin_nan("");
+    double M4 = xor_step<1>(mq, [](double x, double y) { return nan_max(x, y); });
+    M4 = xor_step<2>(M4, [](double x, double y) { return nan_max(x, y); });
+    double c1 = 0.0, c2 = 0.0;
+    if (q < nb) {
+      double b = w1[WPB * q], c = w2[WPB * q];
+#pragma unroll
+      for (int i = 1; i < WPB; ++i) {
+        b += w1[WPB * q + i];
+        c += w2[WPB * q + i];
+      }
+      if (b != 0.0) {
+        const double f = exp(mq - M4);
+        c1 = b * f;
+        c2 = c * (f * f);
+      }
+    }
+    c1 += dpp<QP_XOR1>(c1);
+    c1 += dpp<QP_XOR2>(c1);
+    c2 += dpp<QP_XOR1>(c2);
+    c2 += dpp<QP_XOR2>(c2);
+
+    // ---- BootstrapPF::correct's bookkeeping (pf_bookkeeping)
+    ess = c1 * c1 / c2;
+    lW = M4 + log(c1) - logP;
+    if (p == 0) {
+      a.hist.resampled[k] = gather ? 1 : 0;
+      a.hist.logIncrements[k] = lW - ll;
+      a.hist.ess[k] = ess;
+    }
+    ll = lW;
+    mx = M4;
+    resample = ess < a.essRel * (double)a.P;
+    lw = nlw;
+    ++k;
+  }
+  if (active) a.lws[p] = lw;
+  if (p == 0) {
+    a.dev->k = k;
+    a.dev->status = status;
+    a.dev->resample = resample ? 1 : 0;
+    a.dev->logLikelihood = ll;
+    a.dev->mx = mx;
+    a.dev->ess = ess;
+    a.dev->lW = lW;
+  }
+}
+
+namespace {
+struct SmallFilterRunner {
+  SmallFilterArgs a;
+  int integ;
+  hipStream_t s;
+  bool only_ask;
+  template <class M>
+  int run() {
+    if constexpr (small_filter_model<M>()) {
+      if (only_ask) return BIHIP_OK;
+      const dim3 block(ceil_div(a.P, TRANS_BLOCK) * TRANS_BLOCK);
+      if (integ == BIHIP_RK4)
+        hipLaunchKernelGGL((k_filter_small<M, BIHIP_RK4>), dim3(1), block, 0, s, a);
+      else
+        hipLaunchKernelGGL((k_filter_small<M, BIHIP_DOPRI5>), dim3(1), block, 0, s, a);
+      BIHIP_LAUNCH_CHECK();
+      return BIHIP_OK;
+    } else {
+      return only_ask ? BIHIP_EINVAL
+                      : set_error(BIHIP_EINVAL, "not a model of the one-workgroup filter");
+    }
+  }
+};
+
+int with_small_model(const bihip_model* m, SmallFilterRunner& r) {
+  const bool f64 = m->precision == BIHIP_F64;
+  if (m->model >= BIHIP_MODEL_GENERATED) return with_generated(m, r);
+  if (m->model == BIHIP_MODEL_PZ) return f64 ? r.run<PZ<double>>() : r.run<PZ<float>>();
+  if (m->model == BIHIP_MODEL_LG) return f64 ? r.run<LG<double>>() : r.run<LG<float>>();
+  return r.only_ask ? BIHIP_EINVAL
+                    : set_error(BIHIP_EINVAL, "not a model of the one-workgroup filter");
+}
+}  // namespace
+
+bool small_filter_fits(const bihip_model* m, int P, bool one_delta) {
+  if (P > SMALL_BLOCK) return false;
+  if (m->model >= BIHIP_MODEL_GENERATED && !one_delta) return false;
+  SmallFilterRunner r{};
+  r.only_ask = true;
+  return with_small_model(m, r) == BIHIP_OK;
+}
+
+int launch_small_filter(const SmallFilterLaunch& L, hipStream_t s) {
+  if (L.P <= 0 || L.P > SMALL_BLOCK || L.steps < 0)
+    return set_error(BIHIP_EINVAL, "the one-workgroup filter takes up to %d particles",
+                     SMALL_BLOCK);
+  if (L.steps == 0) return BIHIP_OK;
+  SmallFilterRunner r{};
+  r.a.m = to_args(L.model);
+  r.a.X[0] = L.X;
+  r.a.X[1] = L.Xother;
+  r.a.ld = L.ld;
+  r.a.P = L.P;
+  r.a.steps = L.steps;
+  r.a.resampler = L.resampler;
+  r.a.nobs = L.nobs;
+  r.a.as = L.as;
+  r.a.lws = L.lws;
+  r.a.dev = L.dev;
+  r.a.hist = L.hist;
+  r.a.y = L.y;
+  r.a.t0 = L.t0;
+  r.a.dt = L.dt;
+  r.a.essRel = L.essRel;
+  r.a.seed = L.seed;
+  r.a.batch = L.batch;
+  r.integ = L.model->integrator;
+  r.s = s;
+  return with_small_model(L.model, r);
+}
+
+}  // namespace bihip

@@ -66,6 +66,57 @@ def test_pz_filter_small_population_parity(ctx, orc, P, resampler):
         np.testing.assert_array_equal(anc, ref["ancestors"])
 
 
+SMALL_MODELS = {
+    "pz": lambda prec: (capi.make_model("pz", precision=prec), 2.0),
+    "pz-dopri5": lambda prec: (capi.make_model("pz", precision=prec, integrator=capi.DOPRI5), 2.0),
+    "lg": lambda prec: (capi.make_model("lg", precision=prec), 0.3),
+    "PZ.bi": lambda prec: (capi.generated_model("PZ", precision=prec, mu=0.5, sigma=0.2), 2.0),
+    "AR1.bi": lambda prec: (capi.generated_model("AR1", precision=prec), 0.3),
+    "SIRStochastic.bi": lambda prec: (capi.generated_model("SIRStochastic", precision=prec), 9.0),
+}
+
+
+@pytest.mark.parametrize("prec", [capi.F64, capi.F32])
+@pytest.mark.parametrize("kind", sorted(SMALL_MODELS))
+@pytest.mark.parametrize("P,resampler,ess_rel", [
+    (1, capi.SYSTEMATIC, 1.0), (64, capi.MULTINOMIAL, 1.0), (255, capi.STRATIFIED, 0.5),
+    (257, capi.SYSTEMATIC, 0.7), (600, capi.MULTINOMIAL, 0.5), (1024, capi.STRATIFIED, 1.0)])
+def test_small_filter_equals_the_separate_launches(ctx, kind, prec, P, resampler, ess_rel):
+    """A filter of at most 1024 particles runs its steps in one workgroup; a recorded
+    one keeps the separate launches.  Outputs, states, log-weights and last ancestors are
+    the same bits, whatever way the steps are divided over calls (200 in all, so that one
+    call takes several launches), also after the observations degenerate the weights."""
+    m, y0 = SMALL_MODELS[kind](prec)
+    for i in range(16):  # parameters left at zero: small positive values
+        if m.par[i] == 0.0:
+            m.par[i] = 0.3
+    T = 200
+    y = y0 * (1.0 + 0.1 * np.sin(np.arange(T)))
+    if kind == "SIRStochastic.bi":
+        y = np.round(y)
+    y = y.reshape(T, 1)
+    if P == 255:
+        y[150:] = np.nan
+    got = []
+    for record, parts in ((True, (T,)), (False, (1, 2, 197)), (False, (T,))):
+        pf = capi.ParticleFilter(ctx, m, P, T, 1.0, 7, resampler, ess_rel, record=record,
+                                 use_graph=not record and len(parts) == 1)
+        pf.set_observations(y)
+        pf.init()
+        for n in parts:
+            pf.step(n)
+        out = pf.outputs()
+        X, _, lws = pf.state()
+        out["X"], out["lws"], out["as"] = X[:, :P].cpu().numpy(), lws.cpu().numpy(), pf.ancestors()
+        got.append(out)
+        pf.close()
+    for out in got[1:]:
+        for key, v in got[0].items():
+            if key == "as" and not got[0]["resampled"].any():
+                continue  # never written
+            np.testing.assert_array_equal(out[key], v, err_msg=key)
+
+
 @pytest.mark.parametrize("resampler", [capi.SYSTEMATIC, capi.STRATIFIED, capi.MULTINOMIAL])
 def test_pz_filter_large_population_parity(ctx, orc, resampler):
     """N = 2^21 + 5: more than 1024 tiles of 2048 particles, so the resampling
