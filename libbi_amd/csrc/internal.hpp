@@ -442,17 +442,44 @@ int launch_mse_grad(const float* Y, int ldy, const float* T, long ldt, const lon
 int launch_gauss_grad(const float* Y, int ldy, const float* T, long ldt, const long* idx, int n,
                       int rows, int m, float scale, uint16_t* dY, float* partial, int* nblocks,
                       hipStream_t s);
-int launch_colsum_bf16(const uint16_t* dZ, int ld, int rows, int cols, float* part, float* out,
-                       hipStream_t s);
-int launch_sum_splits(const float* part, int S, long count, float* out, hipStream_t s);
-int launch_sum_all(const float* x, int n, float* out, hipStream_t s);
-int launch_adam(float* w, float* m1, float* m2, const float* grad, long n, float lr, float b1,
-                float b2, float eps, float bc1, float bc2, uint16_t* wbf, hipStream_t s);
 int launch_to_bf16(const float* x, long n, uint16_t* y, hipStream_t s);
+
+constexpr int MLP_MAX_LAYERS = 6;
+// Partial weight gradients dZ^T act and bias gradients of several layers over
+// splits of ksplit rows.
+struct WeightGradLayer {
+  const uint16_t *dZ, *act;  // rows x M (ldz), rows x N (lda), bf16
+  long ldz, lda;
+  int M, N;                  // multiples of 64
+  int block0;                // blocks of the layers before
+  float *partW, *partb;      // splits x M x N, splits x M
+};
+struct WeightGradArgs {
+  int n, rows, ksplit;
+  WeightGradLayer layer[MLP_MAX_LAYERS];
+};
+int launch_weight_grads(const WeightGradArgs& g, hipStream_t s);
+// Sums of the splits of parameter segments: into G, or as an Adam step.
+struct UpdateSegment {
+  const float* part;  // S x count
+  long count, off;    // multiples of 4; offset in the parameter arenas
+  int block0;         // blocks (of 1024 parameters) of the segments before
+};
+struct UpdateArgs {
+  int n, S, adam;
+  UpdateSegment seg[2 * MLP_MAX_LAYERS];
+  float *P, *G, *M1, *M2;
+  uint16_t* Wbf;      // bf16 copy of the first nW parameters
+  long nW;
+  float lr, b1, b2, eps, bc1, bc2;
+  const float* loss;  // loss_out (nullable) gets the sum of nloss terms
+  int nloss;
+  float* loss_out;
+};
+int launch_update(const UpdateArgs& a, hipStream_t s);
 
 // Device parameters of an MLP (bf16 weights [pad_{l+1}][pad_l], FP32 biases),
 // for the fused inference kernels.
-constexpr int MLP_MAX_LAYERS = 6;
 struct MlpView {
   int L;
   int dims[MLP_MAX_LAYERS + 1], pad[MLP_MAX_LAYERS + 1];

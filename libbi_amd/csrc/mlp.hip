@@ -13,45 +13,63 @@ namespace bihip {
 
 namespace {
 
-constexpr int GB_M = 64, GB_N = 64, GB_K = 32, LDS_K = GB_K + 8;  // +8: bank spread
+// K steps of 64: the tiles of one step are 2 loads a thread and operand, and a
+// 256-wide layer takes four round trips to memory instead of eight (forward
+// GEMM of 4096 x 256 x 256 8.4 -> 6.8 us).
+constexpr int GB_M = 64, GB_N = 64, GB_K = 64, LDS_K = GB_K + 8;  // +8: bank spread
 
 // C = op(A) op(B) over k in [z ksplit, (z + 1) ksplit), 64 x 64 tiles, four
 // waves of 32 x 32.  Tiles are staged k-contiguous in LDS whatever the global
 // orientation, so every fragment read is one 16-byte LDS load.
-template <bool TA, bool TB, int EPI>
-__global__ __launch_bounds__(256) void k_gemm(GemmArgs g) {
-  __shared__ __attribute__((aligned(16))) uint16_t As[GB_M * LDS_K];
-  __shared__ __attribute__((aligned(16))) uint16_t Bs[GB_N * LDS_K];
+// One 64 x 64 operand tile of K step k0 into LDS, k-contiguous: rows of X from
+// r0 (TRANS false: X[(r0 + r) ld + k0 + k], true: X[(k0 + k) ld + r0 + r]).
+template <bool TRANS>
+struct TileLoad {
+  u16x8 v[2];
+  __device__ __forceinline__ void load(const uint16_t* X, long ld, int r0, int k0, int tid) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int a = (tid >> 3) + 32 * u, b = (tid & 7) * 8;
+      v[u] = TRANS ? *reinterpret_cast<const u16x8*>(X + (size_t)(k0 + a) * ld + r0 + b)
+                   : *reinterpret_cast<const u16x8*>(X + (size_t)(r0 + a) * ld + k0 + b);
+    }
+  }
+  __device__ __forceinline__ void store(uint16_t* S, int tid) const {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int a = (tid >> 3) + 32 * u, b = (tid & 7) * 8;
+      if (TRANS) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) S[(b + j) * LDS_K + a] = v[u][j];
+      } else {
+        *reinterpret_cast<u16x8*>(&S[a * LDS_K + b]) = v[u];
+      }
+    }
+  }
+};
+
+// acc += A B over K steps [kbeg, kend) of a 64 x 64 tile, four waves of 32 x 32;
+// the next step's tiles are loaded while this one is computed.  each(As): called
+// with every staged A tile.
+template <bool TA, bool TB, class Each>
+__device__ __forceinline__ void gemm_tile(const uint16_t* A, long lda, const uint16_t* B, long ldb,
+                                          int m0, int n0, int kbeg, int kend, uint16_t* As,
+                                          uint16_t* Bs, f32x16& acc, Each each) {
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int wm = w >> 1, wn = w & 1;
-  const int m0 = blockIdx.x * GB_M, n0 = blockIdx.y * GB_N;
-  const int kbeg = blockIdx.z * g.ksplit;
-  const int kend = kbeg + g.ksplit < g.K ? kbeg + g.ksplit : g.K;
-  f32x16 acc;
-#pragma unroll
-  for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+  TileLoad<TA> ta;
+  TileLoad<!TB> tb;
+  ta.load(A, lda, m0, kbeg, tid);
+  tb.load(B, ldb, n0, kbeg, tid);
   for (int k0 = kbeg; k0 < kend; k0 += GB_K) {
-    if (!TA) {
-      const int m = tid >> 2, k8 = (tid & 3) * 8;
-      *reinterpret_cast<u16x8*>(&As[m * LDS_K + k8]) =
-          *reinterpret_cast<const u16x8*>(g.A + (size_t)(m0 + m) * g.lda + k0 + k8);
-    } else {
-      const int k = tid >> 3, m8 = (tid & 7) * 8;
-      const u16x8 v = *reinterpret_cast<const u16x8*>(g.A + (size_t)(k0 + k) * g.lda + m0 + m8);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) As[(m8 + j) * LDS_K + k] = v[j];
-    }
-    if (TB) {
-      const int n = tid >> 2, k8 = (tid & 3) * 8;
-      *reinterpret_cast<u16x8*>(&Bs[n * LDS_K + k8]) =
-          *reinterpret_cast<const u16x8*>(g.B + (size_t)(n0 + n) * g.ldb + k0 + k8);
-    } else {
-      const int k = tid >> 3, n8 = (tid & 7) * 8;
-      const u16x8 v = *reinterpret_cast<const u16x8*>(g.B + (size_t)(k0 + k) * g.ldb + n0 + n8);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) Bs[(n8 + j) * LDS_K + k] = v[j];
-    }
+    ta.store(As, tid);
+    tb.store(Bs, tid);
     __syncthreads();
+    if (k0 + GB_K < kend) {
+      ta.load(A, lda, m0, k0 + GB_K, tid);
+      tb.load(B, ldb, n0, k0 + GB_K, tid);
+    }
+    each(As);
 #pragma unroll
     for (int kk = 0; kk < GB_K; kk += 16) {
       const u16x8 a = *reinterpret_cast<const u16x8*>(
@@ -62,6 +80,22 @@ __global__ __launch_bounds__(256) void k_gemm(GemmArgs g) {
     }
     __syncthreads();
   }
+}
+
+template <bool TA, bool TB, int EPI>
+__global__ __launch_bounds__(256) void k_gemm(GemmArgs g) {
+  __shared__ __attribute__((aligned(16))) uint16_t As[GB_M * LDS_K];
+  __shared__ __attribute__((aligned(16))) uint16_t Bs[GB_N * LDS_K];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int wm = w >> 1, wn = w & 1;
+  const int m0 = blockIdx.x * GB_M, n0 = blockIdx.y * GB_N;
+  const int kbeg = blockIdx.z * g.ksplit;
+  const int kend = kbeg + g.ksplit < g.K ? kbeg + g.ksplit : g.K;
+  f32x16 acc;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+  gemm_tile<TA, TB>(g.A, g.lda, g.B, g.ldb, m0, n0, kbeg, kend, As, Bs, acc,
+                    [](const uint16_t*) {});
   const int col = n0 + wn * 32 + (lane & 31);
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
@@ -159,120 +193,140 @@ __global__ __launch_bounds__(256) void k_gauss_grad(const float* Y, int ldy, con
   if (threadIdx.x == 0) partial[blockIdx.x] = red[0];
 }
 
-// part[s][c] = sum of bf16 dZ[r][c] over rows r in [256 s, 256 s + 256), in a
-// fixed order.  A workgroup takes 64 columns of one split: each thread reads
-// eight columns of eight rows (rows rs, rs + 32, ..., rs + 224 of the split,
-// rs = thread / 8) as 16-byte loads issued together, sums its rows in order,
-// and the 32 row slots are then added in order through LDS.  Needs cols and
-// ld to be multiples of 8 (the padded layer widths are multiples of 64).
-__global__ __launch_bounds__(256) void k_colsum_bf16(const uint16_t* dZ, int ld, int rows,
-                                                     int cols, float* part) {
+// Weight and bias gradients of several layers in one launch, split over the
+// batch: block b takes a 64 x 64 tile of dZ^T A of one layer over one split of
+// the rows and stores its partial sums; the blocks of a layer's first tile
+// column also sum the columns of dZ (the bias gradient) from the tiles they
+// stage, thread (m, eight row slots) adding rows slot, slot + 32, ... in order
+// and then the 32 slots in order.  A layer alone is at most 256 blocks of four
+// K steps: 9.3 us each, and 4.2 + 3.4 us for its column sums in launches of
+// their own; together 17.5 us for four layers.
+__global__ __launch_bounds__(256) void k_weight_grads(WeightGradArgs g) {
+  __shared__ __attribute__((aligned(16))) uint16_t As[GB_M * LDS_K];
+  __shared__ __attribute__((aligned(16))) uint16_t Bs[GB_N * LDS_K];
   __shared__ float red[32][64 + 1];
-  const int cg = threadIdx.x & 7, rs = threadIdx.x >> 3;
-  const int c0 = blockIdx.x * 64 + cg * 8;
-  const int r0 = blockIdx.y * 256;
-  float acc[8];
+  int l = 0;
+  while (l + 1 < g.n && (int)blockIdx.x >= g.layer[l + 1].block0) ++l;
+  const WeightGradLayer& y = g.layer[l];
+  const int nt = y.N / GB_N, mt = y.M / GB_M;
+  int b = (int)blockIdx.x - y.block0;
+  const int n0 = b % nt * GB_N;
+  b /= nt;
+  const int m0 = b % mt * GB_M, z = b / mt;
+  const int kbeg = z * g.ksplit, kend = min(kbeg + g.ksplit, g.rows);
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  f32x16 acc;
 #pragma unroll
-  for (int j = 0; j < 8; ++j) acc[j] = 0.0f;
-  if (c0 < cols) {
-    uint4 v[8];
+  for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+  float col[8];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int r = r0 + rs + 32 * u;
-      v[u] = r < rows ? *reinterpret_cast<const uint4*>(dZ + (size_t)r * ld + c0)
-                      : make_uint4(0u, 0u, 0u, 0u);
-    }
+  for (int j = 0; j < 8; ++j) col[j] = 0.0f;
+  const bool sums = n0 == 0;
+  const int m = tid & 63, slot = (tid >> 6) * 8;
+  gemm_tile<true, false>(y.dZ, y.ldz, y.act, y.lda, m0, n0, kbeg, kend, As, Bs, acc,
+                         [&](const uint16_t* S) {
+                           if (!sums) return;
+                           const u16x8 a =
+                               *reinterpret_cast<const u16x8*>(&S[m * LDS_K + slot]);
+                           const u16x8 c =
+                               *reinterpret_cast<const u16x8*>(&S[m * LDS_K + slot + 32]);
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const uint32_t w[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
+                           for (int j = 0; j < 8; ++j) col[j] += bf2f(a[j]);
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        acc[2 * q] += bf2f((uint16_t)(w[q] & 0xFFFFu));
-        acc[2 * q + 1] += bf2f((uint16_t)(w[q] >> 16));
-      }
-    }
-  }
+                           for (int j = 0; j < 8; ++j) col[j] += bf2f(c[j]);
+                         });
+  float* part = y.partW + (size_t)z * y.M * y.N;
+  const int c0 = n0 + (w & 1) * 32 + (lane & 31);
 #pragma unroll
-  for (int j = 0; j < 8; ++j) red[rs][cg * 8 + j] = acc[j];
+  for (int r = 0; r < 16; ++r)
+    part[(size_t)(m0 + (w >> 1) * 32 + acc_row(r, lane)) * y.N + c0] = acc[r];
+  if (!sums) return;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) red[slot + j][m] = col[j];
   __syncthreads();
-  if (threadIdx.x < 64) {
-    const int c = blockIdx.x * 64 + threadIdx.x;
+  if (tid < 64) {
     float t = 0.0f;
-    for (int q = 0; q < 32; ++q) t += red[q][threadIdx.x];
-    if (c < cols) part[(size_t)blockIdx.y * cols + c] = t;
+    for (int q = 0; q < 32; ++q) t += red[q][tid];
+    y.partb[(size_t)z * y.M + m0 + tid] = t;
   }
 }
 
-// out[i] = sum_s part[s][i], added in the order s = 0, 1, ..., S-1.  Each
-// thread takes four consecutive outputs (one 16-byte load per split when
-// count is a multiple of 4) and issues the loads of eight splits before
-// adding them, so the split loads overlap instead of each waiting for the
-// previous add; the order of the additions is unchanged.
-__global__ void k_sum_splits(const float* part, int S, long count, float* out) {
-  const long i = ((long)blockIdx.x * blockDim.x + threadIdx.x) * 4;
-  if (i >= count) return;
-  if ((count & 3) == 0) {
-    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-    int z = 0;
-    for (; z + 8 <= S; z += 8) {
-      float4 v[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u)
-        v[u] = *reinterpret_cast<const float4*>(part + (size_t)(z + u) * count + i);
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        acc.x += v[u].x;
-        acc.y += v[u].y;
-        acc.z += v[u].z;
-        acc.w += v[u].w;
-      }
+// The splits of several parameter segments summed in the order s = 0, 1, ...,
+// S-1 (four parameters a thread, eight splits in flight), and what becomes of
+// the sums: the gradient (adam == 0), or an Adam step (Kingma & Ba 2015, with
+// bias correction) on the FP32 parameters with their bfloat16 copy.  One more
+// block (loss_out) sums the minibatch's loss terms.  One launch for all layers;
+// as a sum per weight and bias array, two Adam launches and one for the loss it
+// was eleven of 2.4 to 3.5 us.
+__global__ __launch_bounds__(256) void k_update(UpdateArgs a) {
+  if (a.loss_out != nullptr && blockIdx.x == gridDim.x - 1) {
+    __shared__ float red[256];
+    float s = 0.0f;
+    for (int i = threadIdx.x; i < a.nloss; i += 256) s += a.loss[i];
+    red[threadIdx.x] = s;
+    __syncthreads();
+    for (int o = 128; o > 0; o >>= 1) {
+      if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
+      __syncthreads();
     }
-    for (; z < S; ++z) {
-      const float4 v = *reinterpret_cast<const float4*>(part + (size_t)z * count + i);
-      acc.x += v.x;
-      acc.y += v.y;
-      acc.z += v.z;
-      acc.w += v.w;
-    }
-    *reinterpret_cast<float4*>(out + i) = acc;
+    if (threadIdx.x == 0) *a.loss_out = red[0];
     return;
   }
-  const int n = count - i < 4 ? (int)(count - i) : 4;
-  for (int q = 0; q < n; ++q) {
-    float s = 0.0f;
-    for (int z = 0; z < S; ++z) s += part[(size_t)z * count + i + q];
-    out[i + q] = s;
+  int q = 0;
+  while (q + 1 < a.n && (int)blockIdx.x >= a.seg[q + 1].block0) ++q;
+  const UpdateSegment& e = a.seg[q];
+  const long i = ((long)((int)blockIdx.x - e.block0) * 256 + threadIdx.x) * 4;
+  if (i >= e.count) return;
+  float4 g = make_float4(0.f, 0.f, 0.f, 0.f);
+  int z = 0;
+  for (; z + 8 <= a.S; z += 8) {
+    float4 v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      v[u] = *reinterpret_cast<const float4*>(e.part + (size_t)(z + u) * e.count + i);
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      g.x += v[u].x;
+      g.y += v[u].y;
+      g.z += v[u].z;
+      g.w += v[u].w;
+    }
   }
-}
-
-// out[0] = sum of x[0 .. n) by one workgroup: strided partial sums, then a
-// fixed-order tree in LDS
-__global__ __launch_bounds__(256) void k_sum_all(const float* x, int n, float* out) {
-  __shared__ float red[256];
-  float s = 0.0f;
-  for (int i = threadIdx.x; i < n; i += 256) s += x[i];
-  red[threadIdx.x] = s;
-  __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-    __syncthreads();
+  for (; z < a.S; ++z) {
+    const float4 v = *reinterpret_cast<const float4*>(e.part + (size_t)z * e.count + i);
+    g.x += v.x;
+    g.y += v.y;
+    g.z += v.z;
+    g.w += v.w;
   }
-  if (threadIdx.x == 0) out[0] = red[0];
-}
-
-// Adam (Kingma & Ba 2015) with bias correction; wbf (nullable) gets the bf16 copy.
-__global__ void k_adam(float* w, float* m1, float* m2, const float* grad, long n, float lr,
-                       float b1, float b2, float eps, float bc1, float bc2, uint16_t* wbf) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const float gr = grad[i];
-  const float a = b1 * m1[i] + (1.0f - b1) * gr;
-  const float b = b2 * m2[i] + (1.0f - b2) * gr * gr;
-  m1[i] = a;
-  m2[i] = b;
-  const float x = w[i] - lr * (a / bc1) / (sqrtf(b / bc2) + eps);
-  w[i] = x;
-  if (wbf != nullptr) wbf[i] = f2bf(x);
+  const long k = e.off + i;
+  if (a.adam == 0) {
+    *reinterpret_cast<float4*>(a.G + k) = g;
+    return;
+  }
+  float gr[4] = {g.x, g.y, g.z, g.w};
+  float4 m1 = *reinterpret_cast<float4*>(a.M1 + k), m2 = *reinterpret_cast<float4*>(a.M2 + k),
+         w = *reinterpret_cast<float4*>(a.P + k);
+  float* m1v = &m1.x;
+  float* m2v = &m2.x;
+  float* wv = &w.x;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const float x = a.b1 * m1v[u] + (1.0f - a.b1) * gr[u];
+    const float y = a.b2 * m2v[u] + (1.0f - a.b2) * gr[u] * gr[u];
+    m1v[u] = x;
+    m2v[u] = y;
+    wv[u] = wv[u] - a.lr * (x / a.bc1) / (sqrtf(y / a.bc2) + a.eps);
+  }
+  *reinterpret_cast<float4*>(a.M1 + k) = m1;
+  *reinterpret_cast<float4*>(a.M2 + k) = m2;
+  *reinterpret_cast<float4*>(a.P + k) = w;
+  if (k < a.nW) {
+    uint2 h;
+    h.x = pack_bf2(w.x, w.y);
+    h.y = pack_bf2(w.z, w.w);
+    *reinterpret_cast<uint2*>(a.Wbf + k) = h;
+  }
 }
 
 __global__ void k_to_bf16(const float* x, long n, uint16_t* y) {
@@ -393,38 +447,36 @@ int launch_gauss_grad(const float* Y, int ldy, const float* T, long ldt, const l
   return BIHIP_OK;
 }
 
-int launch_colsum_bf16(const uint16_t* dZ, int ld, int rows, int cols, float* part, float* out,
-                       hipStream_t s) {
-  if (cols % 8 || ld % 8 || ((uintptr_t)dZ & 15))
-    return set_error(BIHIP_EINVAL, "column sums need 8-aligned columns (cols %d, ld %d)", cols, ld);
-  const int S = ceil_div(rows, 256);
-  hipLaunchKernelGGL(k_colsum_bf16, dim3(ceil_div(cols, 64), S), dim3(256), 0, s, dZ, ld, rows,
-                     cols, part);
-  BIHIP_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_sum_splits, dim3(ceil_div(cols, 1024)), dim3(256), 0, s, part, S,
-                     (long)cols, out);
-  BIHIP_LAUNCH_CHECK();
-  return BIHIP_OK;
-}
-
-int launch_sum_splits(const float* part, int S, long count, float* out, hipStream_t s) {
-  hipLaunchKernelGGL(k_sum_splits, dim3(ceil_div(count, 1024)), dim3(256), 0, s, part, S, count,
-                     out);
+int launch_weight_grads(const WeightGradArgs& g, hipStream_t s) {
+  if (g.n <= 0) return BIHIP_OK;
+  if (g.rows <= 0 || g.rows % GB_K || g.ksplit <= 0 || g.ksplit % GB_K)
+    return set_error(BIHIP_EINVAL, "weight gradients of %d rows (split %d) off the 64-row steps",
+                     g.rows, g.ksplit);
+  const int S = ceil_div(g.rows, g.ksplit);
+  long blocks = 0;
+  for (int l = 0; l < g.n; ++l) {
+    const WeightGradLayer& y = g.layer[l];
+    if (y.M <= 0 || y.N <= 0 || y.M % GB_M || y.N % GB_N || y.ldz % 8 || y.lda % 8 ||
+        (((uintptr_t)y.dZ | (uintptr_t)y.act) & 15) || y.block0 != blocks)
+      return set_error(BIHIP_EINVAL, "weight gradient %dx%d off the 64x64 tiling", y.M, y.N);
+    blocks += (long)(y.M / GB_M) * (y.N / GB_N) * S;
+  }
+  hipLaunchKernelGGL(k_weight_grads, dim3(blocks), dim3(256), 0, s, g);
   BIHIP_LAUNCH_CHECK();
   return BIHIP_OK;
 }
 
-int launch_sum_all(const float* x, int n, float* out, hipStream_t s) {
-  hipLaunchKernelGGL(k_sum_all, dim3(1), dim3(256), 0, s, x, n, out);
-  BIHIP_LAUNCH_CHECK();
-  return BIHIP_OK;
-}
-
-int launch_adam(float* w, float* m1, float* m2, const float* grad, long n, float lr, float b1,
-                float b2, float eps, float bc1, float bc2, uint16_t* wbf, hipStream_t s) {
-  if (n <= 0) return BIHIP_OK;
-  hipLaunchKernelGGL(k_adam, dim3(ceil_div(n, 256)), dim3(256), 0, s, w, m1, m2, grad, n, lr, b1,
-                     b2, eps, bc1, bc2, wbf);
+int launch_update(const UpdateArgs& a, hipStream_t s) {
+  long blocks = 0;
+  for (int q = 0; q < a.n; ++q) {
+    const UpdateSegment& e = a.seg[q];
+    if (e.count % 4 || e.off % 4 || e.block0 != blocks || ((uintptr_t)e.part & 15))
+      return set_error(BIHIP_EINVAL, "parameter segments of padded widths are needed");
+    blocks += ceil_div(e.count / 4, 256);
+  }
+  if (a.loss_out != nullptr) ++blocks;
+  if (blocks == 0) return BIHIP_OK;
+  hipLaunchKernelGGL(k_update, dim3(blocks), dim3(256), 0, s, a);
   BIHIP_LAUNCH_CHECK();
   return BIHIP_OK;
 }

@@ -62,6 +62,9 @@ void free_work(bihip_mlp* m) {
 }
 
 constexpr int KSPLIT = 256;  // batch rows per split of the weight-gradient GEMMs
+// Floats of partial sums up to which all layers' gradients share one launch
+// (larger networks take a layer at a time).
+constexpr long PART_GROUP = 1L << 26;
 
 int ensure_work(bihip_mlp* m, int rows) {
   if (rows <= m->cap) return BIHIP_OK;
@@ -77,10 +80,11 @@ int ensure_work(bihip_mlp* m, int rows) {
     if ((rc = dalloc(&m->Z[l], (size_t)rows * m->pad[l + 1]))) return rc;
     if ((rc = dalloc(&m->dZ[l], (size_t)rows * m->pad[l + 1]))) return rc;
     if (l + 1 < L && (rc = dalloc(&m->A[l + 1], (size_t)rows * m->pad[l + 1]))) return rc;
-    maxw = std::max(maxw, (long)m->pad[l + 1] * m->pad[l]);
+    maxw = std::max(maxw, (long)m->pad[l + 1] * (m->pad[l] + 1));
   }
   const int S = (rows + KSPLIT - 1) / KSPLIT;
-  m->part_n = maxw * S;
+  // one layer's partial sums, or all of them where they stay small
+  m->part_n = std::max(maxw * S, std::min(m->ntot * S, PART_GROUP));
   if ((rc = dalloc(&m->part, (size_t)m->part_n))) return rc;
   if ((rc = dalloc(&m->lossp, (size_t)rows * m->pad[L] / 256 + 1))) return rc;
   m->cap = rows;
@@ -111,28 +115,13 @@ int forward(bihip_mlp* m, int rows, hipStream_t s) {
   return BIHIP_OK;
 }
 
-// backward from dZ[L-1] (already set) into the gradient arena G
-int backward(bihip_mlp* m, int rows, hipStream_t s) {
+// Backward from dZ[L-1] (already set): the errors of the layers, then their
+// gradients in as few launches as the partial sums' workspace allows (usually
+// one), each followed by the launch that sums them into the gradient arena G or
+// takes the Adam step `u` describes.
+int backward(bihip_mlp* m, int rows, const UpdateArgs& u, hipStream_t s) {
   int rc;
-  for (int l = m->L - 1; l >= 0; --l) {
-    GemmArgs g{};  // dW_l = dZ_l^T A_l, split over the batch
-    g.A = m->dZ[l];
-    g.lda = m->pad[l + 1];
-    g.B = l == 0 ? m->X0 : m->A[l];
-    g.ldb = m->pad[l];
-    g.M = m->pad[l + 1];
-    g.N = m->pad[l];
-    g.K = rows;
-    g.ksplit = std::min(rows, KSPLIT);
-    g.Cf = m->part;
-    g.ldc = m->pad[l];
-    if ((rc = launch_gemm(g, true, false, EPI_STORE, s))) return rc;
-    const int S = (rows + g.ksplit - 1) / g.ksplit;
-    if ((rc = launch_sum_splits(m->part, S, (long)g.M * g.N, m->G + m->offW[l], s))) return rc;
-    if ((rc = launch_colsum_bf16(m->dZ[l], m->pad[l + 1], rows, m->pad[l + 1], m->part,
-                                 m->G + m->offb[l], s)))
-      return rc;
-    if (l == 0) break;
+  for (int l = m->L - 1; l > 0; --l) {
     GemmArgs h{};  // dZ_{l-1} = (dZ_l W_l) * GELU'(Z_{l-1})
     h.A = m->dZ[l];
     h.lda = m->pad[l + 1];
@@ -147,6 +136,44 @@ int backward(bihip_mlp* m, int rows, hipStream_t s) {
     h.Cb = m->dZ[l - 1];
     h.ldcb = m->pad[l];
     if ((rc = launch_gemm(h, false, false, EPI_GELU_GRAD, s))) return rc;
+  }
+  const int ksplit = std::min(rows, KSPLIT), S = (rows + ksplit - 1) / ksplit;
+  for (int l = 0; l < m->L;) {
+    WeightGradArgs g{};  // dW_l = dZ_l^T A_l, split over the batch
+    g.rows = rows;
+    g.ksplit = ksplit;
+    UpdateArgs a = u;
+    a.S = S;
+    a.P = m->P;
+    a.G = m->G;
+    a.M1 = m->M1;
+    a.M2 = m->M2;
+    a.Wbf = m->Wbf;
+    a.nW = m->nW;
+    long used = 0, gblocks = 0, ublocks = 0;
+    for (; l < m->L; ++l) {
+      const int M = m->pad[l + 1], N = m->pad[l];
+      const long cw = (long)M * N, need = (cw + M) * S;
+      if (g.n > 0 && used + need > m->part_n) break;
+      WeightGradLayer& y = g.layer[g.n++];
+      y.dZ = m->dZ[l];
+      y.ldz = M;
+      y.act = l == 0 ? m->X0 : m->A[l];
+      y.lda = N;
+      y.M = M;
+      y.N = N;
+      y.block0 = (int)gblocks;
+      y.partW = m->part + used;
+      y.partb = y.partW + cw * S;
+      gblocks += cw / 4096 * S;
+      used += need;
+      a.seg[a.n++] = UpdateSegment{y.partW, cw, m->offW[l], (int)ublocks};
+      ublocks += (cw / 4 + 255) / 256;
+      a.seg[a.n++] = UpdateSegment{y.partb, M, m->offb[l], (int)ublocks};
+      ublocks += (M / 4 + 255) / 256;
+    }
+    if (l < m->L) a.loss_out = nullptr;  // the last launch sums the loss
+    if ((rc = launch_weight_grads(g, s)) || (rc = launch_update(a, s))) return rc;
   }
   return BIHIP_OK;
 }
@@ -407,7 +434,7 @@ int bihip_mlp_loss_grad(bihip_mlp* m, const float* X_dev, long ldx, const float*
   if ((rc = launch_rows_to_bf16(X_dev, ldx, nullptr, n, rows, m->dims[0], m->X0, m->pad[0], s)) ||
       (rc = forward(m, rows, s)) ||
       (rc = loss_and_error(m, T_dev, ldt, nullptr, n, rows, &sq, s)) ||
-      (rc = backward(m, rows, s)))
+      (rc = backward(m, rows, UpdateArgs{}, s)))
     return rc;
   if (loss_host) *loss_host = sq / ((double)n * targets_per_sample(m));
   if (grad_host) {
@@ -465,16 +492,21 @@ int bihip_mlp_train(bihip_mlp* m, const float* X_dev, long ldx, const float* T_d
     if ((rc = launch_rows_to_bf16(X_dev, ldx, idx, batch, batch, m->dims[0], m->X0, m->pad[0],
                                   s)) ||
         (rc = forward(m, batch, s)) ||
-        (rc = output_error(m, T_dev, ldt, idx, batch, batch, &nb, s)) ||
-        (rc = launch_sum_all(m->lossp, nb, loss_d + it, s)) || (rc = backward(m, batch, s)))
+        (rc = output_error(m, T_dev, ldt, idx, batch, batch, &nb, s)))
       break;
     ++m->adam_t;
-    const float bc1 = 1.0f - std::pow(b1, (float)m->adam_t);
-    const float bc2 = 1.0f - std::pow(b2, (float)m->adam_t);
-    if ((rc = launch_adam(m->P, m->M1, m->M2, m->G, m->nW, lr, b1, b2, eps, bc1, bc2, m->Wbf, s)) ||
-        (rc = launch_adam(m->P + m->nW, m->M1 + m->nW, m->M2 + m->nW, m->G + m->nW,
-                          m->ntot - m->nW, lr, b1, b2, eps, bc1, bc2, nullptr, s)))
-      break;
+    UpdateArgs u{};
+    u.adam = 1;
+    u.lr = lr;
+    u.b1 = b1;
+    u.b2 = b2;
+    u.eps = eps;
+    u.bc1 = 1.0f - std::pow(b1, (float)m->adam_t);
+    u.bc2 = 1.0f - std::pow(b2, (float)m->adam_t);
+    u.loss = m->lossp;
+    u.nloss = nb;
+    u.loss_out = loss_d + it;
+    if ((rc = backward(m, batch, u, s))) break;
   }
   if (rc == BIHIP_OK && loss_host != nullptr && steps > 0) {
     std::vector<float> h(steps);

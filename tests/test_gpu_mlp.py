@@ -90,3 +90,42 @@ def test_training_reduces_loss(ctx, torch_gpu):
     assert np.isfinite(losses).all()
     assert l1 < 0.1 * l0
     net.close()
+
+
+@pytest.mark.parametrize("dims,n", [
+    ([5, 64, 3], 1), ([64, 128, 64], 64), ([41, 256, 256, 256, 40], 257), ([7, 65, 130, 9], 700),
+    ([64, 4096, 4096, 64], 1024)])
+def test_gradients_and_a_training_step_against_float64(ctx, torch_gpu, dims, n):
+    """One row, whole and partial splits of 256 rows, ragged widths, and a network whose
+    partial sums are too large for one launch: the gradient against float64 (bfloat16
+    operands, whose rounding costs under 5%), and one Adam step against the update that
+    this gradient gives (float32 arithmetic)."""
+    torch = torch_gpu
+    net = capi.MLP(ctx, dims, seed=5)
+    X, T, Xd, Td = _data(torch, n, dims[0], dims[-1], seed=8)
+    p0 = net.get_params()
+    loss, g = net.loss_grad(Xd, Td)
+    ps, off = [], 0
+    for i, o in zip(dims[:-1], dims[1:]):
+        ps += [torch.from_numpy(p0[off:off + o * i].reshape(o, i)).double().cuda(),
+               torch.from_numpy(p0[off + o * i:off + o * i + o]).double().cuda()]
+        off += o * i + o
+    ps = [q.requires_grad_() for q in ps]
+    u = Xd.double()
+    for k in range(len(dims) - 1):
+        u = u @ ps[2 * k].T + ps[2 * k + 1]
+        if k + 2 < len(dims):
+            u = u * torch.sigmoid(1.702 * u)
+    ref = (u - Td.double()).square().mean()
+    gr = torch.cat([q.reshape(-1) for q in torch.autograd.grad(ref, ps)]).cpu().numpy()
+    assert loss == pytest.approx(float(ref), rel=2e-2)
+    assert np.linalg.norm(g - gr) < 0.05 * np.linalg.norm(gr)
+    if n % 64 == 0:
+        losses = net.train(Xd, Td, batch=n, steps=1, lr=1e-3, seed=3)
+        # one batch of every row, shuffled: the sums' order differs, the first Adam step
+        # is lr g / (|g| + eps), insensitive to it where g is not tiny
+        step = net.get_params() - p0
+        big = np.abs(g) > 1e-2 * np.abs(g).max()
+        np.testing.assert_allclose(step[big], -1e-3 * np.sign(g[big]), rtol=2e-3, atol=2e-6)
+        assert losses[0] == pytest.approx(loss, rel=1e-4)
+    net.close()
