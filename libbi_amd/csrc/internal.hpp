@@ -211,6 +211,9 @@ int launch_philox(const uint32_t* ctr, uint32_t k0, uint32_t k1, int n, uint32_t
                   hipStream_t s);
 int launch_uniforms(uint64_t seed, uint32_t step, uint32_t tag, uint32_t batch, int n, double* u,
                     hipStream_t s);
+// uniforms of indices base, base + 1, ... as bihip_uniform_host keys them
+int launch_uniforms_at(uint64_t seed, long base, uint32_t step, uint32_t tag, int n, double* u,
+                       hipStream_t s);
 int launch_normals(uint64_t seed, uint32_t index, uint32_t step, uint32_t tag, uint32_t batch,
                    int n, int precision, void* z, hipStream_t s);
 bool model_supported(const bihip_model* m);

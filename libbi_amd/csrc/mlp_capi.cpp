@@ -18,6 +18,7 @@ using namespace bihip;
 namespace {
 constexpr uint32_t TAG_MLP_INIT = 11;
 constexpr uint32_t TAG_MLP_BATCH = 12;
+constexpr long UNIF_CHUNK = 1L << 22;  // uniforms of the shuffle held at once
 int pad64(int d) { return (d + 63) / 64 * 64; }
 }  // namespace
 
@@ -460,10 +461,14 @@ int bihip_mlp_train(bihip_mlp* m, const float* X_dev, long ldx, const float* T_d
   const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
   long* perm_d = nullptr;
   float* loss_d = nullptr;
-  if ((rc = dalloc(&perm_d, (size_t)n)) || (rc = dalloc(&loss_d, (size_t)std::max(steps, 1)))) {
+  double* unif_d = nullptr;  // an epoch's uniforms
+  if ((rc = dalloc(&perm_d, (size_t)n)) || (rc = dalloc(&loss_d, (size_t)std::max(steps, 1))) ||
+      (rc = dalloc(&unif_d, (size_t)std::min(n, UNIF_CHUNK)))) {
     dfree(perm_d);
+    dfree(loss_d);
     return rc;
   }
+  std::vector<double> unif((size_t)std::min(n, UNIF_CHUNK));
   std::vector<long> perm(n);
   std::iota(perm.begin(), perm.end(), 0L);
   long pos = n;  // position in the current epoch's permutation
@@ -471,12 +476,26 @@ int bihip_mlp_train(bihip_mlp* m, const float* X_dev, long ldx, const float* T_d
   for (int it = 0; it < steps && rc == BIHIP_OK; ++it) {
     if (pos + batch > n) {  // new epoch: Fisher-Yates with keyed uniforms
       ++epoch;
-      for (long i = n - 1; i > 0; --i) {
-        const double u = bihip_uniform_host(seed, (uint32_t)i, (uint32_t)epoch, TAG_MLP_BATCH,
-                                            (uint32_t)(i >> 32));
-        const long j = std::min(i, (long)(u * (double)(i + 1)));
-        std::swap(perm[i], perm[j]);
+      // uniform i keyed by (seed, i, epoch), drawn on the device a chunk at a
+      // time: on the host they took four fifths of the shuffle
+      for (long hi = n; hi > 1 && rc == BIHIP_OK;) {
+        const long lo = (hi - 1) / UNIF_CHUNK * UNIF_CHUNK;
+        if ((rc = launch_uniforms_at(seed, lo, (uint32_t)epoch, TAG_MLP_BATCH, (int)(hi - lo),
+                                     unif_d, s)))
+          break;
+        if (hipMemcpyAsync(unif.data(), unif_d, sizeof(double) * (hi - lo), hipMemcpyDeviceToHost,
+                           s) != hipSuccess ||
+            hipStreamSynchronize(s) != hipSuccess) {
+          rc = set_error(BIHIP_EHIP, "reading the batch shuffle's uniforms failed");
+          break;
+        }
+        for (long i = hi - 1; i >= std::max(lo, 1L); --i) {
+          const long j = std::min(i, (long)(unif[i - lo] * (double)(i + 1)));
+          std::swap(perm[i], perm[j]);
+        }
+        hi = lo;
       }
+      if (rc != BIHIP_OK) break;
       // the previous epoch's batches must have read perm_d before it changes
       if (hipStreamSynchronize(s) != hipSuccess ||
           hipMemcpyAsync(perm_d, perm.data(), sizeof(long) * n, hipMemcpyHostToDevice, s) !=
@@ -520,6 +539,7 @@ int bihip_mlp_train(bihip_mlp* m, const float* X_dev, long ldx, const float* T_d
   (void)hipStreamSynchronize(s);
   dfree(perm_d);
   dfree(loss_d);
+  dfree(unif_d);
   return rc;
 }
 

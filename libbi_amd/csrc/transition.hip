@@ -323,6 +323,16 @@ __global__ void k_uniforms(uint64_t seed, uint32_t step, uint32_t tag, uint32_t 
   u[j] = u53(r.x, r.y);
 }
 
+// u[j] of index base + j, its high word as the batch id
+__global__ void k_uniforms_at(uint64_t seed, long base, uint32_t step, uint32_t tag, int n,
+                              double* u) {
+  const int j = blockIdx.x * blockDim.x + threadIdx.x;
+  if (j >= n) return;
+  const long i = base + j;
+  const u32x4 r = philox_block(seed, (uint32_t)i, step, tag, (uint32_t)(i >> 32), 0);
+  u[j] = u53(r.x, r.y);
+}
+
 template <class T>
 __global__ void k_normals(uint64_t seed, uint32_t index, uint32_t step, uint32_t tag,
                           uint32_t batch, int n, T* z) {
@@ -627,6 +637,15 @@ int launch_uniforms(uint64_t seed, uint32_t step, uint32_t tag, uint32_t batch, 
                     hipStream_t s) {
   if (n <= 0) return BIHIP_OK;
   hipLaunchKernelGGL(k_uniforms, dim3(ceil_div(n, 256)), dim3(256), 0, s, seed, step, tag, batch,
+                     n, u);
+  BIHIP_LAUNCH_CHECK();
+  return BIHIP_OK;
+}
+
+int launch_uniforms_at(uint64_t seed, long base, uint32_t step, uint32_t tag, int n, double* u,
+                       hipStream_t s) {
+  if (n <= 0) return BIHIP_OK;
+  hipLaunchKernelGGL(k_uniforms_at, dim3(ceil_div(n, 256)), dim3(256), 0, s, seed, base, step, tag,
                      n, u);
   BIHIP_LAUNCH_CHECK();
   return BIHIP_OK;

@@ -118,7 +118,7 @@ def test_gradients_and_a_training_step_against_float64(ctx, torch_gpu, dims, n):
             u = u * torch.sigmoid(1.702 * u)
     ref = (u - Td.double()).square().mean()
     gr = torch.cat([q.reshape(-1) for q in torch.autograd.grad(ref, ps)]).cpu().numpy()
-    assert loss == pytest.approx(float(ref), rel=2e-2)
+    assert loss == pytest.approx(float(ref.detach()), rel=2e-2)
     assert np.linalg.norm(g - gr) < 0.05 * np.linalg.norm(gr)
     if n % 64 == 0:
         losses = net.train(Xd, Td, batch=n, steps=1, lr=1e-3, seed=3)
@@ -128,4 +128,28 @@ def test_gradients_and_a_training_step_against_float64(ctx, torch_gpu, dims, n):
         big = np.abs(g) > 1e-2 * np.abs(g).max()
         np.testing.assert_allclose(step[big], -1e-3 * np.sign(g[big]), rtol=2e-3, atol=2e-6)
         assert losses[0] == pytest.approx(loss, rel=1e-4)
+    net.close()
+
+
+@pytest.mark.parametrize("n", [64, 5000, (1 << 22) + 64])
+def test_minibatches_follow_the_keyed_shuffle(ctx, torch_gpu, n):
+    """The first minibatch is the head of the Fisher-Yates shuffle with the keyed
+    uniforms (tag 12, step = epoch), also where its uniforms come in two chunks: a linear
+    network of one weight sees the mean square of its inputs."""
+    torch = torch_gpu
+    seed, batch = 11, 64
+    net = capi.MLP(ctx, [1, 1], seed=1)
+    net.set_params(np.array([1.0, 0.0], np.float32))
+    x = torch.from_numpy((np.arange(n) % 251).astype(np.float32)).cuda()  # exact in bfloat16
+    loss = net.train(x[:, None], torch.zeros((n, 1), device="cuda"), batch, 1, 1e-6, seed=seed)[0]
+    u = torch.empty(n, dtype=torch.float64, device="cuda")
+    capi.check(capi.lib().bihip_uniforms(ctx.h, seed, 0, 12, 0, n, capi.ptr(u)))
+    ctx.sync()
+    i = np.arange(n)
+    j = np.minimum(i, (u.cpu().numpy() * (i + 1)).astype(np.int64)).tolist()
+    perm = list(range(n))
+    for k in range(n - 1, 0, -1):
+        perm[k], perm[j[k]] = perm[j[k]], perm[k]
+    ref = np.mean((np.array(perm[:batch]) % 251).astype(np.float64) ** 2)
+    assert loss == pytest.approx(ref, rel=1e-5)
     net.close()
