@@ -64,50 +64,33 @@ __device__ __forceinline__ M make_model(const BatchArgs& a, int j) {
   return M(ma);
 }
 
-template <int BLOCK>
-__device__ __forceinline__ u128 block_incl_scan_u128(u128 v, u128* lds, u128& total) {
+// Scans of one integer value per thread of a workgroup of BLOCK threads: DPP
+// within the waves, one row of lanes over the waves' sums.
+template <int BLOCK, class V>
+__device__ __forceinline__ V block_incl_scan(V v, V* lds, V& total) {
   constexpr int NW = BLOCK / WAVE;
-  const int lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE;
-#pragma unroll
-  for (int o = 1; o < WAVE; o <<= 1) {
-    const u128 u = shfl_up_v(v, o);
-    if (lane >= o) v = u + v;
-  }
+  static_assert(NW <= 16, "the waves' sums fit a row of lanes");
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE));
+  v = wave_inclusive_scan(v);
   if (lane == WAVE - 1) lds[w] = v;
   __syncthreads();
-  u128 pre(0), tot(0);
-#pragma unroll
-  for (int i = 0; i < NW; ++i) {
-    if (i < w) pre = pre + lds[i];
-    tot = tot + lds[i];
-  }
+  const int q = lane & 15;
+  const V s = row_inclusive_scan(q < NW ? lds[q] : V(0));
   __syncthreads();
-  total = tot;
-  return pre + v;
+  total = read_lane(s, 15);
+  return w > 0 ? read_lane(s, w - 1) + v : v;
+}
+
+template <int BLOCK>
+__device__ __forceinline__ u128 block_incl_scan_u128(u128 v, u128* lds, u128& total) {
+  return block_incl_scan<BLOCK>(v, lds, total);
 }
 
 template <int BLOCK>
 __device__ __forceinline__ uint64_t block_excl_scan_u64(uint64_t v, uint64_t* lds,
                                                         uint64_t& total) {
-  constexpr int NW = BLOCK / WAVE;
-  const int lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE;
-  uint64_t incl = v;
-#pragma unroll
-  for (int o = 1; o < WAVE; o <<= 1) {
-    const uint64_t u = __shfl_up(incl, o, WAVE);
-    if (lane >= o) incl += u;
-  }
-  if (lane == WAVE - 1) lds[w] = incl;
-  __syncthreads();
-  uint64_t pre = 0, tot = 0;
-#pragma unroll
-  for (int i = 0; i < NW; ++i) {
-    if (i < w) pre += lds[i];
-    tot += lds[i];
-  }
-  __syncthreads();
-  total = tot;
-  return pre + incl - v;
+  return block_incl_scan<BLOCK>(v, lds, total) - v;
 }
 
 __device__ __forceinline__ int sys_offspring(double Ws, double W, int n, double a) {

@@ -127,15 +127,54 @@ __device__ __forceinline__ u128 shfl_xor_v<u128>(const u128& v, int o) {
   return u128(__shfl_xor(v.lo, o, WAVE), __shfl_xor(v.hi, o, WAVE));
 }
 
-// Block sum in a fixed order for any V with operator+.
+// The value `CTRL` names, zero where no lane is (or ROWS leaves the row out).
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint64_t dpp_or_zero(uint64_t v) {
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)v, CTRL, ROWS, 0xF,
+                                                            false);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(v >> 32), CTRL,
+                                                            ROWS, 0xF, false);
+  return ((uint64_t)hi << 32) | lo;
+}
+template <int CTRL, int ROWS>
+__device__ __forceinline__ u128 dpp_or_zero(const u128& v) {
+  return u128(dpp_or_zero<CTRL, ROWS>(v.lo), dpp_or_zero<CTRL, ROWS>(v.hi));
+}
+
+// Inclusive scans of integer values over a row of 16 lanes and over the wave
+// (row shifts, then the last lane of each row to the rows after it).
+template <class V>
+__device__ __forceinline__ V row_inclusive_scan(V v) {
+  v = v + dpp_or_zero<0x111, 0xF>(v);  // row_shr 1
+  v = v + dpp_or_zero<0x112, 0xF>(v);
+  v = v + dpp_or_zero<0x114, 0xF>(v);
+  return v + dpp_or_zero<0x118, 0xF>(v);
+}
+template <class V>
+__device__ __forceinline__ V wave_inclusive_scan(V v) {
+  v = row_inclusive_scan(v);
+  v = v + dpp_or_zero<0x142, 0xA>(v);  // row_bcast 15 into rows 1 and 3
+  return v + dpp_or_zero<0x143, 0xC>(v);  // row_bcast 31 into rows 2 and 3
+}
+
+__device__ __forceinline__ uint64_t read_lane(uint64_t v, int lane) {
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, lane);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), lane);
+  return ((uint64_t)hi << 32) | lo;
+}
+__device__ __forceinline__ u128 read_lane(const u128& v, int lane) {
+  return u128(read_lane(v.lo, lane), read_lane(v.hi, lane));
+}
+
+// Sum of an integer value over the workgroup of SCAN_BLOCK threads.  (Through
+// DPP: a shuffle through LDS costs its latency in each of the six steps.)
 template <class V>
 __device__ __forceinline__ V block_sum_v(V v, V* lds) {
   constexpr int NW = SCAN_BLOCK / WAVE;
-#pragma unroll
-  for (int o = 1; o < WAVE; o <<= 1) v = v + shfl_xor_v(v, o);
+  v = wave_inclusive_scan(v);
   const int w = threadIdx.x / WAVE, l = threadIdx.x & (WAVE - 1);
   __syncthreads();
-  if (l == 0) lds[w] = v;
+  if (l == WAVE - 1) lds[w] = v;
   __syncthreads();
   V r = lds[0];
 #pragma unroll
@@ -143,20 +182,14 @@ __device__ __forceinline__ V block_sum_v(V v, V* lds) {
   return r;
 }
 
-// Exclusive scan of one value per thread across the block, in a fixed order;
-// agg receives the block total.  lds holds SCAN_BLOCK / WAVE values.
+// Exclusive scan of one integer value per thread across the block; agg receives
+// the block total.  lds holds SCAN_BLOCK / WAVE values.
 template <class V>
 __device__ __forceinline__ V block_exclusive_scan(V v, V* lds, V& agg) {
   constexpr int NW = SCAN_BLOCK / WAVE;
   const int lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE;
-  V incl = v;
-#pragma unroll
-  for (int o = 1; o < WAVE; o <<= 1) {
-    const V u = shfl_up_v(incl, o);
-    if (lane >= o) incl = u + incl;
-  }
-  V excl = shfl_up_v(incl, 1);
-  if (lane == 0) excl = V(0);
+  const V incl = wave_inclusive_scan(v);
+  const V excl = incl - v;
   __syncthreads();  // lds may still be read by an earlier reduction
   if (lane == WAVE - 1) lds[w] = incl;
   __syncthreads();

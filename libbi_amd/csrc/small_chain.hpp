@@ -38,45 +38,6 @@ __device__ __forceinline__ uint64_t ef_pair(int o) {
 
 constexpr int SMALL_BLOCK = 1024;
 
-// The value `CTRL` names, zero where no lane is (or ROWS leaves the row out).
-template <int CTRL, int ROWS>
-__device__ __forceinline__ uint64_t dpp_or_zero(uint64_t v) {
-  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)v, CTRL, ROWS, 0xF,
-                                                            false);
-  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(v >> 32), CTRL,
-                                                            ROWS, 0xF, false);
-  return ((uint64_t)hi << 32) | lo;
-}
-template <int CTRL, int ROWS>
-__device__ __forceinline__ u128 dpp_or_zero(const u128& v) {
-  return u128(dpp_or_zero<CTRL, ROWS>(v.lo), dpp_or_zero<CTRL, ROWS>(v.hi));
-}
-
-// Inclusive scans of integer values over a row of 16 lanes and over the wave
-// (row shifts, then the last lane of each row to the rows after it).
-template <class V>
-__device__ __forceinline__ V row_inclusive_scan(V v) {
-  v = v + dpp_or_zero<0x111, 0xF>(v);  // row_shr 1
-  v = v + dpp_or_zero<0x112, 0xF>(v);
-  v = v + dpp_or_zero<0x114, 0xF>(v);
-  return v + dpp_or_zero<0x118, 0xF>(v);
-}
-template <class V>
-__device__ __forceinline__ V wave_inclusive_scan(V v) {
-  v = row_inclusive_scan(v);
-  v = v + dpp_or_zero<0x142, 0xA>(v);  // row_bcast 15 into rows 1 and 3
-  return v + dpp_or_zero<0x143, 0xC>(v);  // row_bcast 31 into rows 2 and 3
-}
-
-__device__ __forceinline__ uint64_t read_lane(uint64_t v, int lane) {
-  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, lane);
-  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), lane);
-  return ((uint64_t)hi << 32) | lo;
-}
-__device__ __forceinline__ u128 read_lane(const u128& v, int lane) {
-  return u128(read_lane(v.lo, lane), read_lane(v.hi, lane));
-}
-
 // Inclusive scan of one integer value per thread over the workgroup (at most
 // 16 waves); total receives the sum.  Each wave scans the waves' sums in one
 // row of lanes; through shuffles and a serial pass over the 16 sums in every
