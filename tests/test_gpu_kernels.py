@@ -61,6 +61,26 @@ def test_normals(ctx, orc, torch_gpu, precision):
     np.testing.assert_allclose(host(out), ref, rtol=tol, atol=tol)
 
 
+# Draws 2^21 of index 10 hold a pair of radius zero (u1 = 1) and the largest radius
+# (u1 = 2^-24, 5.768); index 5 holds neither.  The radius is correctly rounded from a
+# base-2 logarithm within one unit (2^-23 relative, halved by the root) times a constant;
+# v_sin and v_cos are within 2^-21 absolute: |error| <= 5.77 (2^-22 + 2^-21) < 4.2e-6.
+@pytest.mark.parametrize("index", [5, 10])
+def test_normals_f32_radius_range(ctx, orc, torch_gpu, index):
+    n = 1 << 21
+    out = empty(n, torch_gpu.float32)
+    capi.check(L().bihip_normals(ctx.h, 77, index, 9, capi.TAG_NOISE, 1, n, capi.F32, _c(out)))
+    z = host(out).astype(np.float64)
+    ref = orc.normals(77, index, 9, orc.TAG_NOISE, n, bits=24, batch=1)
+    r = np.hypot(ref[0::2], ref[1::2])
+    assert (np.any(r == 0.0) and r.max() > 5.76) == (index == 10)
+    assert np.all(z.reshape(-1, 2)[r == 0.0] == 0.0)
+    np.testing.assert_allclose(z, ref, rtol=0, atol=4.2e-6)
+    # the root itself: the pair's length against the exact radius, where the angle's
+    # error enters as cos^2 + sin^2 only
+    np.testing.assert_allclose(np.hypot(z[0::2], z[1::2]), r, rtol=0, atol=4.2e-6)
+
+
 # ---------------------------------------------------------------- model kernels
 MODELS = [
     ("pz", capi.RK4, capi.F64, 0),
