@@ -250,9 +250,14 @@ int mlp_inference_weights(bihip_mlp* m, hipStream_t user, const uint16_t* W[MLP_
                                                out_interleave > m->pad[L]))
     return set_error(BIHIP_EINVAL, "output interleave does not fit the padded width");
   int rc;
+  hipStream_t s = ctx_stream_of(m->ctx);
+  // a replay would not lay out the weights that the network has by then
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  BIHIP_HIP(hipStreamIsCapturing(s, &cap));
+  if (cap != hipStreamCaptureStatusNone)
+    return set_error(BIHIP_EHIP, "inference weights are not laid out under stream capture");
   if (m->Winf == nullptr && (rc = dalloc(&m->Winf, m->nW))) return rc;
   if (m->binf == nullptr && (rc = dalloc(&m->binf, m->ntot - m->nW))) return rc;
-  hipStream_t s = ctx_stream_of(m->ctx);
   InferenceWeightsArgs a{};
   a.P = m->P;
   a.W = m->Winf;
