@@ -73,9 +73,13 @@ HBM_PEAK_GBS = 8000.0
 #    (SQ_INSTS_VALU_FMA_F32, _ADD_F32, _MUL_F32, _TRANS_F32, _CVT, _INT64); the
 #    rest (SQ_INSTS_VALU_INT32 and the moves, DPP, compares, selects and bit
 #    operations no class counter covers) issue at the integer probe's rate.
-L96_TRAFFIC_BYTES = 396_513_232
-L96_VALU_PER_LAUNCH = 1.289e8
-L96_VALU_FP32_SHARE = 0.735
+# Both follow the DOPRI5 steps of the window's particles, so they are counted
+# again when a change moves the FP32 trajectory.  The probe's FMA reads one
+# operand from a scalar register, which halves its rate; the kernel's mostly do
+# not, so a fraction near 1 is the probe's rate reached, not the chip's limit.
+L96_TRAFFIC_BYTES = 390_671_360
+L96_VALU_PER_LAUNCH = 1.374e8
+L96_VALU_FP32_SHARE = 0.766
 
 
 def parse():
