@@ -16,6 +16,8 @@
 // in the state type T.
 #pragma once
 
+#include <type_traits>
+
 #include "common.hpp"
 
 namespace bihip {
@@ -220,6 +222,10 @@ struct ModelL96 {
     eval<false>(grp, x, k);
   }
   __device__ __forceinline__ T forcing() const { return F; }
+  // d = 8 differs between the first step of an interval and the later ones
+  __device__ __forceinline__ static constexpr bool fuse_first(bool host_k7, int n) {
+    return host_k7 || (LPP == 2 && n > 0);
+  }
 };
 
 // Scalar linear-Gaussian: dx/dt = -lambda x.
@@ -261,15 +267,41 @@ __device__ __forceinline__ bool slice_has(int g, int i) {
   else return i + 1 < M::DL || (g & 1) == 0;
 }
 
+__device__ __forceinline__ float fused(float a, float b, float c) {
+  return __builtin_fmaf(a, b, c);
+}
+__device__ __forceinline__ double fused(double a, double b, double c) {
+  return __builtin_fma(a, b, c);
+}
+
 // Sum of squares over the particle's dimensions, the same bits in every lane of
 // the group: each slice in order, then the slices by a butterfly.  With uneven
 // slices a pair of lanes is summed in order as one slice (the even lane's sum
 // is where the odd lane starts), as half as many lanes would.
+//
+// e0 e0 + e1 e1 is one rounded product and one fused multiply-add.  A filter's
+// particles follow from the last bit of its FP32 step sizes (an ancestor that
+// moves relabels the ones after it), so a model may state which of the two is
+// fused (fuse_first, of step n of an interval with the integrator's convention
+// of k7): left to the compiler it changes with the code around it.
+template <class M, class = void>
+struct states_fused_square : std::false_type {};
+template <class M>
+struct states_fused_square<M, std::void_t<decltype(M::fuse_first(false, 0))>> : std::true_type {};
+
 template <class M, class G, class T, int DL>
-__device__ __forceinline__ T sum_squares(const G& grp, const T (&e)[DL]) {
+__device__ __forceinline__ T sum_squares(const G& grp, const T (&e)[DL], bool host_k7, int n) {
   T s = T(0);
+  if constexpr (sizeof(T) == 4 && DL >= 2 && states_fused_square<M>::value) {
+    const bool first = M::fuse_first(host_k7, n);
+    const T a = first ? e[0] : e[1], b = first ? e[1] : e[0];
+    s = fused(a, a, b * b);
 #pragma unroll
-  for (int i = 0; i < DL; ++i) s += e[i] * e[i];
+    for (int i = 2; i < DL; ++i) s = fused(e[i], e[i], s);
+  } else {
+#pragma unroll
+    for (int i = 0; i < DL; ++i) s += e[i] * e[i];
+  }
   if constexpr (uneven_slices<M>()) {
     const T before = grp.prev(s);  // outside the choice: every lane takes part
     s = (grp.g & 1) != 0 ? before : T(0);
@@ -500,7 +532,7 @@ __device__ __forceinline__ int dopri5_loop(const M& m, const G& grp, T (&x0)[M::
         er[i] = er[i] * hT / (atol + rtol * fmax(fabs(x0[i]), fabs(y6[i])));
       }
     }
-    T e2 = sum_squares<M>(grp, er) * invD;
+    T e2 = sum_squares<M>(grp, er, QUIRK, n) * invD;
     if constexpr (F32) e2 *= hT * hT;
     if (e2 <= T(1)) {
       t += h;

@@ -1,0 +1,119 @@
+"""Outputs of fixed calls as CRC-32 of their bytes (tests/golden/fixed_seed_results.json,
+test_gpu_fixed_seed.py).  A filter's particles follow from the last bits of its
+single-precision arithmetic: one ancestor that moves relabels the particles after it,
+which then draw other noise.  So a change that only regroups the arithmetic of a kernel
+shows here and nowhere else.
+
+Written by `python tests/fixed_seed.py`, on an MI355X; only where a change of the results
+is meant.
+"""
+import ctypes
+import json
+import os
+import sys
+import zlib
+
+import numpy as np
+
+if __name__ == "__main__":
+    sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+from libbi_amd import capi
+
+GOLDEN = os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden",
+                      "fixed_seed_results.json")
+
+
+def l96_state(d):
+    """A point near the Lorenz-96 attractor, from elementary float64 operations only."""
+    x = 8.0 + 0.01 * np.arange(d) * (-1.0) ** np.arange(d)
+
+    def f(u):
+        return (np.roll(u, -1) - np.roll(u, 2)) * np.roll(u, 1) - u + 8.0
+    for _ in range(400):
+        a = f(x)
+        b = f(x + 0.0125 * a)
+        c = f(x + 0.0125 * b)
+        x = x + 0.025 / 6.0 * (a + 2.0 * b + 2.0 * c + f(x + 0.025 * c))
+    return np.ascontiguousarray(x)
+
+
+def observations(d, T):
+    y = l96_state(d)[0::2][None, :] + 0.8 * np.random.default_rng(d).standard_normal((T, d // 2))
+    return np.ascontiguousarray(y)
+
+
+def crc(*arrays):
+    c = 0
+    for a in arrays:
+        c = zlib.crc32(np.ascontiguousarray(a).tobytes(), c)
+    return c
+
+
+def _transition(ctx, torch, d, prec, integ, quirk):
+    """Initial particles, one interval, its flow and the observation density (5003
+    particles: not a whole number of workgroups)."""
+    L, P = capi.lib(), 5003
+    # several steps in an interval, some rejected
+    m = capi.make_model("l96", d=d, precision=prec, integrator=integ, h0=0.02, atol=1e-6,
+                        rtol=1e-6)
+    m.host_quirk = quirk
+    dt = torch.float64 if prec == capi.F64 else torch.float32
+    X = torch.empty((d, P), dtype=dt, device="cuda")
+    Y = torch.empty_like(X)
+    lws = torch.zeros(P, dtype=torch.float64, device="cuda")
+    y = torch.from_numpy(observations(d, 1)[0]).cuda()
+    mean = l96_state(d)
+    torch.cuda.synchronize()
+    capi.check(L.bihip_init_samples(ctx.h, ctypes.byref(m), 21, 0, P, capi.ptr(X), P,
+                                    mean.ctypes.data_as(ctypes.POINTER(ctypes.c_double))))
+    capi.check(L.bihip_transition(ctx.h, ctypes.byref(m), 5, 0, 1, 0.0, 0.05, P, capi.ptr(X),
+                                  capi.ptr(Y), P, None, None))
+    capi.check(L.bihip_obs_logdensity(ctx.h, ctypes.byref(m), capi.ptr(y), P, capi.ptr(Y), P,
+                                      capi.ptr(lws)))
+    ctx.sync()
+    out = [X.cpu().numpy(), Y.cpu().numpy(), lws.cpu().numpy()]
+    capi.check(L.bihip_flow(ctx.h, ctypes.byref(m), 0.05, 0.1, P, capi.ptr(Y), P, None, None))
+    ctx.sync()
+    return crc(*out, Y.cpu().numpy())
+
+
+def _filter(ctx, model, d, P, T, resampler=capi.SYSTEMATIC, learn=None):
+    """States, log-weights, log-likelihood increments and effective sample sizes after T
+    intervals."""
+    f = capi.ParticleFilter(ctx, model, P, T, 0.05, 7, resampler, 0.5)
+    f.set_observations(observations(d, T))
+    if learn is not None:
+        learn(f)
+    f.init(l96_state(d))
+    f.step(T)
+    out = f.outputs()
+    X, _, lws = f.state()
+    r = crc(X[:, :P].cpu().numpy(), lws.cpu().numpy(), out["logIncrements"], out["ess"])
+    f.close()
+    return r
+
+
+def cases():
+    """name -> function of (context, torch)"""
+    out = {}
+    for d in (8, 40):
+        for p, prec in (("f32", capi.F32), ("f64", capi.F64)):
+            for i, integ, quirk in (("dopri5", capi.DOPRI5, 0), ("host-dopri5", capi.DOPRI5, 1),
+                                    ("rk4", capi.RK4, 0)):
+                out[f"transition-l96-{d}-{p}-{i}"] = (
+                    lambda ctx, torch, a=(d, prec, integ, quirk): _transition(ctx, torch, *a))
+            for r, res in (("systematic", capi.SYSTEMATIC), ("multinomial", capi.MULTINOMIAL)):
+                out[f"filter-l96-{d}-{p}-{r}"] = (
+                    lambda ctx, torch, a=(d, prec, res): _filter(
+                        ctx, capi.make_model("l96", d=a[0], precision=a[1], init_sd=0.3), a[0],
+                        30011, 6, a[2]))
+    return out
+
+
+if __name__ == "__main__":
+    import torch
+    ctx = capi.Context(0)
+    got = {name: f(ctx, torch) for name, f in cases().items()}
+    with open(GOLDEN, "w") as f:
+        json.dump(got, f, indent=1, sort_keys=True)
+        f.write("\n")
