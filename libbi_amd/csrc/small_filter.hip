@@ -51,7 +51,11 @@ __global__ __launch_bounds__(SMALL_BLOCK) void k_filter_small(SmallFilterArgs a)
   constexpr int DL = M::DL, NB = SMALL_BLOCK / TRANS_BLOCK, WPB = TRANS_BLOCK / WAVE;
   static_assert(NB == 4 && WPB == 4, "a quad of lanes combines the partials");
   __shared__ SmallChainLds<1, true> chain;
-  __shared__ double wm[SMALL_BLOCK / WAVE], w1[SMALL_BLOCK / WAVE], w2[SMALL_BLOCK / WAVE];
+  // the waves' maxima, in two buffers in turn: the last reads of a step's maxima
+  // and the writes of the next one's have no barrier between them in a step that
+  // does not resample (the sums' have the maxima's)
+  __shared__ double wmax[2][SMALL_BLOCK / WAVE];
+  __shared__ double w1[SMALL_BLOCK / WAVE], w2[SMALL_BLOCK / WAVE];
   const int p = threadIdx.x, lane = p & (WAVE - 1), w = p / WAVE;
   const bool active = p < a.P;
   const int nb = (a.P + TRANS_BLOCK - 1) / TRANS_BLOCK;
@@ -116,6 +120,7 @@ __global__ __launch_bounds__(SMALL_BLOCK) void k_filter_small(SmallFilterArgs a)
     }
 
     // ---- partials of TRANS_BLOCK particles, as block_weight_partial forms them
+    double* const wm = wmax[s & 1];
     const double vm = wave_max(nlw);
     if (lane == 0) wm[w] = vm;
     __syncthreads();  // also: the new states are visible to the next step's gather

@@ -117,6 +117,29 @@ def test_small_filter_equals_the_separate_launches(ctx, kind, prec, P, resampler
             np.testing.assert_array_equal(out[key], v, err_msg=key)
 
 
+@pytest.mark.parametrize("P", [513, 1000, 1024])
+def test_small_filter_without_resampling(ctx, P):
+    """Steps that do not resample follow each other with the fewest barriers, and the
+    waves' work differs (adaptive steps): the same bits as the separate launches."""
+    m = capi.make_model("pz", integrator=capi.DOPRI5, h0=0.01)
+    T = 256
+    y = (2.0 + 0.2 * np.sin(np.arange(T))).reshape(T, 1)
+    got = []
+    for record in (True, False):
+        pf = capi.ParticleFilter(ctx, m, P, T, 1.0, 7, ess_rel=0.0, record=record)
+        pf.set_observations(y)
+        pf.init()
+        pf.step(T)
+        out = pf.outputs()
+        X, _, lws = pf.state()
+        out["X"], out["lws"] = X[:, :P].cpu().numpy(), lws.cpu().numpy()
+        got.append(out)
+        pf.close()
+    assert not got[0]["resampled"].any()
+    for key, v in got[0].items():
+        np.testing.assert_array_equal(got[1][key], v, err_msg=key)
+
+
 @pytest.mark.parametrize("resampler", [capi.SYSTEMATIC, capi.STRATIFIED, capi.MULTINOMIAL])
 def test_pz_filter_large_population_parity(ctx, orc, resampler):
     """N = 2^21 + 5: more than 1024 tiles of 2048 particles, so the resampling
