@@ -153,8 +153,8 @@ struct ModelPZ {
 //
 // UNEVEN: LPP leaves LPP / 2 of D over; the even lanes of a group then hold DL
 // elements and the odd ones DL - 1, their last register standing for nothing
-// (its derivative is kept at zero, so it adds nothing to an error norm, and no
-// neighbour reads it).
+// (its derivative is kept at zero, no error norm takes it, and no neighbour
+// reads it).
 template <class T, int D_, int LPP_>
 struct ModelL96 {
   static constexpr int D = D_, LPP = LPP_, DL = (D_ + LPP_ - 1) / LPP_, NOBS = D_ / 2;
@@ -303,10 +303,12 @@ __device__ __forceinline__ T sum_squares(const G& grp, const T (&e)[DL], bool ho
     for (int i = 0; i < DL; ++i) s += e[i] * e[i];
   }
   if constexpr (uneven_slices<M>()) {
-    const T before = grp.prev(s);  // outside the choice: every lane takes part
-    s = (grp.g & 1) != 0 ? before : T(0);
+    // the even lane's sum is its whole slice; the odd lane goes on from there with
+    // the elements it has (its last register stands for none: its scaled error is
+    // 0 / 0 for atol = 0), and both take the odd lane's result
+    s = grp.prev(s);
 #pragma unroll
-    for (int i = 0; i < DL; ++i) s += e[i] * e[i];
+    for (int i = 0; i + 1 < DL; ++i) s += e[i] * e[i];
     return grp.sum_pairs(dpp<QP_ODD>(s));
   } else {
     return grp.sum(s);

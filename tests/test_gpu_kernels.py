@@ -212,6 +212,33 @@ def test_l96_d200_uneven_slices(ctx, orc, torch_gpu, P, prec, integ):
     np.testing.assert_allclose(host(lws), ref_l, rtol=1e-12, atol=1e-10)
 
 
+@pytest.mark.parametrize("F", [8.0, 0.0])
+@pytest.mark.parametrize("prec", [capi.F64, capi.F32])
+@pytest.mark.parametrize("d", [8, 40, 200])
+def test_l96_relative_tolerance_alone(ctx, orc, torch_gpu, d, prec, F):
+    """atol = 0: the scaled error of a component divides by rtol |x|, so nothing that is
+    not a component may enter the norm.  One interval against the oracle: for float64 its
+    step counts too; for float32 both trajectories are within the tolerance's error."""
+    P = 19
+    gm = capi.make_model("l96", d=d, precision=prec, atol=0.0, rtol=1e-5, F=F, h0=0.02)
+    om = oracle_model(orc, gm)
+    rng = np.random.default_rng(d)
+    X = (l96_spun_up(orc, d=d)[:, None] + 0.3 * rng.normal(size=(d, P)))
+    X = X.astype(np.float64 if prec == capi.F64 else np.float32)
+    Xg, Y = dev(X), dev(np.zeros_like(X))
+    ns = empty(P, torch_gpu.int32)
+    capi.check(L().bihip_transition(ctx.h, ctypes.byref(gm), 5, 0, 4, 0.25, 0.30, P, _c(Xg),
+                                    _c(Y), P, None, _c(ns)))
+    ref, rns = orc.transition(om, 5, 4, 0.25, 0.30, X.astype(np.float64), return_steps=True)
+    # float64: rounding, which the norm of a component near zero magnifies; float32: steps
+    # of other sizes, each within rtol |x|, and rounding
+    tol = 1e-10 if prec == capi.F64 else 2e-4
+    np.testing.assert_allclose(host(Y).astype(np.float64), ref, rtol=tol, atol=tol)
+    assert host(ns).max() < gm.nsteps
+    if prec == capi.F64:
+        np.testing.assert_array_equal(host(ns), rns)
+
+
 @pytest.mark.parametrize("prec", [capi.F64, capi.F32])
 def test_transition_gathers_rows(ctx, orc, torch_gpu, prec):
     P = 3000
