@@ -189,6 +189,7 @@ struct TransLaunch {
 // Noise variables per particle of a built-in model (PZ: alpha; Lorenz-96:
 // w[d]; LG: w), 0 for a generated one.
 int noise_width_of(const bihip_model* m);
+// Weight partials that a transition with `partials` writes.
 int transition_blocks(const bihip_model* m, int P);
 // A generated model whose steps [t0 + k dt, t0 + (k+1) dt], k < steps, are each
 // one sub-interval of its delta starting at a multiple of it.

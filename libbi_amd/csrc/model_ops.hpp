@@ -64,6 +64,30 @@ __device__ __forceinline__ double obs_terms(const ModelL96<T, D, LPP>& m,
       const double z = (y[(lo + i) >> 1] - (double)x[i]) * inv;
       s += -0.5 * (z * z) + c;
     }
+  } else if constexpr (ModelL96<T, D, LPP>::UNEVEN) {
+    // a pair of lanes is summed in order as one slice: the odd lane goes on from
+    // the even one's sum and returns the pair's, the even one zero
+    const int o = lo & 1;
+    const bool even = (threadIdx.x & 1) == 0;
+    double v[DL / 2];
+#pragma unroll
+    for (int i = 0; i + 1 < DL; i += 2) {
+      // two values, not an element picked by a run-time index (which the
+      // compiler would turn into a chain of compares over the slice)
+      T xe = x[i], xo = x[i + 1];
+      asm("" : "+v"(xe), "+v"(xo));
+      const double z = (y[(lo + i + o) >> 1] - (double)(o ? xo : xe)) * inv;
+      v[i / 2] = -0.5 * (z * z) + c;
+      s += v[i / 2];
+    }
+    if (o == 0 && even) {  // the last element of a slice that has it
+      const double z = (y[(lo + DL - 1) >> 1] - (double)x[DL - 1]) * inv;
+      s += -0.5 * (z * z) + c;
+    }
+    s = dpp<ROW_ROR1>(s);
+#pragma unroll
+    for (int i = 0; i < DL / 2; ++i) s += v[i];
+    s = even ? 0.0 : s;
   } else {  // odd slices: the observed (even) dimensions alternate with the lane
     const int o = lo & 1;
 #pragma unroll
@@ -77,8 +101,7 @@ __device__ __forceinline__ double obs_terms(const ModelL96<T, D, LPP>& m,
       const double z = (y[(lo + j) >> 1] - xv) * inv;
       s += -0.5 * (z * z) + c;
     }
-    // the last element is observed only for even starts, in lanes that have it
-    if (o == 0 && (!ModelL96<T, D, LPP>::UNEVEN || lo % (2 * DL - 1) == 0)) {
+    if (o == 0) {  // the last element is observed only for even starts
       const double z = (y[(lo + DL - 1) >> 1] - (double)x[DL - 1]) * inv;
       s += -0.5 * (z * z) + c;
     }

@@ -152,9 +152,9 @@ struct ModelPZ {
 // Lorenz-96: dx_i/dt = (x_{i+1} - x_{i-2}) x_{i-1} - x_i + F, cyclic.
 //
 // UNEVEN: LPP leaves LPP / 2 of D over; the even lanes of a group then hold DL
-// elements and the odd ones DL - 1, their last register standing for nothing
-// (its derivative is kept at zero, no error norm takes it, and no neighbour
-// reads it).
+// elements and the odd ones DL - 1.  The odd lanes' last register goes through
+// the arithmetic but stands for nothing: no neighbour, error norm, observation
+// or store reads it.
 template <class T, int D_, int LPP_>
 struct ModelL96 {
   static constexpr int D = D_, LPP = LPP_, DL = (D_ + LPP_ - 1) / LPP_, NOBS = D_ / 2;
@@ -193,7 +193,6 @@ struct ModelL96 {
         if constexpr (FORCED) k[i] = (a - b) * c - x[i] + F;
         else k[i] = (a - b) * c - x[i];
       }
-      k[DL - 1] = full ? k[DL - 1] : T(0);
       return;
     } else if constexpr (LPP == 1) {
       xm2 = x[DL - 2];

@@ -93,10 +93,26 @@ def _filter(ctx, model, d, P, T, resampler=capi.SYSTEMATIC, learn=None):
     return r
 
 
+def _bank(ctx, d, B, P, T, learn=None):
+    """Increments, effective sample sizes and the last filter's states of a bank."""
+    m = capi.make_model("l96", d=d, precision=capi.F32, init_sd=0.3)
+    b = capi.FilterBank(ctx, m, P, T, 0.05, 11, np.linspace(7.6, 8.4, B), ess_rel=0.5)
+    if learn is not None:
+        learn(b)
+    b.set_observations(observations(d, T))
+    b.init(l96_state(d))
+    b.step(T)
+    out = b.outputs()
+    X = b.state(B - 1)[0]
+    r = crc(out["logIncrements"], out["ess"], X[:, :P].cpu().numpy())
+    b.close()
+    return r
+
+
 def cases():
     """name -> function of (context, torch)"""
     out = {}
-    for d in (8, 40):
+    for d in (8, 40, 200):
         for p, prec in (("f32", capi.F32), ("f64", capi.F64)):
             for i, integ, quirk in (("dopri5", capi.DOPRI5, 0), ("host-dopri5", capi.DOPRI5, 1),
                                     ("rk4", capi.RK4, 0)):
@@ -106,7 +122,8 @@ def cases():
                 out[f"filter-l96-{d}-{p}-{r}"] = (
                     lambda ctx, torch, a=(d, prec, res): _filter(
                         ctx, capi.make_model("l96", d=a[0], precision=a[1], init_sd=0.3), a[0],
-                        30011, 6, a[2]))
+                        30011 if a[0] < 200 else 5003, 6, a[2]))
+        out[f"bank-l96-{d}"] = lambda ctx, torch, d=d: _bank(ctx, d, 3, 2049, 5)
     return out
 
 
