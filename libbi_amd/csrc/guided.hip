@@ -190,7 +190,8 @@ __global__ __launch_bounds__(GP_THREADS) void k_guided(GuidedArgs a) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) xt[i] = xn[i];
       if (t + 1 < GOUT_TILES) load_tile(t + 1, xn);
-      const f32x16 o = linear_tile<GH / 16, GH>(buf[AT & 1], dt, t, bias + 3 * GH, nxt, lane);
+      const f32x16 o =
+          linear_tile<GH / 16, GH, true>(buf[AT & 1], dt, t, bias + 3 * GH, nxt, lane);
 #pragma unroll
       for (int q = 0; q < 2; ++q) {
         if (16 * t + 8 * q < GD) {

@@ -63,11 +63,6 @@ __device__ __forceinline__ float gelu_grad_f(float z) {
   return s + 1.702f * z * s * (1.0f - s);
 }
 
-// The same with the exponential's two factors as one (the fused kernels).
-__device__ __forceinline__ float gelu_fused(float z) {
-  return z * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-2.45546696f * z));
-}
-
 __device__ __forceinline__ f32x16 mfma32(const u16x8& a, const u16x8& b, const f32x16& c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
                                                  __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
@@ -252,24 +247,28 @@ __device__ __forceinline__ void gelu_tiles(const uint8_t* buf, const float* bias
     }
 #pragma unroll
     for (int q = 0; q < 8; ++q)
-      out[2 * t + (q >> 2)][q & 3] = cvt_pk_bf16(gelu_fused(acc[2 * q] + b[2 * q]),
-                                                 gelu_fused(acc[2 * q + 1] + b[2 * q + 1]));
+      out[2 * t + (q >> 2)][q & 3] = cvt_pk_bf16(gelu_f(acc[2 * q] + b[2 * q]),
+                                                 gelu_f(acc[2 * q + 1] + b[2 * q + 1]));
   }
 }
 
 // one linear output tile (rows [32 tl, 32 tl + 32) of the staged chunk; biases
-// of tile t) of a layer with KC input chunks
-template <int KC, int K>
+// of tile t) of a layer with KC input chunks; BIAS_FIRST: the products are added
+// to the bias, else the bias to their sum
+template <int KC, int K, bool BIAS_FIRST>
 __device__ __forceinline__ f32x16 linear_tile(const uint8_t* buf, int tl, int t,
                                               const float* bias, const uint32_t (&in)[KC][4],
                                               int lane) {
   const StagedTile<K> W(buf, lane);
-  f32x16 acc = bias_tile(bias, t, lane);
+  const f32x16 b = bias_tile(bias, t, lane);
+  f32x16 acc{};
+  if constexpr (BIAS_FIRST) acc = b;
 #pragma unroll
   for (int c = 0; c < KC; ++c) {
     const u32v4 bv = {in[c][0], in[c][1], in[c][2], in[c][3]};
     acc = mfma32(W(tl, c), bv, acc);
   }
+  if constexpr (!BIAS_FIRST) acc += b;
   return acc;
 }
 

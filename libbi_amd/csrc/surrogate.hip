@@ -163,7 +163,7 @@ __global__ __launch_bounds__(SG_THREADS) void k_surrogate(SurrArgs a) {
   f32x16 yv[DO / 32];
 #pragma unroll
   for (int t = 0; t < DO / 32; ++t)
-    yv[t] = linear_tile<H / 16, H>(buf[1], t, t, bias + 3 * H, nxt, lane);
+    yv[t] = linear_tile<H / 16, H, false>(buf[1], t, t, bias + 3 * H, nxt, lane);
 
   // x' = x + s_dx y (+ noise), observation density over the even dimensions
   double obs = 0.0;

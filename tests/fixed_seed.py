@@ -17,7 +17,7 @@ import numpy as np
 
 if __name__ == "__main__":
     sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
-from libbi_amd import capi
+from libbi_amd import capi, guided, surrogate
 
 GOLDEN = os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden",
                       "fixed_seed_results.json")
@@ -109,6 +109,48 @@ def _bank(ctx, d, B, P, T, learn=None):
     return r
 
 
+SURROGATE_NORM = capi.SurrogateNorm(x_shift=2.3, x_scale=3.6, par_shift=8.0, par_scale=1.0,
+                                    dx_scale=0.3)
+GUIDED_NORM = capi.GuidedNorm(x_shift=2.3, x_scale=3.6, innov_scale=1.0, par_shift=8.0,
+                              par_scale=1.0)
+
+
+def _states(torch, d, P):
+    x = 2.3 + 3.6 * np.random.default_rng(P).standard_normal((d, P))
+    x = torch.from_numpy(x.astype(np.float32)).cuda()
+    torch.cuda.synchronize()
+    return x
+
+
+def _surrogate_flow(ctx, torch):
+    net = capi.MLP(ctx, surrogate.DIMS, seed=4)
+    out = net.surrogate_flow(SURROGATE_NORM, 8.1, _states(torch, 40, 3001))
+    ctx.sync()
+    r = crc(out.cpu().numpy())
+    net.close()
+    return r
+
+
+def _guided_propose(ctx, torch):
+    net = capi.MLP(ctx, guided.DIMS, seed=5)
+    X = _states(torch, 200, 3001)
+    inc = net.guided_propose(GUIDED_NORM, 8.2, X, observations(200, 1)[0], 5, 2)
+    ctx.sync()
+    r = crc(X.cpu().numpy(), inc.cpu().numpy())
+    net.close()
+    return r
+
+
+def _learned(ctx, kind, run):
+    """run(set): a filter or bank that the function `set` gives the network to."""
+    surr = kind == "surrogate"
+    net = capi.MLP(ctx, surrogate.DIMS if surr else guided.DIMS, seed=4)
+    r = run(lambda f: f.set_surrogate(net, SURROGATE_NORM) if surr else
+            f.set_guided(net, GUIDED_NORM))
+    net.close()
+    return r
+
+
 def cases():
     """name -> function of (context, torch)"""
     out = {}
@@ -124,6 +166,14 @@ def cases():
                         ctx, capi.make_model("l96", d=a[0], precision=a[1], init_sd=0.3), a[0],
                         30011 if a[0] < 200 else 5003, 6, a[2]))
         out[f"bank-l96-{d}"] = lambda ctx, torch, d=d: _bank(ctx, d, 3, 2049, 5)
+    out["surrogate-flow"] = _surrogate_flow
+    out["guided-propose"] = _guided_propose
+    for kind, d in (("surrogate", 40), ("guided", 200)):
+        m = capi.make_model("l96", d=d, precision=capi.F32, init_sd=0.3)
+        out[f"filter-{kind}"] = lambda ctx, torch, k=kind, m=m, d=d: _learned(
+            ctx, k, lambda give: _filter(ctx, m, d, 5003, 5, learn=give))
+        out[f"bank-{kind}"] = lambda ctx, torch, k=kind, d=d: _learned(
+            ctx, k, lambda give: _bank(ctx, d, 3, 2049, 4, learn=give))
     return out
 
 
