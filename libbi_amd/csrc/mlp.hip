@@ -312,8 +312,10 @@ __global__ __launch_bounds__(256) void k_update(UpdateArgs a) {
   float* wv = &w.x;
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
-    const float x = a.b1 * m1v[u] + (1.0f - a.b1) * gr[u];
-    const float y = a.b2 * m2v[u] + (1.0f - a.b2) * gr[u] * gr[u];
+    // which of the two products is fused is stated: a training's parameters
+    // follow from it
+    const float x = __builtin_fmaf(1.0f - a.b1, gr[u], a.b1 * m1v[u]);
+    const float y = __builtin_fmaf((1.0f - a.b2) * gr[u], gr[u], a.b2 * m2v[u]);
     m1v[u] = x;
     m2v[u] = y;
     wv[u] = wv[u] - a.lr * (x / a.bc1) / (sqrtf(y / a.bc2) + a.eps);

@@ -151,6 +151,22 @@ def _learned(ctx, kind, run):
     return r
 
 
+def _training(ctx, torch, dims, n, batch, loss):
+    """Gradient, minibatch losses and parameters of a short training."""
+    net = capi.MLP(ctx, dims, seed=5)
+    net.set_loss(loss)
+    rng = np.random.default_rng(n)
+    X = torch.from_numpy(rng.standard_normal((n, dims[0])).astype(np.float32)).cuda()
+    m = dims[-1] // 2 if loss == capi.LOSS_GAUSS else dims[-1]
+    T = torch.from_numpy(rng.standard_normal((n, m)).astype(np.float32)).cuda()
+    torch.cuda.synchronize()
+    _, g = net.loss_grad(X, T)
+    losses = net.train(X, T, batch, 30, 1e-3, seed=3)
+    r = crc(g, losses, net.get_params())
+    net.close()
+    return r
+
+
 def cases():
     """name -> function of (context, torch)"""
     out = {}
@@ -174,6 +190,12 @@ def cases():
             ctx, k, lambda give: _filter(ctx, m, d, 5003, 5, learn=give))
         out[f"bank-{kind}"] = lambda ctx, torch, k=kind, d=d: _learned(
             ctx, k, lambda give: _bank(ctx, d, 3, 2049, 4, learn=give))
+    for dims, n, batch in (([41, 256, 256, 256, 40], 1000, 320), ([5, 64, 3], 64, 64),
+                           ([7, 65, 130, 9], 700, 64)):
+        out["training-" + "-".join(map(str, dims))] = (
+            lambda ctx, torch, a=(dims, n, batch): _training(ctx, torch, *a, capi.LOSS_MSE))
+    out["training-gauss"] = (lambda ctx, torch: _training(ctx, torch, [20, 128, 16], 500, 128,
+                                                          capi.LOSS_GAUSS))
     return out
 
 
