@@ -157,8 +157,7 @@ struct StagedRows<320> {
 // the builtin the compiler waits for the copy before the next LDS read of any
 // address, which ends the overlap.  The loads write no register; they are
 // counted in vmcnt, so a wait of the compiler's own can only come late because
-// of them, never early.  m0 (their LDS address) has no other use in these
-// kernels.
+// of them, never early.  m0 holds their LDS address.
 template <int NROWS, int K, int THREADS>
 __device__ __forceinline__ void stage_async(const uint16_t* __restrict__ W, int row0,
                                             uint8_t* buf) {
@@ -177,7 +176,7 @@ __device__ __forceinline__ void stage_async(const uint16_t* __restrict__ W, int 
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
                  :
                  : "s"(lds0 + (uint32_t)(run * (1024 + S::GAP))), "v"(src)
-                 : "memory");
+                 : "m0", "memory");
   }
 }
 
