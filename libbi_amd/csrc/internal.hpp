@@ -497,8 +497,9 @@ MlpView mlp_view(const bihip_mlp* m);
 // out_interleave outputs, [m of outputs 16 t .., then s of the same outputs],
 // for networks whose outputs are a mean (first half) and a log variance;
 // b (nullable) then gets biases in the same row order.
-// Written by a kernel on the network's stream; `user` is the stream that reads
-// them next (the call waits for the kernel if it is another one).
+// Written by a kernel on the network's stream, after what other streams that
+// called for them have queued; `user` is the stream that reads them next (the
+// call waits for the kernel if it is another one).
 int mlp_inference_weights(bihip_mlp* m, hipStream_t user, const uint16_t* W[MLP_MAX_LAYERS],
                           const float* b[MLP_MAX_LAYERS] = nullptr, int out_interleave = 0);
 

@@ -98,6 +98,7 @@ def test_inference_weights_follow_the_parameters(ctx, torch_gpu, other_stream):
     X = torch.randn((40, 1000), device="cuda")
     new = capi.MLP(ctx, surrogate.DIMS, seed=9)
     net = capi.MLP(ctx, surrogate.DIMS, seed=4)
+    old = net.surrogate_flow(norm, 8.1, X)
     user = net
     s = torch.cuda.Stream()
     if other_stream:
@@ -111,12 +112,73 @@ def test_inference_weights_follow_the_parameters(ctx, torch_gpu, other_stream):
     torch.cuda.synchronize()
     ref = new.surrogate_flow(norm, 8.1, X)
     torch.cuda.synchronize()
-    assert torch.equal(second, ref) and not torch.equal(first, ref)
+    assert torch.equal(second, ref) and torch.equal(first, old)
+    assert not torch.equal(first, ref)
     if other_stream:
         user.h = None
         c2.close()
     net.close()
     new.close()
+
+
+def test_layout_waits_for_the_reads_of_other_streams(ctx, torch_gpu):
+    """Flows of many particles queued on two other streams, then new parameters and a
+    flow on the network's own stream at once: the first flows still see the old weights."""
+    torch = torch_gpu
+    norm = _norm()
+    new = capi.MLP(ctx, surrogate.DIMS, seed=9)
+    net = capi.MLP(ctx, surrogate.DIMS, seed=4)
+    X = torch.randn((40, 1 << 20), device="cuda")
+    torch.cuda.synchronize()
+    old, ref = net.surrogate_flow(norm, 8.1, X), new.surrogate_flow(norm, 8.1, X)
+    p = new.get_params()
+    ctx.sync()
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    users = [capi.Context(0, stream=s) for s in streams]
+    outs = [torch.empty_like(X) for _ in range(6)]
+    torch.cuda.synchronize()
+    for i, out in enumerate(outs):
+        capi.check(capi.lib().bihip_surrogate_flow(
+            users[i % 2].h, net.h, ctypes.byref(norm), 8.1, capi.ptr(X), capi.ptr(out),
+            X.shape[1], X.shape[1]))
+    net.set_params(p)
+    last = net.surrogate_flow(norm, 8.1, X)
+    torch.cuda.synchronize()
+    assert all(torch.equal(out, old) for out in outs)
+    assert torch.equal(last, ref) and not torch.equal(old, ref)
+    for c in users:
+        c.close()
+    net.close()
+    new.close()
+
+
+def test_layout_refuses_a_captured_stream(ctx, torch_gpu):
+    """A replay would not lay out the weights that the network has by then."""
+    torch = torch_gpu
+    s = torch.cuda.Stream()
+    c2 = capi.Context(0, stream=s)
+    net = capi.MLP(c2, surrogate.DIMS, seed=4)
+    X = torch.randn((40, 64), device="cuda")
+    out = torch.empty_like(X)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(s):
+        graph.capture_begin()
+        rc = capi.lib().bihip_surrogate_flow(c2.h, net.h, ctypes.byref(_norm()), 8.1,
+                                             capi.ptr(X), capi.ptr(out), 64, 64)
+        out.add_(1.0)  # a graph of something
+        graph.capture_end()
+    assert rc != capi.OK
+    torch.cuda.synchronize()
+    a = net.surrogate_flow(_norm(), 8.1, X)  # the network is as before
+    c2.sync()
+    ref = capi.MLP(ctx, surrogate.DIMS, seed=4)
+    b = ref.surrogate_flow(_norm(), 8.1, X)
+    ctx.sync()
+    assert torch.equal(a, b)
+    ref.close()
+    net.close()
+    c2.close()
 
 
 @pytest.mark.parametrize("P", [1, 31, 33, 256, 257, 600])
