@@ -542,7 +542,7 @@ int bihip_pfbank_set_surrogate(bihip_pfbank* b, bihip_mlp* mlp, const bihip_surr
     S.net = mlp_view(mlp);
     if (S.net.L != 4 || S.net.dims[0] != 41 || S.net.dims[4] != 40)
       return set_error(BIHIP_EINVAL, "the surrogate must be a 41-256-256-256-40 network");
-    if ((rc = mlp_inference_weights(mlp, ctx_stream_of(b->ctx), S.Winf))) return rc;
+    if ((rc = mlp_inference_weights(mlp, ctx_stream_of(b->ctx), S.Winf, S.binf))) return rc;
     S.x_shift = norm->x_shift;
     S.x_scale = norm->x_scale;
     S.dx_scale = norm->dx_scale;

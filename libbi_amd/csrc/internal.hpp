@@ -518,6 +518,7 @@ int launch_inference_weights(const InferenceWeightsArgs& a, hipStream_t s);
 struct SurrogateLaunch {
   MlpView net;
   const uint16_t* Winf[MLP_MAX_LAYERS];
+  const float* binf[MLP_MAX_LAYERS];
   float x_shift, x_scale, dx_scale;  // u = (x - x_shift) / x_scale; x' = x + dx_scale y
   double par, par_shift, par_scale;  // u_d = (par - par_shift) / par_scale
   const void* Xin;

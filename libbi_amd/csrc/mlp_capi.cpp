@@ -45,50 +45,11 @@ struct bihip_mlp {
   float* lossp = nullptr;
   uint16_t* Winf = nullptr;      // inference copy of the weights (permuted columns)
   float* binf = nullptr;         // inference copy of the biases (row order of Winf)
-  // reads of Winf, binf and the biases in P queued on other streams than the
-  // network's: what writes these next waits for them
+  // reads of Winf and binf queued on other streams than the network's: the next
+  // layout waits for them
   std::mutex readers_lock;
   std::vector<std::pair<hipStream_t, hipEvent_t>> readers;
 };
-
-// Notes that what is queued on `user` so far may read the network.  (A captured
-// stream has nothing queued, and an event recorded there would not be one of
-// this run.)
-static int note_reader(bihip_mlp* m, hipStream_t user) {
-  if (user == ctx_stream_of(m->ctx)) return BIHIP_OK;
-  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  BIHIP_HIP(hipStreamIsCapturing(user, &cap));
-  if (cap != hipStreamCaptureStatusNone) return BIHIP_OK;
-  std::lock_guard<std::mutex> hold(m->readers_lock);
-  for (auto& r : m->readers)
-    if (r.first == user) {
-      BIHIP_HIP(hipEventRecord(r.second, user));
-      return BIHIP_OK;
-    }
-  hipEvent_t e;
-  BIHIP_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-  if (hipEventRecord(e, user) != hipSuccess) {
-    (void)hipEventDestroy(e);
-    return set_error(BIHIP_EHIP, "noting a reader of the network failed");
-  }
-  m->readers.emplace_back(user, e);
-  return BIHIP_OK;
-}
-
-// The network's stream waits for the noted reads.
-static int await_readers(bihip_mlp* m, hipStream_t s) {
-  std::lock_guard<std::mutex> hold(m->readers_lock);
-  hipError_t err = hipSuccess;
-  for (auto& r : m->readers) {
-    const hipError_t e = hipStreamWaitEvent(s, r.second, 0);
-    if (err == hipSuccess) err = e;
-    (void)hipEventDestroy(r.second);  // takes effect once the event has completed
-  }
-  m->readers.clear();
-  return err == hipSuccess ? BIHIP_OK
-                           : set_error(BIHIP_EHIP, "waiting for readers of the network: %s",
-                                       hipGetErrorString(err));
-}
 
 namespace {
 
@@ -267,10 +228,8 @@ int upload_params(bihip_mlp* m, const float* flat, hipStream_t s) {
       for (int c = 0; c < din; ++c) P[m->offW[l] + (long)r * m->pad[l] + c] = flat[o++];
     for (int r = 0; r < dout; ++r) P[m->offb[l] + r] = flat[o++];
   }
-  int rc = await_readers(m, s);
-  if (rc) return rc;
   BIHIP_HIP(hipMemcpyAsync(m->P, P.data(), sizeof(float) * m->ntot, hipMemcpyHostToDevice, s));
-  rc = launch_to_bf16(m->P, m->nW, m->Wbf, s);
+  int rc = launch_to_bf16(m->P, m->nW, m->Wbf, s);
   if (rc) return rc;
   BIHIP_HIP(hipStreamSynchronize(s));
   return BIHIP_OK;
@@ -287,6 +246,45 @@ void unpack(const bihip_mlp* m, const std::vector<float>& P, float* flat) {
 }
 
 }  // namespace
+
+// Notes that what is queued on `user` so far may read the inference copy.  (A
+// captured stream has nothing queued, and an event recorded there would not be
+// one of this run.)
+static int note_reader(bihip_mlp* m, hipStream_t user) {
+  if (user == ctx_stream_of(m->ctx)) return BIHIP_OK;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  BIHIP_HIP(hipStreamIsCapturing(user, &cap));
+  if (cap != hipStreamCaptureStatusNone) return BIHIP_OK;
+  std::lock_guard<std::mutex> hold(m->readers_lock);
+  for (auto& r : m->readers)
+    if (r.first == user) {
+      BIHIP_HIP(hipEventRecord(r.second, user));
+      return BIHIP_OK;
+    }
+  hipEvent_t e;
+  BIHIP_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  if (hipEventRecord(e, user) != hipSuccess) {
+    (void)hipEventDestroy(e);
+    return set_error(BIHIP_EHIP, "noting a reader of the network failed");
+  }
+  m->readers.emplace_back(user, e);
+  return BIHIP_OK;
+}
+
+// The network's stream waits for the noted reads.
+static int await_readers(bihip_mlp* m, hipStream_t s) {
+  std::lock_guard<std::mutex> hold(m->readers_lock);
+  hipError_t err = hipSuccess;
+  for (auto& r : m->readers) {
+    const hipError_t e = hipStreamWaitEvent(s, r.second, 0);
+    if (err == hipSuccess) err = e;
+    (void)hipEventDestroy(r.second);  // takes effect once the event has completed
+  }
+  m->readers.clear();
+  return err == hipSuccess ? BIHIP_OK
+                           : set_error(BIHIP_EHIP, "waiting for readers of the network: %s",
+                                       hipGetErrorString(err));
+}
 
 namespace bihip {
 int mlp_inference_weights(bihip_mlp* m, hipStream_t user, const uint16_t* W[MLP_MAX_LAYERS],
@@ -512,7 +510,7 @@ int bihip_mlp_train(bihip_mlp* m, const float* X_dev, long ldx, const float* T_d
   int rc = ctx_enter_device(m->ctx);
   if (rc) return rc;
   hipStream_t s = ctx_stream_of(m->ctx);
-  if ((rc = ensure_work(m, batch)) || (rc = await_readers(m, s))) return rc;
+  if ((rc = ensure_work(m, batch))) return rc;
   const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
   long* perm_d = nullptr;
   float* loss_d = nullptr;
@@ -618,7 +616,7 @@ int bihip_surrogate_flow(bihip_ctx* ctx, bihip_mlp* m, const bihip_surrogate_nor
   if (Xin_dev == Xout_dev) return set_error(BIHIP_EINVAL, "the flow is out of place");
   SurrogateLaunch L{};
   L.net = mlp_view(m);
-  if ((rc = mlp_inference_weights(m, ctx_stream_of(ctx), L.Winf))) return rc;
+  if ((rc = mlp_inference_weights(m, ctx_stream_of(ctx), L.Winf, L.binf))) return rc;
   L.x_shift = norm->x_shift;
   L.x_scale = norm->x_scale;
   L.dx_scale = norm->dx_scale;

@@ -220,7 +220,7 @@ int launch_surrogate(const SurrogateLaunch& L, hipStream_t s) {
   SurrArgs a{};
   for (int l = 0; l < n.L; ++l) {
     a.W[l] = L.Winf[l];
-    a.b[l] = n.b[l];
+    a.b[l] = L.binf[l];
   }
   a.x_shift = L.x_shift;
   a.x_inv_scale = 1.0f / L.x_scale;

@@ -152,6 +152,29 @@ def test_layout_waits_for_the_reads_of_other_streams(ctx, torch_gpu):
     new.close()
 
 
+def test_filter_keeps_the_network_it_was_given(ctx, torch_gpu):
+    """The network is read when it is attached: new parameters reach neither the weights
+    nor the biases of a filter that already has it."""
+    m = capi.make_model("l96", d=40, precision=capi.F32, init_sd=0.3)
+    y = np.random.default_rng(2).normal(2.3, 3.6, (4, 20))
+    got = []
+    for change in (False, True):
+        net = capi.MLP(ctx, surrogate.DIMS, seed=4)
+        pf = capi.ParticleFilter(ctx, m, 3000, 4, 0.05, 7)
+        pf.set_observations(y)
+        pf.set_surrogate(net, _norm())
+        pf.init(np.full(40, 2.0))
+        pf.step(1)
+        if change:
+            net.set_params(0.5 * net.get_params())
+        pf.step(3)
+        got.append((pf.outputs()["logIncrements"], pf.state()[0][:, :3000].cpu().numpy()))
+        pf.close()
+        net.close()
+    for a, b in zip(*got):
+        np.testing.assert_array_equal(a, b)
+
+
 def test_layout_refuses_a_captured_stream(ctx, torch_gpu):
     """A replay would not lay out the weights that the network has by then."""
     torch = torch_gpu
