@@ -899,9 +899,6 @@ static bool pf_small_steps(const bihip_pf* pf) {
          pf->obs_mask == nullptr && pf->inputs == nullptr && !pf->surr && !pf->guided;
 }
 
-// At most this many steps a launch, so that no launch lasts long.
-constexpr int SMALL_STEPS = 128;
-
 static int pf_enqueue_small(bihip_pf* pf, int n, hipStream_t s) {
   SmallFilterLaunch L{};
   L.model = &pf->model;
@@ -949,7 +946,7 @@ int bihip_pf_create(bihip_ctx* ctx, const bihip_model* m, const bihip_pf_config*
   pf->model = *m;
   pf->cfg = *cfg;
   pf->one_delta = gen_one_delta(m, cfg->t0, cfg->dt, cfg->T);
-  pf->small = cfg->record == 0 && small_filter_fits(m, cfg->P, pf->one_delta);
+  pf->small = cfg->record == 0 && small_filter_fits(m, cfg->P, pf->one_delta, cfg->dt);
   const int P = cfg->P;
   pf->ld = (P + 63) / 64 * 64;
   pf->elem = bihip_model_elem_size(m);
@@ -1117,8 +1114,9 @@ int bihip_pf_step(bihip_pf* pf, int n) {
   if (rc) return rc;
   hipStream_t s = pf->ctx->stream;
   if (pf_small_steps(pf)) {
+    const int most = small_filter_steps(&pf->model, pf->cfg.dt);
     while (n > 0) {
-      const int m = std::min(n, SMALL_STEPS);
+      const int m = std::min(n, most);
       if ((rc = pf_enqueue_small(pf, m, s))) return rc;
       pf->cur = (pf->cur + m) & 1;
       pf->k += m;

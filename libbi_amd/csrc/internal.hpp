@@ -329,9 +329,12 @@ struct SmallFilterLaunch {
   uint64_t seed;
   uint32_t batch;
 };
-// The model and size are compiled for it (one_delta: every interval of the
-// filter is one delta of its generated model, gen_one_delta).
-bool small_filter_fits(const bihip_model* m, int P, bool one_delta);
+// The model is compiled for it and intervals of dt run faster so than as
+// separate launches (one_delta: every interval of the filter is one delta of its
+// generated model, gen_one_delta).
+bool small_filter_fits(const bihip_model* m, int P, bool one_delta, double dt);
+// Steps one launch may take.
+int small_filter_steps(const bihip_model* m, double dt);
 int launch_small_filter(const SmallFilterLaunch& L, hipStream_t s);
 struct MultinomialLaunch {
   const double* Ws;

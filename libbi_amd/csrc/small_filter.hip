@@ -12,10 +12,14 @@
 // the combination's butterfly), so results equal theirs bit for bit.
 //
 // Bound by the latency of a step's arithmetic on one CU, and above 512 particles
-// by its FP64 rate.  Predator-prey filter in FP64, resampling every step: 6.8 us
-// a step at 256 particles, 9.3 at 512, 14.9 at 1000, against 29 to 30 us in five
-// launches (21.7 to 21.9 in three).  Two particles a thread would be slower than
-// the separate launches, so the line lies at 1024.
+// by its FP64 rate: up to four waves share a SIMD, where the separate launches
+// give each wave its own.  Predator-prey filter (ten RK4 steps an interval) in
+// FP64: 6.5 us a step at 200 particles, 9.0 at 500, 14.8 at 1000, against 12.2,
+// 13.9 and 15.5 us in three launches (18 to 20 as graphs).  Long intervals turn
+// this round above 256 particles (100 RK4 steps at 1000: 53.9 against 32 us), so
+// small_filter_fits weighs the interval.  One particle a thread: up to 1024.
+#include <cmath>
+
 #include "blockreduce.hpp"
 #include "gen_model.hpp"
 #include "internal.hpp"
@@ -189,15 +193,33 @@ __global__ __launch_bounds__(SMALL_BLOCK) void k_filter_small(SmallFilterArgs a)
 }
 
 namespace {
+// Instructions of a particle's interval: of one right-hand side and of what is not
+// the integrator (variates, actions, density; generated functors count theirs).
+template <class M>
+void model_work(double& rhs, double& rest) {
+  if constexpr (is_generated<M>::value) {
+    rhs = M::RHS_WORK;
+    rest = M::ONCE_WORK;
+  } else {
+    rhs = M::D == 2 ? 10.0 : 1.0;
+    rest = 250.0;
+  }
+}
+
 struct SmallFilterRunner {
   SmallFilterArgs a;
   int integ;
   hipStream_t s;
   bool only_ask;
+  double d, rhs, rest;  // the answer
   template <class M>
   int run() {
     if constexpr (small_filter_model<M>()) {
-      if (only_ask) return BIHIP_OK;
+      if (only_ask) {
+        d = M::D;
+        model_work<M>(rhs, rest);
+        return BIHIP_OK;
+      }
       const dim3 block(ceil_div(a.P, TRANS_BLOCK) * TRANS_BLOCK);
       if (integ == BIHIP_RK4)
         hipLaunchKernelGGL((k_filter_small<M, BIHIP_RK4>), dim3(1), block, 0, s, a);
@@ -222,12 +244,62 @@ int with_small_model(const bihip_model* m, SmallFilterRunner& r) {
 }
 }  // namespace
 
-bool small_filter_fits(const bihip_model* m, int P, bool one_delta) {
-  if (P > SMALL_BLOCK) return false;
-  if (m->model >= BIHIP_MODEL_GENERATED && !one_delta) return false;
+// Instructions of one particle's interval of length dt, as far as the model and
+// its settings tell: of its integrator steps and of the rest.  DOPRI5 chooses its
+// steps itself; h0 is taken for its step at a tolerance of 1e-5, and the step for
+// others from its order.
+struct IntervalWork {
+  double steps, rest;
+};
+static int interval_work(const bihip_model* m, double dt, IntervalWork& w) {
   SmallFilterRunner r{};
   r.only_ask = true;
-  return with_small_model(m, r) == BIHIP_OK;
+  const int rc = with_small_model(m, r);
+  if (rc) return rc;
+  w = {0.0, r.rest};
+  if (r.rhs == 0.0) return BIHIP_OK;  // no ode
+  double n = m->h0 > 0.0 ? std::fmax(1.0, std::ceil(dt / m->h0 - 1e-6)) : 1e9;
+  if (m->integrator == BIHIP_RK4) {
+    w.steps = n * (4.0 * r.rhs + 12.0 * r.d + 12.0);
+    return BIHIP_OK;
+  }
+  const double tol = std::fmax(1e-14, std::fmin(m->atol, m->rtol));
+  n = std::fmin(n * std::fmax(1.0, std::pow(1e-5 / tol, 0.2)), (double)m->nsteps);
+  w.steps = n * (7.0 * r.rhs + 34.0 * r.d + (m->precision == BIHIP_F64 ? 150.0 : 40.0));
+  return BIHIP_OK;
+}
+
+// One workgroup saves launches.  It pays, above 256 particles, with w waves a SIMD
+// that wait for each other, so the integrator's share of an interval is bounded,
+// from predator-prey intervals of 76 instructions an RK4 step: us a step, 256 a
+// call, with one workgroup and with three launches,
+//   FP64 10 steps: 9.0 / 13.9 at w = 2, 12.0 / 14.7 at 3, 14.8 / 15.5 at 4;
+//        50 steps: 18.9 / 20, 25.8 / 21, 32.4 / 22;
+//   FP32 10 steps: 7.4 / 13.2, 9.5 / 14.2, 11.7 / 14.9;
+//        100 steps: 22.7 / 30, 28.8 / 31, 36.6 / 32;
+//        500 steps: 90 / 106, 115 / 106, 146 / 107.
+// And each launch first fetches the whole step's code, tens of KB for a model with
+// binomial draws: one step a call of SIRStochastic.bi takes 25.4 us at 500
+// particles and 33 at 700, against 14.9 and 15.4 (SIR.bi 23.3 at 500 against 16.6,
+// 16.5 at 100 against 15.1 but 10.1 in calls of many steps).
+bool small_filter_fits(const bihip_model* m, int P, bool one_delta, double dt) {
+  if (P <= 0 || P > SMALL_BLOCK) return false;
+  if (m->model >= BIHIP_MODEL_GENERATED && !one_delta) return false;
+  constexpr double STEPS_F64[5] = {0.0, 1e30, 5300.0, 2000.0, 1000.0};
+  constexpr double STEPS_F32[5] = {0.0, 1e30, 40000.0, 10000.0, 4000.0};
+  constexpr double REST[5] = {0.0, 1500.0, 700.0, 500.0, 400.0};
+  const int w = ceil_div(P, TRANS_BLOCK);
+  IntervalWork i;
+  if (interval_work(m, dt, i) != BIHIP_OK) return false;
+  return i.steps <= (m->precision == BIHIP_F64 ? STEPS_F64 : STEPS_F32)[w] && i.rest <= REST[w];
+}
+
+// A launch lasts a few milliseconds at most where the estimate of the interval
+// holds (2.5 ns an instruction and wave); one step always fits.
+int small_filter_steps(const bihip_model* m, double dt) {
+  IntervalWork i;
+  if (interval_work(m, dt, i) != BIHIP_OK) return 1;
+  return (int)std::fmin(128.0, std::fmax(1.0, 1e6 / (i.steps + i.rest)));
 }
 
 int launch_small_filter(const SmallFilterLaunch& L, hipStream_t s) {

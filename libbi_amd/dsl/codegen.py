@@ -1343,6 +1343,30 @@ def _emit_obs_sample(g: GenModel, w):
     w("  }")
 
 
+# Instructions of a call, beside one of an operator (a division: 12)
+_CALL_WORK = (("gen_", 1000), ("lgamma", 150), ("normals4", 150), ("pow", 80),
+              ("philox_block", 60), ("", 30))
+
+
+def _operations(text: str) -> int:
+    """Rough number of instructions of generated code: operators and calls, a call that is
+    written several times (same name and beginning) once, as the compiler shares it."""
+    n = sum(text.count(o) for o in (" + ", " - ", " * ")) + 12 * text.count(" / ")
+    calls = set(re.findall(r"\b(gen_\w+|lgamma|normals4|pow|philox_block|exp|log|log1p|expm1|sqrt|"
+                           r"sin|cos|tan|tanh|fabs|floor|ceil|fmin|fmax)\b(?:<T>)?\((.{0,60})", text))
+    return n + sum(next(w for p, w in _CALL_WORK if name.startswith(p)) for name, _ in calls)
+
+
+def _work(g: GenModel, functor: str) -> tuple:
+    """(instructions of one right-hand side, of the rest of an interval) of a functor of one
+    lane: what the library weighs a small filter's steps by."""
+    def body(start, end):
+        i = functor.index(start)
+        return functor[i:functor.index(end, i)]
+    once = body("if constexpr (ONE) {", "return n;") + body("double obs(", "return lp;")
+    return _operations(body("void rhs(", "\n  }")) if g.has_ode else 0, _operations(once)
+
+
 def generate_model(g: GenModel) -> str:
     """The device functor of one model."""
     if g.lpp > 1:
@@ -1359,6 +1383,7 @@ def generate_model(g: GenModel) -> str:
     w(f"  static constexpr bool HAS_FORCING = {'true' if _forcing(g) else 'false'};")
     w(f"  static constexpr int MIN_WAVES = sizeof(T) == 8 ? {_min_waves(g, S)} : 1;")
     w(f"  static constexpr double DELTA = {_lit(g.delta)};")
+    delta = len(out)
     slots = [v for v in g.vars.values() if v.kind in ("param", "input")]
     noises = [v for v in g.vars.values() if v.kind == "noise"]
     for v in slots:  # in double, and in the state type for the transition's arithmetic
@@ -1486,6 +1511,8 @@ def generate_model(g: GenModel) -> str:
         w(ln)
     w("  }")
     w("};")
+    rhs, once = _work(g, "\n".join(out))
+    out.insert(delta, f"  static constexpr int RHS_WORK = {rhs}, ONCE_WORK = {once};")
     return "\n".join(out)
 
 

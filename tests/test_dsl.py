@@ -553,3 +553,17 @@ int main() {{
            stats.norm.logpdf(y[40:60], 8.0, 0.7).sum())
     assert one == pytest.approx(ref, rel=1e-12)
     assert lanes == pytest.approx(ref, rel=1e-12)
+
+
+def test_work_of_generated_models():
+    """The counts that decide how a small filter steps: operators, divisions and calls of
+    the right-hand side and of the rest; a call written twice counts once; lane models have
+    no counts."""
+    assert codegen._operations("k[0] = ((a * exp(w)) + (b / exp(w)));") == 2 + 12 + 30
+    path = os.path.join(os.path.dirname(codegen.__file__), "..", "bi")
+    models = {m.name: m for m in codegen.load_models(
+        [os.path.join(path, f) for f in ("PZ.bi", "SIRStochastic.bi", "Lorenz96d40.bi")])}
+    assert "RHS_WORK" not in codegen.generate_model(models.pop("Lorenz96d40"))
+    work = {n: codegen._work(m, codegen.generate_model(m)) for n, m in models.items()}
+    assert 8 <= work["PZ"][0] <= 16 and 150 <= work["PZ"][1] <= 500
+    assert work["SIRStochastic"][0] == 0 and work["SIRStochastic"][1] > 2000

@@ -117,6 +117,31 @@ def test_small_filter_equals_the_separate_launches(ctx, kind, prec, P, resampler
             np.testing.assert_array_equal(out[key], v, err_msg=key)
 
 
+@pytest.mark.parametrize("integ,kw", [(capi.RK4, {"h0": 0.002}), (capi.DOPRI5, {"atol": 1e-9,
+                                                                               "rtol": 1e-9})])
+@pytest.mark.parametrize("prec", [capi.F64, capi.F32])
+@pytest.mark.parametrize("P", [200, 500, 700, 1000])
+def test_small_filter_long_intervals(ctx, P, prec, integ, kw):
+    """Intervals of many integrator steps: fewer of them a launch, or separate launches,
+    with the same bits as a recorded filter."""
+    m = capi.make_model("pz", precision=prec, integrator=integ, **kw)
+    T = 40
+    y = (2.0 + 0.2 * np.sin(np.arange(T))).reshape(T, 1)
+    got = []
+    for record in (True, False):
+        pf = capi.ParticleFilter(ctx, m, P, T, 1.0, 7, ess_rel=0.7, record=record)
+        pf.set_observations(y)
+        pf.init()
+        pf.step(T)
+        out = pf.outputs()
+        X, _, lws = pf.state()
+        out["X"], out["lws"] = X[:, :P].cpu().numpy(), lws.cpu().numpy()
+        got.append(out)
+        pf.close()
+    for key, v in got[0].items():
+        np.testing.assert_array_equal(got[1][key], v, err_msg=key)
+
+
 @pytest.mark.parametrize("P", [513, 1000, 1024])
 def test_small_filter_without_resampling(ctx, P):
     """Steps that do not resample follow each other with the fewest barriers, and the
