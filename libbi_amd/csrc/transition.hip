@@ -204,9 +204,9 @@ void k_transition(TransArgs a) {
 // half a partial's particles.  Sums in the order of a workgroup with a lane per
 // slice (waves of eight particles: a butterfly, then the four waves), whatever
 // the lanes of a particle, so that log-likelihoods and effective sample sizes keep
-// their bits.  Workgroups of 512 threads, which hold a partial's particles, run
-// two waves per SIMD where these registers allow three: a bank of 16 x 16384
-// filters of d = 200 over five intervals 2.84 ms, with this launch 1.90 ms.
+// their bits.  3 us; workgroups of 512 threads, which hold a partial's particles,
+// run two waves per SIMD where the registers allow three (a bank of 16 x 16384
+// filters over five intervals 2.84 ms against 1.85).
 constexpr int PAIR_PARTIAL = 32;
 
 __global__ __launch_bounds__(256) void k_pair_partials(const double* lws, int P,
@@ -415,15 +415,32 @@ bool model_supported(const bihip_model* m) {
 #ifndef L96_D40_LPP
 #define L96_D40_LPP 4
 #endif
-// d = 200: sixteen lanes of 13 or 12 dimensions, the group a DPP row.  Eight
-// lanes of 25 needed 262 to 309 registers (one wave per SIMD) and LDS
-// permutes for the halos: 487 us against 317 us per N = 2^18 FP32 transition,
-// 369 us against 208 us per 2^16 FP64 ones.
-constexpr int L96_D200_LPP = 16;
+// d = 200: eight lanes of 25 dimensions or sixteen of 13 and 12 (a DPP row), the
+// same bits.  Sixteen need fewer registers (FP32 DOPRI5 138 against 246, FP64 256
+// with 12 bytes of spills against 512 with 260) and no LDS permutes for the halos,
+// and half the steps' latency; but a wave's load or store of a row spans four
+// particles, 16 bytes in FP32, which costs more where memory bounds.  us per
+// transition, eight / sixteen lanes, of
+//                       1000         8192         30000        262144 particles
+//   FP32 DOPRI5         15.4 / 10.2  16.4 / 15.4  35.9 / 41.9   254 / 289
+//   FP32 RK4, 5 steps   12.4 /  8.7  13.4 / 13.3  26.5 / 33.5   189 / 246
+//   FP64 DOPRI5         28.9 / 15.0  31.7 / 25.5   117 / 81     964 / 672
+//   FP64 RK4, 1 step    12.3 /  8.6  15.0 / 14.5  38.6 / 36.1   336 / 368
+//   FP64 RK4, 5 steps   17.3 / 11.5  19.9 / 19.5  52.3 / 53.9   409 / 437
+// so FP32 takes sixteen up to 8192 particles, FP64 always but for RK4 above 2^16
+// (60000 particles, five steps: 96.1 / 94.4).  A bank's FP32 DOPRI5 kernel takes
+// sixteen too: with eight its 273 registers leave one wave per SIMD (16 x 16384
+// filters over five intervals 2.85 ms, with sixteen 1.85).
+static bool d200_sixteen_lanes(const bihip_model* m, long particles, bool bank) {
+  const bool rk4 = m->integrator == BIHIP_RK4;
+  if (m->precision == BIHIP_F32) return particles <= 8192 || (bank && !rk4);
+  return !rk4 || particles <= 1L << 16;
+}
 
-// Calls F::template run<M>() for the model type selected by m.
+// Calls F::template run<M>() for the model type selected by m (sixteen: d = 200
+// over sixteen lanes).
 template <class F>
-static int with_model(const bihip_model* m, F& f) {
+static int with_model(const bihip_model* m, F& f, bool sixteen = false) {
   const bool f64 = m->precision == BIHIP_F64;
   if (m->model >= BIHIP_MODEL_GENERATED) return with_generated(m, f);
   switch (m->model) {
@@ -434,25 +451,27 @@ static int with_model(const bihip_model* m, F& f) {
         return f64 ? f.template run<L96<double, 40, L96_D40_LPP>>()
                    : f.template run<L96<float, 40, L96_D40_LPP>>();
       if (m->d == 200)
-        return f64 ? f.template run<L96<double, 200, L96_D200_LPP>>()
-                   : f.template run<L96<float, 200, L96_D200_LPP>>();
+        return sixteen ? (f64 ? f.template run<L96<double, 200, 16>>()
+                              : f.template run<L96<float, 200, 16>>())
+                       : (f64 ? f.template run<L96<double, 200, 8>>()
+                              : f.template run<L96<float, 200, 8>>());
       return f64 ? f.template run<L96<double, 8, 2>>() : f.template run<L96<float, 8, 2>>();
     default:
       return f64 ? f.template run<LG<double>>() : f.template run<LG<float>>();
   }
 }
 
-// Workgroups of the model's kernels.
-static int model_blocks(const bihip_model* m, int P) {
-  int lpp = 1;
-  if (m->model == BIHIP_MODEL_L96) lpp = m->d == 200 ? L96_D200_LPP : (m->d == 40 ? L96_D40_LPP : 2);
-  if (const GenInfo* g = generated_info(m->model)) lpp = g->lpp;
-  return ceil_div((long)P * lpp, TRANS_BLOCK);
+// Workgroups of model M's kernels.
+template <class M>
+static int model_blocks(int P) {
+  return ceil_div((long)P * M::LPP, TRANS_BLOCK);
 }
 
 int transition_blocks(const bihip_model* m, int P) {
-  if (m->model == BIHIP_MODEL_L96 && m->d == 200) return ceil_div(P, PAIR_PARTIAL);
-  return model_blocks(m, P);
+  int lpp = 1;
+  if (m->model == BIHIP_MODEL_L96) lpp = m->d == 200 ? 8 : (m->d == 40 ? L96_D40_LPP : 2);
+  if (const GenInfo* g = generated_info(m->model)) lpp = g->lpp;
+  return ceil_div((long)P * lpp, TRANS_BLOCK);
 }
 
 // [t1, t2] is one sub-interval of delta starting at a multiple of it, with a
@@ -474,7 +493,6 @@ bool gen_one_delta(const bihip_model* m, double t0, double dt, int steps) {
 
 struct TransitionRunner {
   TransArgs a;
-  int blocks;
   hipStream_t s;
   int integ;
   bool one;
@@ -494,6 +512,7 @@ struct TransitionRunner {
   }
   template <class M>
   int run_transition() {
+    const int blocks = model_blocks<M>(a.P);
     const bool sched = a.dev != nullptr && (a.times != nullptr || a.mask != nullptr ||
                                             a.inputs != nullptr || a.noise_hist != nullptr);
     if (banks > 1 || a.bank_par != nullptr) {  // a bank, also of one filter: its rows
@@ -577,21 +596,22 @@ int launch_transition(const TransLaunch& L, hipStream_t s) {
   r.a.noise_hist = L.noise_hist;
   r.a.noise_width = L.noise_width;
   r.banks = L.banks;
-  r.blocks = model_blocks(L.model, L.P);
   r.s = s;
   r.integ = L.model->integrator;
   if (const GenInfo* g = generated_info(L.model->model))
     r.one = L.dev != nullptr ? L.one_delta != 0 : one_interval(L.t1, L.t2, g->delta);
   else
     r.one = false;
-  return with_model(L.model, r);
+  return with_model(L.model, r,
+                    d200_sixteen_lanes(L.model, (long)L.P * (L.banks > 1 ? L.banks : 1),
+                                       L.bank_par != nullptr));
 }
 
 struct InitRunner {
   ModelArgs ma;
   uint64_t seed;
   uint32_t batch;
-  int P, ld, blocks;
+  int P, ld;
   void* X;
   const double* mean0;
   hipStream_t s;
@@ -600,7 +620,7 @@ struct InitRunner {
   long bx;
   template <class M>
   int run() {
-    hipLaunchKernelGGL((k_init<M>), dim3(blocks, banks), dim3(TRANS_BLOCK), 0, s, ma, seed, batch,
+    hipLaunchKernelGGL((k_init<M>), dim3(model_blocks<M>(P), banks), dim3(TRANS_BLOCK), 0, s, ma, seed, batch,
                        P, X, ld, mean0, bank_par, bx);
     BIHIP_LAUNCH_CHECK();
     return BIHIP_OK;
@@ -610,7 +630,7 @@ struct InitRunner {
 int launch_init_samples(const bihip_model* m, uint64_t seed, uint32_t batch, int P, void* X,
                         int ld, const double* mean0_dev, hipStream_t s) {
   if (P <= 0) return BIHIP_OK;
-  InitRunner r{to_args(m), seed, batch, P, ld, model_blocks(m, P), X, mean0_dev, s,
+  InitRunner r{to_args(m), seed, batch, P, ld, X, mean0_dev, s,
                1, nullptr, 0};
   return with_model(m, r);
 }
@@ -619,7 +639,7 @@ int launch_init_bank(const bihip_model* m, uint64_t seed, uint32_t batch, int P,
                      const double* mean0_dev, int banks, long x, const double* bank_par,
                      hipStream_t s) {
   if (P <= 0 || banks <= 0) return BIHIP_OK;
-  InitRunner r{to_args(m), seed, batch, P, ld, model_blocks(m, P), X, mean0_dev, s,
+  InitRunner r{to_args(m), seed, batch, P, ld, X, mean0_dev, s,
                banks, bank_par, x};
   return with_model(m, r);
 }
@@ -647,13 +667,13 @@ void bank_row(const bihip_model* m, double* row) {
 struct ObsRunner {
   ModelArgs ma;
   const double* y;
-  int P, ld, blocks;
+  int P, ld;
   const void* X;
   double* lws;
   hipStream_t s;
   template <class M>
   int run() {
-    hipLaunchKernelGGL((k_obs_logdensity<M>), dim3(blocks), dim3(TRANS_BLOCK), 0, s, ma, y, P, X,
+    hipLaunchKernelGGL((k_obs_logdensity<M>), dim3(model_blocks<M>(P)), dim3(TRANS_BLOCK), 0, s, ma, y, P, X,
                        ld, lws);
     BIHIP_LAUNCH_CHECK();
     return BIHIP_OK;
@@ -663,7 +683,7 @@ struct ObsRunner {
 int launch_obs_logdensity(const bihip_model* m, const double* y, int P, const void* X, int ld,
                           double* lws, hipStream_t s) {
   if (P <= 0) return BIHIP_OK;
-  ObsRunner r{to_args(m), y, P, ld, model_blocks(m, P), X, lws, s};
+  ObsRunner r{to_args(m), y, P, ld, X, lws, s};
   return with_model(m, r);
 }
 

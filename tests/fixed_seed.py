@@ -49,10 +49,9 @@ def crc(*arrays):
     return c
 
 
-def _transition(ctx, torch, d, prec, integ, quirk):
-    """Initial particles, one interval, its flow and the observation density (5003
-    particles: not a whole number of workgroups)."""
-    L, P = capi.lib(), 5003
+def _transition(ctx, torch, d, prec, integ, quirk, P):
+    """Initial particles, one interval, its flow and the observation density."""
+    L = capi.lib()
     # several steps in an interval, some rejected
     m = capi.make_model("l96", d=d, precision=prec, integrator=integ, h0=0.02, atol=1e-6,
                         rtol=1e-6)
@@ -174,14 +173,25 @@ def cases():
         for p, prec in (("f32", capi.F32), ("f64", capi.F64)):
             for i, integ, quirk in (("dopri5", capi.DOPRI5, 0), ("host-dopri5", capi.DOPRI5, 1),
                                     ("rk4", capi.RK4, 0)):
-                out[f"transition-l96-{d}-{p}-{i}"] = (
-                    lambda ctx, torch, a=(d, prec, integ, quirk): _transition(ctx, torch, *a))
+                # d = 200: both layouts of its lanes
+                for P in (5003,) if d < 200 else (
+                        (5003, 66001) if (p, i) == ("f64", "rk4") else (5003, 9001)):
+                    out[f"transition-l96-{d}-{p}-{i}" + (f"-{P}" if P != 5003 else "")] = (
+                        lambda ctx, torch, a=(d, prec, integ, quirk, P): _transition(
+                            ctx, torch, *a))
             for r, res in (("systematic", capi.SYSTEMATIC), ("multinomial", capi.MULTINOMIAL)):
                 out[f"filter-l96-{d}-{p}-{r}"] = (
                     lambda ctx, torch, a=(d, prec, res): _filter(
                         ctx, capi.make_model("l96", d=a[0], precision=a[1], init_sd=0.3), a[0],
                         30011 if a[0] < 200 else 5003, 6, a[2]))
+            if d == 200:
+                for P in (9001,):
+                    out[f"filter-l96-200-{p}-{P}"] = (
+                        lambda ctx, torch, prec=prec, P=P: _filter(
+                            ctx, capi.make_model("l96", d=200, precision=prec, init_sd=0.3), 200,
+                            P, 4))
         out[f"bank-l96-{d}"] = lambda ctx, torch, d=d: _bank(ctx, d, 3, 2049, 5)
+    out["bank-l96-200-12k"] = lambda ctx, torch: _bank(ctx, 200, 4, 3001, 4)
     out["surrogate-flow"] = _surrogate_flow
     out["guided-propose"] = _guided_propose
     for kind, d in (("surrogate", 40), ("guided", 200)):
