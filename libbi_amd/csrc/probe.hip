@@ -12,7 +12,9 @@
 //   kind 1: v_xor_b32 + v_add_u32 (the Philox rounds' integer work)
 //   kind 2: v_mul_f32 + v_add_f32 alternating (stage sums and norms)
 // Each loop trip of a lane issues VALU_PER_TRIP instructions of its kind.
-#include <hip/hip_runtime.h>
+//
+// biprobe_sqrt: the FP32 normals' square root over an array, for its test.
+#include "common.hpp"
 #include <stdint.h>
 
 namespace {
@@ -107,4 +109,20 @@ extern "C" int biprobe_valu(int kind, int blocks, int trips, float* out_dev, flo
   *ms = t;
   *wave_instr = (double)blocks * (PROBE_BLOCK / 64) * (double)trips * VALU_PER_TRIP;
   return 0;
+}
+
+namespace {
+__global__ void k_sqrt_probe(const float* x, long n, float* y) {
+  const long i = (long)blockIdx.x * 256 + threadIdx.x;
+  if (i < n) y[i] = bihip::sqrt_plain(x[i]);
+}
+}  // namespace
+
+// y[i] = sqrt_plain(x[i]), device arrays of n floats; waits for the result.
+extern "C" int biprobe_sqrt(const float* x_dev, long n, float* y_dev) {
+  if (n <= 0 || n > (1L << 31)) return (int)hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_sqrt_probe, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, nullptr, x_dev,
+                     n, y_dev);
+  const hipError_t e = hipGetLastError();
+  return e != hipSuccess ? (int)e : (int)hipStreamSynchronize(nullptr);
 }

@@ -4,6 +4,7 @@ Integer and index work (Philox words, uniforms, offspring, ancestors,
 permutations, gathers) must be bit-exact; floating-point results are
 checked to the tolerance written in each test."""
 import ctypes
+import os
 
 import numpy as np
 import pytest
@@ -76,9 +77,32 @@ def test_normals_f32_radius_range(ctx, orc, torch_gpu, index):
     assert (np.any(r == 0.0) and r.max() > 5.76) == (index == 10)
     assert np.all(z.reshape(-1, 2)[r == 0.0] == 0.0)
     np.testing.assert_allclose(z, ref, rtol=0, atol=4.2e-6)
-    # the root itself: the pair's length against the exact radius, where the angle's
-    # error enters as cos^2 + sin^2 only
+    # the pair's length against the exact radius
     np.testing.assert_allclose(np.hypot(z[0::2], z[1::2]), r, rtol=0, atol=4.2e-6)
+
+
+def test_normals_f32_square_root(torch_gpu):
+    """The radius' root is the correctly rounded one over its stated range: zeros, both
+    ends, squares and their neighbours (where a wrong unit shows), the radii's arguments
+    and a sweep of every exponent, bit for bit."""
+    P = ctypes.CDLL(os.path.join(os.path.dirname(capi.LIB_PATH), "libbiprobe.so"))
+    P.biprobe_sqrt.argtypes = [ctypes.c_void_p, ctypes.c_long, ctypes.c_void_p]
+    rng = np.random.default_rng(4)
+    f32 = np.float32
+    ends = np.array([0.0, -0.0, np.nextafter(f32(1e-30), f32(1)), np.nextafter(f32(1e30), f32(0))],
+                    f32)
+    sq = (np.arange(1, 4097, dtype=np.float64)[:, None] ** 2 * 2.0 ** np.arange(-60, 60, 3)).ravel()
+    sq = sq[(sq > 2e-30) & (sq < 9e29)].astype(f32)
+    u1 = 1.0 - np.arange(1 << 24) * 2.0 ** -24
+    radii = (-2.0 * np.log(u1)).astype(f32)
+    sweep = np.exp(rng.uniform(np.log(1.1e-30), np.log(9e29), 1 << 22)).astype(f32)
+    x = np.concatenate([ends, sq, np.nextafter(sq, f32(0)), np.nextafter(sq, f32(np.inf)), radii,
+                        sweep])
+    xd = dev(x)
+    y = empty(x.size, torch_gpu.float32)
+    torch_gpu.cuda.synchronize()
+    assert P.biprobe_sqrt(xd.data_ptr(), x.size, y.data_ptr()) == 0
+    np.testing.assert_array_equal(host(y).view(np.uint32), np.sqrt(x).view(np.uint32))
 
 
 # ---------------------------------------------------------------- model kernels
