@@ -17,6 +17,7 @@
 
 #include "model_ops.hpp"
 #include "scan.hpp"
+#include "small_chain.hpp"
 #include "gen_model.hpp"
 
 namespace bihip {
@@ -64,52 +65,12 @@ __device__ __forceinline__ M make_model(const BatchArgs& a, int j) {
   return M(ma);
 }
 
-// Scans of one integer value per thread of a workgroup of BLOCK threads: DPP
-// within the waves, one row of lanes over the waves' sums.
-template <int BLOCK, class V>
+// Inclusive scan of one integer value per thread; lds is free again after it.
+template <class V>
 __device__ __forceinline__ V block_incl_scan(V v, V* lds, V& total) {
-  constexpr int NW = BLOCK / WAVE;
-  static_assert(NW <= 16, "the waves' sums fit a row of lanes");
-  const int lane = threadIdx.x & (WAVE - 1);
-  const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE));
-  v = wave_inclusive_scan(v);
-  if (lane == WAVE - 1) lds[w] = v;
+  v = small_inclusive_scan(v, lds, total);
   __syncthreads();
-  const int q = lane & 15;
-  const V s = row_inclusive_scan(q < NW ? lds[q] : V(0));
-  __syncthreads();
-  total = read_lane(s, 15);
-  return w > 0 ? read_lane(s, w - 1) + v : v;
-}
-
-template <int BLOCK>
-__device__ __forceinline__ u128 block_incl_scan_u128(u128 v, u128* lds, u128& total) {
-  return block_incl_scan<BLOCK>(v, lds, total);
-}
-
-template <int BLOCK>
-__device__ __forceinline__ uint64_t block_excl_scan_u64(uint64_t v, uint64_t* lds,
-                                                        uint64_t& total) {
-  return block_incl_scan<BLOCK>(v, lds, total) - v;
-}
-
-__device__ __forceinline__ int sys_offspring(double Ws, double W, int n, double a) {
-#pragma clang fp contract(off)
-  const double v = Ws / W * (double)n + a;
-  const int o = (int)v;
-  return o < n ? o : n;
-}
-
-__device__ __forceinline__ int strat_offspring(double Ws, double W, int n, uint64_t seed,
-                                               uint32_t step, uint32_t batch) {
-#pragma clang fp contract(off)
-  const double reach = Ws / W * (double)n;
-  int k = (int)reach;
-  if (k > n - 1) k = n - 1;
-  const u32x4 r = philox_block(seed, (uint32_t)k, step, TAG_STRATIFIED, batch, 0);
-  const double alpha = u53(r.x, r.y);
-  const int o = (int)(reach + alpha);
-  return o < n ? o : n;
+  return v;
 }
 
 template <class M, int INTEG, int BLOCK, int BITEMS = BITEMS_DEFAULT>
@@ -157,7 +118,7 @@ __global__ __launch_bounds__(BLOCK) void k_batch_step(BatchArgs a) {
           if (base + u < N) part = part + fix_weight(nanexp(a.lws[off + base + u] - F.mx));
       }
       u128 Wfix;
-      (void)block_incl_scan_u128<BLOCK>(part, l128, Wfix);
+      (void)block_incl_scan(part, l128, Wfix);
       const double W = fix_to_double(Wfix);
       if (!(W > 0.0)) {
         if (tid == 0) a.f[j].status = BIHIP_DEGENERATE;
@@ -171,8 +132,8 @@ __global__ __launch_bounds__(BLOCK) void k_batch_step(BatchArgs a) {
         auto offspring = [&](const u128& P) {  // cumulative offspring at prefix P
           const double Ws = fix_to_double(P);
           return a.resampler == BIHIP_SYSTEMATIC
-                     ? sys_offspring(Ws, W, N, av)
-                     : strat_offspring(Ws, W, N, a.seed, (uint32_t)k, batch);
+                     ? systematic_offspring(Ws, W, N, av)
+                     : stratified_keyed(Ws, W, N, a.seed, (uint32_t)k, batch);
         };
         u128 carry(0);
         uint64_t efcarry = 0;
@@ -186,7 +147,7 @@ __global__ __launch_bounds__(BLOCK) void k_batch_step(BatchArgs a) {
             loc = loc + w[u];
           }
           u128 tot;
-          const u128 incl = block_incl_scan_u128<BLOCK>(loc, l128, tot);
+          const u128 incl = block_incl_scan(loc, l128, tot);
           u128 P = carry + (incl - loc);  // prefix before this thread's first particle
           int O0 = base > 0 && base < N ? offspring(P) : 0;
           uint64_t ef[BITEMS];
@@ -205,7 +166,7 @@ __global__ __launch_bounds__(BLOCK) void k_batch_step(BatchArgs a) {
             eloc += e | (fz << 32);
           }
           uint64_t eftot;
-          const uint64_t ex0 = efcarry + block_excl_scan_u64<BLOCK>(eloc, l64, eftot);
+          const uint64_t ex0 = efcarry + block_incl_scan(eloc, l64, eftot) - eloc;
 #pragma unroll
           for (int u = 0; u < BITEMS; ++u) {
             const int i = base + u;

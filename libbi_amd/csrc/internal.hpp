@@ -424,23 +424,22 @@ int launch_batch_copy(const long* dst_off, const long* src_off, const int* len, 
                       const double* lws_s, void* Xd, long ldd, double* lws_d, hipStream_t s);
 
 // ---- BF16 MFMA multilayer perceptron (mlp.hip)
-enum { EPI_STORE = 0, EPI_BIAS_GELU = 1, EPI_BIAS = 2, EPI_GELU_GRAD = 3 };
+enum { EPI_BIAS_GELU, EPI_BIAS, EPI_GELU_GRAD };
 struct GemmArgs {
-  const uint16_t* A;  // A(m,k) = TA ? A[k lda + m] : A[m lda + k]  (bf16)
+  const uint16_t* A;  // A(m,k) = A[m lda + k]  (bf16)
   long lda;
-  const uint16_t* B;  // B(k,n) = TB ? B[n ldb + k] : B[k ldb + n]  (bf16)
+  const uint16_t* B;  // B(k,n) = B[n ldb + k], EPI_GELU_GRAD: B[k ldb + n]  (bf16)
   long ldb;
-  int M, N, K;        // multiples of 64, 64, 32
-  int ksplit;         // k range per split (multiple of 32); splits write Cf + z M ldc
+  int M, N, K;        // multiples of 64
   const float* bias;  // [N] (EPI_BIAS_GELU, EPI_BIAS)
-  float* Cf;          // f32 out: product, pre-activation or linear output
+  float* Cf;          // f32 out: pre-activation or linear output
   long ldc;
   uint16_t* Cb;       // bf16 out: GELU activation or back-propagated error
   long ldcb;
   const float* Zprev; // EPI_GELU_GRAD: pre-activation whose GELU derivative scales the product
   long ldz;
 };
-int launch_gemm(const GemmArgs& g, bool ta, bool tb, int epi, hipStream_t s);
+int launch_gemm(const GemmArgs& g, int epi, hipStream_t s);
 int launch_rows_to_bf16(const float* X, long ldx, const long* idx, int n, int rows, int d,
                         uint16_t* Y, int ldy, hipStream_t s);
 int launch_mse_grad(const float* Y, int ldy, const float* T, long ldt, const long* idx, int n,
@@ -485,13 +484,10 @@ struct UpdateArgs {
 };
 int launch_update(const UpdateArgs& a, hipStream_t s);
 
-// Device parameters of an MLP (bf16 weights [pad_{l+1}][pad_l], FP32 biases),
-// for the fused inference kernels.
+// Shape of an MLP, for the fused inference kernels.
 struct MlpView {
   int L;
   int dims[MLP_MAX_LAYERS + 1], pad[MLP_MAX_LAYERS + 1];
-  const uint16_t* W[MLP_MAX_LAYERS];
-  const float* b[MLP_MAX_LAYERS];
 };
 MlpView mlp_view(const bihip_mlp* m);
 // bf16 weights with the input columns of layers l >= 1 permuted for the fused

@@ -1,6 +1,7 @@
 // BF16 MFMA kernels of the multilayer perceptron: the tiled GEMM with fused
-// epilogues that the forward and backward passes are built from, the loss,
-// column sums, split-K reduction, Adam, and input conversion.
+// epilogues of the forward and backward passes, the loss, weight and bias
+// gradients split over the batch, their sums with the Adam step, the inference
+// copy of the weights, and input conversion.
 //
 // The network has no counterpart in the reference (LibBi has no learned
 // components): it is the learned surrogate flow and guided proposal built
@@ -18,9 +19,10 @@ namespace {
 // GEMM of 4096 x 256 x 256 8.4 -> 6.8 us).
 constexpr int GB_M = 64, GB_N = 64, GB_K = 64, LDS_K = GB_K + 8;  // +8: bank spread
 
-// C = op(A) op(B) over k in [z ksplit, (z + 1) ksplit), 64 x 64 tiles, four
-// waves of 32 x 32.  Tiles are staged k-contiguous in LDS whatever the global
-// orientation, so every fragment read is one 16-byte LDS load.
+// Products are computed in 64 x 64 tiles, four waves of 32 x 32.  Operand tiles
+// are staged k-contiguous in LDS whatever the global orientation, so every
+// fragment read is one 16-byte LDS load.
+//
 // One 64 x 64 operand tile of K step k0 into LDS, k-contiguous: rows of X from
 // r0 (TRANS false: X[(r0 + r) ld + k0 + k], true: X[(k0 + k) ld + r0 + r]).
 template <bool TRANS>
@@ -82,28 +84,25 @@ __device__ __forceinline__ void gemm_tile(const uint16_t* A, long lda, const uin
   }
 }
 
-template <bool TA, bool TB, int EPI>
+// C = A op(B), with B transposed in the forward products.
+template <int EPI>
 __global__ __launch_bounds__(256) void k_gemm(GemmArgs g) {
   __shared__ __attribute__((aligned(16))) uint16_t As[GB_M * LDS_K];
   __shared__ __attribute__((aligned(16))) uint16_t Bs[GB_N * LDS_K];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int wm = w >> 1, wn = w & 1;
   const int m0 = blockIdx.x * GB_M, n0 = blockIdx.y * GB_N;
-  const int kbeg = blockIdx.z * g.ksplit;
-  const int kend = kbeg + g.ksplit < g.K ? kbeg + g.ksplit : g.K;
   f32x16 acc;
 #pragma unroll
   for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
-  gemm_tile<TA, TB>(g.A, g.lda, g.B, g.ldb, m0, n0, kbeg, kend, As, Bs, acc,
-                    [](const uint16_t*) {});
+  gemm_tile<false, EPI != EPI_GELU_GRAD>(g.A, g.lda, g.B, g.ldb, m0, n0, 0, g.K, As, Bs, acc,
+                                         [](const uint16_t*) {});
   const int col = n0 + wn * 32 + (lane & 31);
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
     const int row = m0 + wm * 32 + acc_row(r, lane);
     const float v = acc[r];
-    if constexpr (EPI == EPI_STORE) {
-      g.Cf[(size_t)blockIdx.z * g.M * g.ldc + (size_t)row * g.ldc + col] = v;
-    } else if constexpr (EPI == EPI_BIAS_GELU) {
+    if constexpr (EPI == EPI_BIAS_GELU) {
       const float z = v + g.bias[col];
       g.Cf[(size_t)row * g.ldc + col] = z;
       g.Cb[(size_t)row * g.ldcb + col] = f2bf(gelu_f(z));
@@ -383,38 +382,25 @@ __global__ __launch_bounds__(256) void k_inference_weights(InferenceWeightsArgs 
   }
 }
 
-template <bool TA, bool TB>
-int gemm_epi(const GemmArgs& g, int epi, dim3 grid, hipStream_t s) {
+}  // namespace
+
+int launch_gemm(const GemmArgs& g, int epi, hipStream_t s) {
+  // the kernel's tiling assumptions, checked here so that no access leaves the operands
+  if (g.M <= 0 || g.N <= 0 || g.K <= 0 || g.M % GB_M || g.N % GB_N || g.K % GB_K ||
+      g.lda % 8 || g.ldb % 8)
+    return set_error(BIHIP_EINVAL, "GEMM shape %dx%dx%d (lda %ld, ldb %ld) off the 64x64x64 "
+                     "tiling", g.M, g.N, g.K, g.lda, g.ldb);
+  if (((uintptr_t)g.A | (uintptr_t)g.B) & 15)
+    return set_error(BIHIP_EINVAL, "GEMM operands must be 16-byte aligned");
+  const dim3 grid(g.M / GB_M, g.N / GB_N), block(256);
   switch (epi) {
-    case EPI_STORE: hipLaunchKernelGGL((k_gemm<TA, TB, EPI_STORE>), grid, dim3(256), 0, s, g); break;
-    case EPI_BIAS_GELU:
-      hipLaunchKernelGGL((k_gemm<TA, TB, EPI_BIAS_GELU>), grid, dim3(256), 0, s, g);
-      break;
-    case EPI_BIAS: hipLaunchKernelGGL((k_gemm<TA, TB, EPI_BIAS>), grid, dim3(256), 0, s, g); break;
-    case EPI_GELU_GRAD:
-      hipLaunchKernelGGL((k_gemm<TA, TB, EPI_GELU_GRAD>), grid, dim3(256), 0, s, g);
-      break;
+    case EPI_BIAS_GELU: hipLaunchKernelGGL(k_gemm<EPI_BIAS_GELU>, grid, block, 0, s, g); break;
+    case EPI_BIAS: hipLaunchKernelGGL(k_gemm<EPI_BIAS>, grid, block, 0, s, g); break;
+    case EPI_GELU_GRAD: hipLaunchKernelGGL(k_gemm<EPI_GELU_GRAD>, grid, block, 0, s, g); break;
     default: return set_error(BIHIP_EINVAL, "unknown GEMM epilogue %d", epi);
   }
   BIHIP_LAUNCH_CHECK();
   return BIHIP_OK;
-}
-
-}  // namespace
-
-int launch_gemm(const GemmArgs& g, bool ta, bool tb, int epi, hipStream_t s) {
-  // the kernel's tiling assumptions, checked here so that no access leaves the operands
-  if (g.M <= 0 || g.N <= 0 || g.K <= 0 || g.M % GB_M || g.N % GB_N || g.K % GB_K ||
-      g.ksplit <= 0 || g.ksplit % GB_K || g.lda % 8 || g.ldb % 8)
-    return set_error(BIHIP_EINVAL, "GEMM shape %dx%dx%d (split %d, lda %ld, ldb %ld) off the "
-                     "64x64x32 tiling", g.M, g.N, g.K, g.ksplit, g.lda, g.ldb);
-  if (((uintptr_t)g.A | (uintptr_t)g.B) & 15)
-    return set_error(BIHIP_EINVAL, "GEMM operands must be 16-byte aligned");
-  const dim3 grid(g.M / GB_M, g.N / GB_N, (g.K + g.ksplit - 1) / g.ksplit);
-  if (!ta && tb) return gemm_epi<false, true>(g, epi, grid, s);
-  if (!ta && !tb) return gemm_epi<false, false>(g, epi, grid, s);
-  if (ta && !tb) return gemm_epi<true, false>(g, epi, grid, s);
-  return gemm_epi<true, true>(g, epi, grid, s);
 }
 
 int launch_rows_to_bf16(const float* X, long ldx, const long* idx, int n, int rows, int d,

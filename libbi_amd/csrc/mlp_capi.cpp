@@ -110,13 +110,12 @@ int forward(bihip_mlp* m, int rows, hipStream_t s) {
     g.M = rows;
     g.N = m->pad[l + 1];
     g.K = m->pad[l];
-    g.ksplit = g.K;
     g.bias = m->P + m->offb[l];
     g.Cf = m->Z[l];
     g.ldc = m->pad[l + 1];
     g.Cb = l + 1 < L ? m->A[l + 1] : nullptr;
     g.ldcb = m->pad[l + 1];
-    int rc = launch_gemm(g, false, true, l + 1 < L ? EPI_BIAS_GELU : EPI_BIAS, s);
+    int rc = launch_gemm(g, l + 1 < L ? EPI_BIAS_GELU : EPI_BIAS, s);
     if (rc) return rc;
   }
   return BIHIP_OK;
@@ -137,12 +136,11 @@ int backward(bihip_mlp* m, int rows, const UpdateArgs& u, hipStream_t s) {
     h.M = rows;
     h.N = m->pad[l];
     h.K = m->pad[l + 1];
-    h.ksplit = h.K;
     h.Zprev = m->Z[l - 1];
     h.ldz = m->pad[l];
     h.Cb = m->dZ[l - 1];
     h.ldcb = m->pad[l];
-    if ((rc = launch_gemm(h, false, false, EPI_GELU_GRAD, s))) return rc;
+    if ((rc = launch_gemm(h, EPI_GELU_GRAD, s))) return rc;
   }
   const int ksplit = std::min(rows, KSPLIT), S = (rows + ksplit - 1) / ksplit;
   for (int l = 0; l < m->L;) {
@@ -326,17 +324,13 @@ int mlp_inference_weights(bihip_mlp* m, hipStream_t user, const uint16_t* W[MLP_
   return BIHIP_OK;
 }
 
-// Device parameters of an MLP for the fused inference kernels (surrogate.hip).
+// Shape of an MLP for the fused inference kernels (surrogate.hip, guided.hip).
 MlpView mlp_view(const bihip_mlp* m) {
   MlpView v{};
   v.L = m->L;
   for (int l = 0; l <= m->L && l < MLP_MAX_LAYERS + 1; ++l) {
     v.dims[l] = m->dims[l];
     v.pad[l] = m->pad[l];
-  }
-  for (int l = 0; l < m->L && l < MLP_MAX_LAYERS; ++l) {
-    v.W[l] = m->Wbf + m->offW[l];
-    v.b[l] = m->P + m->offb[l];
   }
   return v;
 }

@@ -111,14 +111,6 @@ __device__ __forceinline__ V await_value(uint64_t* words, uint32_t epoch, uint32
 }
 
 template <class V>
-__device__ __forceinline__ V shfl_up_v(const V& v, int o) {
-  return __shfl_up(v, o, WAVE);
-}
-template <>
-__device__ __forceinline__ u128 shfl_up_v<u128>(const u128& v, int o) {
-  return u128(__shfl_up(v.lo, o, WAVE), __shfl_up(v.hi, o, WAVE));
-}
-template <class V>
 __device__ __forceinline__ V shfl_xor_v(const V& v, int o) {
   return __shfl_xor(v, o, WAVE);
 }

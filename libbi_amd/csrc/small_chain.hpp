@@ -1,5 +1,6 @@
-// Resampling of one filter by one workgroup, and the offspring expressions it
-// shares with the tiled chain (resample.hip).
+// Resampling of one filter by one workgroup, and the offspring expressions and
+// the scan it shares with the tiled chain (resample.hip) and the batched step
+// (batch.hip).
 //
 // Replaces (ON_DEVICE): see resample.hip.
 #pragma once
@@ -27,6 +28,16 @@ __device__ __forceinline__ int stratified_offspring(double reach, double alpha, 
 #pragma clang fp contract(off)
   const int o = (int)(reach + alpha);
   return o < n ? o : n;
+}
+
+// The cumulative offspring with the stratum's keyed uniform.
+__device__ __forceinline__ int stratified_keyed(double Ws, double W, int n, uint64_t seed,
+                                                uint32_t step, uint32_t batch) {
+  const double reach = stratified_reach(Ws, W, n);
+  int k = (int)reach;
+  if (k > n - 1) k = n - 1;
+  const u32x4 r = philox_block(seed, (uint32_t)k, step, TAG_STRATIFIED, batch, 0);
+  return stratified_offspring(reach, u53(r.x, r.y), n);
 }
 
 // (e, f) = (max(o - 1, 0), [o == 0]) packed as e | f << 32.
@@ -69,8 +80,8 @@ struct SmallChainLds {
 };
 
 // Ancestors src of the thread's ITEMS consecutive particles (from
-// threadIdx.x * ITEMS; blockDim.x * ITEMS >= P) of a filter of P particles with log-weights lw and
-// maximum m, n = P draws of step `step`; false (for the whole workgroup) if the
+// threadIdx.x * ITEMS; blockDim.x * ITEMS >= P) of a filter of P particles with
+// log-weights lw and maximum m, n = P draws of step `step`; false (for the whole workgroup) if the
 // weights sum to no positive number.  Exact integer sums and the tiled chain's
 // expressions, so its ancestors.  Ends with reads of the LDS.
 template <int MODE, int ITEMS, class Lds>
@@ -122,11 +133,7 @@ __device__ __forceinline__ bool small_chain(const double (&lw)[ITEMS], double m,
     auto cumulative = [&](const u128& incl) -> int {
       const double Wsi = fix_to_double(incl);
       if (MODE == BIHIP_SYSTEMATIC) return systematic_offspring(Wsi, W, n, av);
-      const double reach = stratified_reach(Wsi, W, n);
-      int k = (int)reach;
-      if (k > n - 1) k = n - 1;
-      const u32x4 r = philox_block(seed, (uint32_t)k, step, TAG_STRATIFIED, batch, 0);
-      return stratified_offspring(reach, u53(r.x, r.y), n);
+      return stratified_keyed(Wsi, W, n, seed, step, batch);
     };
     int prev = base > 0 && base < P ? cumulative(start) : 0;
 #pragma unroll
