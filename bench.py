@@ -30,8 +30,9 @@ Other workloads (`--workload`), each printing one JSON line of the same form:
          the known-size kernel that scales the FETCH_SIZE / WRITE_SIZE
          counters into bytes;
   valu   the vector-ALU issue-rate probe (FP32 FMA, integer, FP32 mul/add
-         mixes): the achievable VALU ceiling, and the known-count kernel that
-         scales the SQ_INSTS_VALU counter;
+         mixes): rates to compare a kernel's with (the FMA reads one operand
+         from a scalar register, so it is no limit of the chip), and the
+         known-count kernel that scales the SQ_INSTS_VALU counter;
   guided the Lorenz-96 d=200 filter with a learned guided proposal
          (301-256-256-256-400 BF16 MFMA network, trained on the GPU before the
          timed region) and the exact importance-weight correction, N=2^18
@@ -77,9 +78,9 @@ HBM_PEAK_GBS = 8000.0
 # again when a change moves the FP32 trajectory.  The probe's FMA reads one
 # operand from a scalar register, which halves its rate; the kernel's mostly do
 # not, so a fraction near 1 is the probe's rate reached, not the chip's limit.
-L96_TRAFFIC_BYTES = 390_671_360
-L96_VALU_PER_LAUNCH = 1.374e8
-L96_VALU_FP32_SHARE = 0.766
+L96_TRAFFIC_BYTES = 396_544_000
+L96_VALU_PER_LAUNCH = 1.254e8
+L96_VALU_FP32_SHARE = 0.751
 
 
 def parse():
@@ -1058,24 +1059,25 @@ def main():
         },
     }
     if not generated and P == P_DEFAULT:
-        # what bounds the kernel: its VALU issue rate against the ceiling that
-        # the issue-rate probe measures now, on this GPU, for its instruction mix
+        # what bounds the kernel: its VALU issue rate against the rate that the
+        # issue-rate probes reach now, on this GPU, weighted by its instruction mix
+        # (no limit of the chip, see above)
         rates, _, _ = valu_probe(kinds=(0, 1))
         launch_s = trans_ms * 1e-3 / max(trans_n, 1)
         rate = L96_VALU_PER_LAUNCH / launch_s
-        ceiling = 1.0 / (L96_VALU_FP32_SHARE / rates[0] + (1.0 - L96_VALU_FP32_SHARE) / rates[1])
+        probe_rate = 1.0 / (L96_VALU_FP32_SHARE / rates[0] + (1.0 - L96_VALU_FP32_SHARE) / rates[1])
         line["roofline"]["limiter"] = "valu"
-        line["roofline"]["valu_frac"] = rate / ceiling
+        line["roofline"]["valu_frac"] = rate / probe_rate
         line["roofline"]["valu"] = {
             "wave_instr_per_launch": L96_VALU_PER_LAUNCH,
             "issue_rate": rate,
-            "ceiling": ceiling,
+            "probe_rate": probe_rate,
             "unit": "wave-instr/s",
             "probe_fp32_fma": rates[0],
             "probe_int32": rates[1],
             "fp32_rate_share": L96_VALU_FP32_SHARE,
             "source": "SQ_INSTS_VALU and its class counters per launch (rocprofv3 --pmc, this "
-                      "command's timed window) / this run's average launch time; ceiling = the "
+                      "command's timed window) / this run's average launch time; probe_rate = the "
                       "issue-rate probes (bench.py --workload valu) weighted by the mix",
         }
     if generated:
