@@ -93,8 +93,8 @@ struct Normal<double> {
 // s (s - ulp) < x <= s (s + ulp): Agarwal et al., IBM J. Res. Dev. 30, 1986),
 // its products as exact residuals.  (A zero's neighbours fail both tests: NaN
 // below, no positive residual above.)  With
-// xor3, the FP32 transition takes 44.4 us at 2^20 x 8 (45.7 before), 205 at
-// 2^20 x 40 (206.5) and 313 at 2^18 x 200 (319).
+// xor3, the FP32 transition takes 44.4 us at 2^20 x 8 (45.7 with the general
+// sequence and two XORs) and 205 at 2^20 x 40 (206.5).
 __device__ __forceinline__ float sqrt_plain(float x) {
   const float s = __builtin_amdgcn_sqrtf(x);
   const float dn = __int_as_float(__float_as_int(s) - 1);

@@ -19,10 +19,13 @@
 // MFMA with FP32 accumulation, laid out as the surrogate kernel's (32
 // particles per wave, weights staged in LDS in row chunks that are copied
 // while the chunk before is computed, activations in registers).  2^17
-// particles take 0.160 ms (508 TFLOP/s); with every state of the output read
-// behind the store before it and the chunks loaded between barriers, 0.233 ms.  The inference weights of the output layer interleave the rows
-// per 16 dimensions (m of dimensions 16 t .. 16 t + 15, then their s), so one
-// 32-row output tile carries both numbers of the dimensions it covers.
+// particles take 0.157 ms (518 TFLOP/s); with every state of the output read
+// behind the store before it and the chunks loaded between barriers, 0.233 ms.
+// Bound by vector work beside the matrix cores (10600 vector and 624 matrix
+// instructions a wave, 37% of the wave cycles waiting) at two waves per SIMD.
+// The inference weights of the output layer interleave the rows per 16
+// dimensions (m of dimensions 16 t .. 16 t + 15, then their s), so one 32-row
+// output tile carries both numbers of the dimensions it covers.
 #include <type_traits>
 
 #include "blockreduce.hpp"

@@ -51,8 +51,7 @@ __device__ __forceinline__ uint32_t cvt_pk_bf16(float a, float b) {
 }
 
 // GELU in its sigmoid form z sigma(1.702 z) (Hendrycks & Gimpel 2016, sec. 2):
-// one exponential and one reciprocal per activation, which keeps the hidden
-// layers' vector work below the matrix-core time.  Derivative
+// one exponential and one reciprocal per activation.  Derivative
 // s + 1.702 z s (1 - s) with s = sigma(1.702 z).
 __device__ __forceinline__ float gelu_sigmoid(float z) {
   return __builtin_amdgcn_rcpf(1.0f + __expf(-1.702f * z));
@@ -228,8 +227,7 @@ __device__ __forceinline__ f32x16 bias_tile(const float* bias, int t, int lane) 
 // from 32 T0 on; out[2 t + s] receives the packed activations of tile t.  (Two
 // waves share a SIMD: one's activations run beside the other's matrix
 // instructions.  Computing a tile's activations between the next tile's matrix
-// instructions of the same wave measured the same, 433 us per 2^20 particles
-// of the surrogate flow.)
+// instructions of the same wave measured the same on the surrogate flow.)
 template <int KC, int NOUTC, int K, int T0, int T1>
 __device__ __forceinline__ void gelu_tiles(const uint8_t* buf, const float* bias,
                                            const uint32_t (&in)[KC][4],

@@ -3,10 +3,10 @@
 // One particle is owned by a group of LPP consecutive lanes of a wavefront;
 // lane g of the group holds the state dimensions from slice_lo(g) on in
 // registers, DL of them (DL = D / LPP rounded up; where LPP does not divide D
-// the even lanes hold DL and the odd ones DL - 1).  The Lorenz-96 stencil fetches its three halo values from
-// the neighbouring lanes of the group; error norms are group butterfly sums,
-// so every lane of a group computes bit-identical step-control decisions and
-// the group never diverges internally.
+// the even lanes hold DL and the odd ones DL - 1).  The Lorenz-96 stencil
+// fetches its three halo values from the neighbouring lanes of the group; error
+// norms are group butterfly sums, so every lane of a group computes
+// bit-identical step-control decisions and the group never diverges internally.
 //
 // Semantics follow the reference host integrators:
 //   RK4    share/src/bi/host/ode/RK4IntegratorHost.hpp:63-97,  share/src/bi/ode/RK4Stage.hpp:26-76

@@ -20,13 +20,13 @@
 // weights).  The weights pass through LDS in chunks of 128 rows, each copied
 // while the one before is computed (mlp.hpp).
 //
-// What bounds it: 2^20 particles take 0.416 ms (762 TFLOP/s, 30% of the dense
-// bf16 rate).  Before, every layer was loaded through registers behind two
-// barriers, and the input and output states were read one load after another
-// (each behind its own branch): 0.94 ms, 60% of the wave cycles waiting, now
-// 40%.  The rest is vector work: 4450 vector instructions a wave, an
-// exponential and a reciprocal per activation among them, at two waves per
-// SIMD (182 registers).
+// What bounds it: 2^20 particles take 0.45 ms (708 TFLOP/s, 28% of the dense
+// bf16 rate), 0.48 in a filter's step.  With every layer loaded through
+// registers behind two barriers, and the input and output states read one load
+// after another (each behind its own branch), 0.94 ms and 60% of the wave
+// cycles waiting, now 39%.  The rest is vector work: 3900 vector instructions a
+// wave, an exponential and a reciprocal per activation among them, at two waves
+// per SIMD (184 registers).
 #include "blockreduce.hpp"
 #include "internal.hpp"
 #include "mlp.hpp"
