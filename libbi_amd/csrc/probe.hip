@@ -4,9 +4,11 @@
 // when nothing else limits a kernel: every lane runs eight independent
 // dependency chains (so latency never stalls issue), the grid fills every
 // SIMD eight waves deep, and there are no memory accesses inside the loop.
-// The result is the ceiling against which a VALU-bound kernel's
-// SQ_INSTS_VALU rate is read; the same kernel, with its known instruction
-// count, also calibrates that counter.
+// The result is the rate that a VALU-bound kernel's SQ_INSTS_VALU rate is
+// compared with, no limit of the chip: kind 0's FMA reads one operand from a
+// scalar register, which takes 4.2 cycles of a SIMD where vector and literal
+// operands take 2.2-2.5.  The same kernel, with its known instruction count,
+// also calibrates that counter.
 //
 //   kind 0: v_fma_f32            (the DOPRI5 stages' arithmetic)
 //   kind 1: v_xor_b32 + v_add_u32 (the Philox rounds' integer work)
